@@ -488,7 +488,7 @@ def bench_decode(args, torch, dev):
         # entries, the queries and the outputs
         algo = B * ctx * (2 * 2 * 256 + 4) + 2 * B * NT * 16 * 256 * 2
         res[name] = dict(us_per_step=ms * 1e3, bytes=algo, gbs=algo / (ms * 1e-3) / 1e9, sequences=B,
-                         query_tokens=B * NT, context=ctx, splits=_decode_splits(B))
+                         query_tokens=B * NT, context=ctx, splits="balanced")
         del q, kc, vc, pt, ws, out
     return res
 
@@ -551,12 +551,6 @@ def _hybrid_form(args, torch, dev, hybrid, synth, w, B, T, ctx, form):
     del st, ws
     return dict(us_per_step=ms * 1e3, us_eager=ms_eager * 1e3, rows=B * T, tokens_per_s=B * T / (ms * 1e-3),
                 sequences=B, verify_tokens=T, context=ctx)
-
-
-def _decode_splits(B):
-    import torch
-    cus = torch.cuda.get_device_properties(0).multi_processor_count
-    return max(1, min(64, cus // (B * 2)))
 
 
 MFMA_I8_PEAK_TOPS = 5000.0  # MI355X dense int8, published

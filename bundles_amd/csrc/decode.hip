@@ -11,8 +11,9 @@
 //
 // Kernels:
 //   kv_scatter      the new tokens' e4m3 K and V rows into the cache slots out_loc[t].
-//   decode_split    workgroup = (split, KV head, request), 4 independent waves; each wave streams
-//                   its own contiguous run of 32-key steps for the group's 8 query heads x NT tokens
+//   decode_split    workgroup = an equal share of all requests' keys (or one of a fixed number of splits
+//                   of a request, when the caller asks for that), for one KV head; 4 independent waves,
+//                   each streaming its own contiguous run of 32-key steps for the group's 8 query heads x NT tokens
 //                   (16 or 32 query rows) with its own running max / weight sum / output, and the
 //                   four are merged once at the end.  Scores S^T = K Q^T: e4m3 16x16x128 MFMA with
 //                   the keys as operand A straight from the cache (registers) and the e4m3 query
@@ -24,8 +25,8 @@
 //                   per-wave pipeline (2 stages at two waves a SIMD for one row tile, 4 at one wave
 //                   a SIMD for two) with no workgroup barrier; the output is rescaled only
 //                   when a row max grows by more than 2^8 (weights up to 2^8 are exact in f16).
-//   decode_combine  the splits' partials weighted by exp2(m_s - M) / L (with one split the split
-//                   kernel writes the output itself).
+//   decode_combine  a cut request's partials weighted by exp2(m_p - M) / L (a request that one
+//                   workgroup holds whole is written by the split kernel itself).
 #include <math.h>
 
 #include <type_traits>
@@ -40,7 +41,6 @@ constexpr int kQH = 16, kKVH = 2, kDD = 256, kGQ = kQH / kKVH, kDNT = 4, kDRows 
 constexpr int kST = 32;              // keys per wave step
 // NS (kernel template): key / value stages per wave (steps in flight + 1); the page-table entries run
 // 2 NS steps ahead, so an entry's DMA is older than every key and value load a wait leaves in flight
-constexpr int kPTR = 8;              // page-table ring entries per wave (one step each)
 // The two forms' shapes (alternating builds on one box, three rounds): the one-row-tile form (decode,
 // NT <= 2) with 2 stages fits 224 registers and 77 KB of LDS, so two workgroups share a CU (two waves
 // a SIMD): decode 189.9 -> 182.7 us against 3 stages at one wave a SIMD; the two-row-tile form
@@ -54,14 +54,16 @@ constexpr float kLazy = 8.f;
 // inside the hybrid node (after a GDN verify has left ~0.5 GB of snapshot writes dirty in the
 // caches) the plain reads ran at half speed, evicting that data; measured 111 -> 63 us per call.
 constexpr int kKVAux = 2;         // rescale when a row max grows past the reference by 2^8
-static_assert((kPTR & (kPTR - 1)) == 0, "page-table ring");
 static_assert(kVS >= 2 * 16 * kDD * 4, "a stage holds two waves' fp32 output of one row tile at the merge");
 
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 
 struct DecodeDev {
-  int B, NT, splits, pt_stride;
+  int B, NT, pt_stride;
+  int splits;               // > 0: every request in this many equal splits; 0: balanced (see decode_split)
+  int nocut;                // balanced: no request is cut (the launch is followed by no combine)
+  int max_steps;            // steps the page table's width holds: the most a request weighs
   const uint16_t* q;        // bf16 [B*NT, 16, 256]
   const uint8_t* kc;        // e4m3 [slots, 2, 256]
   const uint8_t* vc;
@@ -69,8 +71,9 @@ struct DecodeDev {
   const int32_t* pt;        // [B, pt_stride]
   const int32_t* seqlens;   // [B], new tokens included
   float scale_log2;
-  float* ws_o;              // [B*2*splits][32][256] unnormalised partial outputs
-  float* ws_ml;             // [B*2*splits][2][32]: running max (base 2) and weight sum per row
+  float* ws_o;              // [slots][16 RT][256] unnormalised partial outputs
+  float* ws_ml;             // [slots][2][16 RT]: running max (base 2) and weight sum per row
+  int2* meta;               // balanced: [B] first and last share of each request
   uint16_t* out;            // bf16 [B*NT, 16, 256]
   const uint16_t* gate;     // bf16 [B*NT, 16 * 256] or null: with oq, the o_proj's quantized input
   uint8_t* oq;              // e4m3 [B*NT, 16 * 256] of bf16(out * sigmoid(gate)) per 128-group
@@ -131,9 +134,63 @@ __global__ __launch_bounds__(256) void kv_scatter_kernel(const uint8_t* k8, cons
   *reinterpret_cast<v4i*>((isv ? vc : kc) + dst) = *reinterpret_cast<const v4i*>((isv ? v8 : k8) + src);
 }
 
+// How one call's keys are dealt to the workgroups of a KV head (G of them fit on the chip at once), in
+// steps of kST keys:
+//   pieces  each request in ceil(steps / c) equal pieces, one piece a workgroup, with the smallest c (from
+//           kMinPiece up) that needs no more than G pieces;
+//   line    where there are more requests than G, or a few long ones among many would make that c much
+//           more than an equal share: a request weighs its steps plus ovh (what starting and merging a
+//           run costs beside its steps), half before and half after them, and the line of all
+//           weights is cut into G equal shares.  A share holds the end of one request, whole requests
+//           and the start of another; requests of at most kWhole steps are not cut but belong to the
+//           share that holds their start.
+// Every workgroup works the dealing out for itself from seqlens (about 1 us, before its first key), so a
+// captured launch follows the lengths it finds.  With a fixed number of splits per request, as before,
+// the longest request sets a call's time.  Measured, us a call (fixed -> dealt): 64 x 4 rows over 128 ..
+// 8192 keys 86.9 -> 47.9, 256 x 1 over 20 .. 4000 107.8 -> 58.0, 150 x 4 over 300 .. 6000 134 -> 83.9, 12 x 2
+// over 3000 .. 30000 60.1 -> 41.9; equal lengths: 64 x 4 over 4096 64.5 -> 64.8, 256 x 1 over 4000 177 -> 182
+// (the combine launch, which finds nothing cut).
+// ovh: 4 / 12 / 20 / 28 steps gave 58.5 / 52.2 / 49.3 / 50.3 us on the first of these (two row tiles) and
+// 56.5 / 57.2 / 63.7 / 70.7 on the second (one).  kMinPiece: 2 / 4 / 8 steps 25.0 / 22.5 / 22.9 us for one
+// request of 4 rows over 8000 keys, 14.0 / 14.6 / 16.0 us for one of 1 row over 1000.
+constexpr int kMinPiece = 4, kWhole = 8;
+constexpr int ovh(int RT) { return RT == 1 ? 8 : 16; }
+// share w of nsh begins at total * w / nsh; the share that holds position x
+__device__ __forceinline__ int share_begin(int total, int nsh, int w) { return (int)((int64_t)total * w / nsh); }
+__device__ __forceinline__ int share_of(int total, int nsh, int x) { return (int)((((int64_t)x + 1) * nsh - 1) / total); }
+__device__ __forceinline__ int req_steps(int nk) { return nk > 0 ? (nk + kST - 1) / kST : 0; }
+// Integer sum over the wave, and inclusive scan, without LDS (the plan runs before the first load of a key).
+__device__ __forceinline__ int wave_sum_i(int v) {
+  v += (int)dpp_u32<0xB1>((uint32_t)v);
+  v += (int)dpp_u32<0x4E>((uint32_t)v);
+  v += (int)dpp_u32<0x141>((uint32_t)v);
+  v += (int)dpp_u32<0x140>((uint32_t)v);
+  const auto p16 = __builtin_amdgcn_permlane16_swap((uint32_t)v, (uint32_t)v, false, false);
+  v = (int)(p16[0] + p16[1]);
+  const auto p32 = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false);
+  return (int)(p32[0] + p32[1]);
+}
+__device__ __forceinline__ int wave_scan_i(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr 1, 2, 4, 8: within rows of 16
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  const int r0 = __builtin_amdgcn_readlane(v, 15), r1 = __builtin_amdgcn_readlane(v, 31),
+            r2 = __builtin_amdgcn_readlane(v, 47), row = (threadIdx.x & 63) >> 4;
+  return v + (row > 0 ? r0 : 0) + (row > 1 ? r1 : 0) + (row > 2 ? r2 : 0);
+}
+// threadIdx.x through an empty asm: values derived from it are formed afresh for each run of steps
+// instead of being kept, or spilled, across the step loop of the run before
+__device__ __forceinline__ int run_tid() {
+  int t = (int)threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
 template <int RT, int NS, int WPE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void decode_split_kernel(DecodeDev d) {
-  constexpr int PTD = 2 * NS;
+  constexpr int PTD = 2 * NS, kPTR = PTD <= 4 ? 4 : 8;  // page-table entries ahead, ring entries (one step each)
+  constexpr int kRows = 16 * RT;
   static_assert(NS >= 2 && NS <= 4, "the prologue and the step loop are written out for 2 to 4 stages");
   static_assert(kPTR >= PTD, "the ring holds the entries of every step in flight");
   // one object per stage: the compiler then sees that a stage's DMA does not write what another
@@ -143,19 +200,147 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
   __shared__ __align__(16) uint8_t vs2[NS >= 3 ? kVS : 16];
   __shared__ __align__(16) uint8_t vs3[NS >= 4 ? kVS : 16];
   __shared__ __align__(16) int32_t ptl[4][kPTR][64];
-  __shared__ float mw[4][kDRows], lwv[4][kDRows], rowM[kDRows], rowL[kDRows];
-  const int s = blockIdx.x, h = blockIdx.y, b = blockIdx.z, S = d.splits;
-  const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, lg = lane >> 4;
+  __shared__ float mw[4][kRows], lwv[4][kRows], rowM[kRows], rowL[kRows];
+  // balanced: offset and key count of each of 256 requests, the waves' sums, and the loop's state (in LDS,
+  // so that no register holds it across a run): the share, the next request, the chunk of requests
+  __shared__ int roff[256], rkeys[256], rsum[4], npiece[16];
+  __shared__ int lx0, lx1, ltotal, lnsh, lpc, li, lhi, lc0, lbase;
+  constexpr int kOvh = ovh(RT);
+  const int h = blockIdx.x & 1;
+  {
+    const int t = run_tid();
+    if (d.splits == 0) {
+      const int wg = blockIdx.x >> 1, G = gridDim.x >> 1;
+      const int rk = t < d.B ? d.seqlens[t] : 0, st = min(req_steps(rk), d.max_steps);
+      int w = st;
+      for (int q = t + 256; q < d.B; q += 256) w += min(req_steps(d.seqlens[q]), d.max_steps);
+      w = wave_sum_i(w);
+      if ((t & 63) == 0) rsum[t >> 6] = w;
+      roff[t] = st;
+      rkeys[t] = rk;
+      __syncthreads();
+      const int steps = rsum[0] + rsum[1] + rsum[2] + rsum[3], total = steps + d.B * kOvh;
+      const int c0 = max((steps + G - 1) / G, kMinPiece);
+      int pc = 0;
+      if (d.B <= min(G, 256)) {
+        // 16 piece sizes c0 .. about 2 c0, four a wave
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int kk = 4 * (t >> 6) + k, c = c0 + (c0 * kk + 15) / 16;
+          int n = 0;
+          for (int q = t & 63; q < d.B; q += 64) n += max((roff[q] + c - 1) / c, 1);
+          n = wave_sum_i(n);
+          if ((t & 63) == 0) npiece[kk] = n;
+        }
+        __syncthreads();
+        const int n = npiece[t & 15];
+        const uint64_t fits = __builtin_amdgcn_ballot_w64(n <= G) & 0xffffu;
+        const int k = fits ? __builtin_ctzll(fits) : 0, c = c0 + (c0 * k + 15) / 16;
+        if (fits && c <= total / G + total / (4 * G) + 2) {
+          if (wg >= __builtin_amdgcn_readlane(n, k)) return;
+          pc = c;
+        }
+      }
+      if (t == 0) {
+        lpc = pc;
+        if (pc) lx0 = wg, lx1 = wg + 1;
+        else lx0 = share_begin(total, G, wg), lx1 = share_begin(total, G, wg + 1), ltotal = total, lnsh = G;
+      }
+    }
+    if (t == 0) li = 0, lhi = 0, lc0 = -256, lbase = 0;
+    __syncthreads();
+  }
+  for (;;) {
+  // the run of steps [st0, st0 + nst) of request b, its key count, and the slot of its partial result
+  // (-1: the whole request, written out here)
+  int b, nk, st0, nst, slot;
+  if (d.splits == 0) {
+    const int t = run_tid(), x0 = __builtin_amdgcn_readfirstlane(lx0), x1 = __builtin_amdgcn_readfirstlane(lx1);
+    const int pc = __builtin_amdgcn_readfirstlane(lpc);
+    int i = __builtin_amdgcn_readfirstlane(li);
+    if (i >= __builtin_amdgcn_readfirstlane(lhi)) {  // the next 256 requests
+      const int c0 = __builtin_amdgcn_readfirstlane(lc0) + 256, base = __builtin_amdgcn_readfirstlane(lbase);
+      if (c0 >= d.B || base >= x1) return;
+      const bool in = c0 + t < d.B;
+      const int rk = c0 == 0 ? rkeys[t] : in ? d.seqlens[c0 + t] : 0, st = min(req_steps(rk), d.max_steps);
+      const int w = !in ? 0 : pc ? max((st + pc - 1) / pc, 1) : st + kOvh;
+      const int inc = wave_scan_i(w);
+      __syncthreads();  // the state above has been read
+      if ((t & 63) == 63) rsum[t >> 6] = inc;
+      __syncthreads();
+      int off = base + inc - w;
+#pragma unroll
+      for (int v = 0; v < 3; ++v) off += v < (t >> 6) ? rsum[v] : 0;
+      roff[t] = off;
+      rkeys[t] = rk;
+      // the requests of the chunk that touch the share
+      const int lo = __syncthreads_count(in && off + w <= x0), hi = __syncthreads_count(in && off < x1);
+      if (t == 0) li = lo, lhi = hi, lc0 = c0, lbase = base + rsum[0] + rsum[1] + rsum[2] + rsum[3];
+      __syncthreads();
+      continue;
+    }
+    b = __builtin_amdgcn_readfirstlane(lc0) + i;
+    nk = __builtin_amdgcn_readfirstlane(rkeys[i]);
+    const int off0 = __builtin_amdgcn_readfirstlane(roff[i]), off = off0 + kOvh / 2;  // (line) of its first step
+    const int steps = req_steps(nk);
+    __syncthreads();
+    if (t == 0) li = i + 1;
+    __syncthreads();
+    if (pc) {
+      const int n = max((min(steps, d.max_steps) + pc - 1) / pc, 1), p = x0 - off0, per = steps / n, rem = steps % n;
+      st0 = p * per + min(p, rem);
+      nst = per + (p < rem ? 1 : 0);
+      slot = n > 1 ? 2 * (int)blockIdx.x + (p == 0) : -1;
+      if (p == 0 && t == 0 && h == 0) d.meta[b] = make_int2(x0, x0 + n - 1);
+    } else
+    // (a key count past the page table's width is not cut either: its weight is the table's)
+    if (steps <= kWhole || steps > d.max_steps || d.nocut) {
+      if (off0 < x0) continue;
+      st0 = 0, nst = steps, slot = -1;
+      if (t == 0 && h == 0) d.meta[b] = make_int2(0, 0);
+    } else {
+      const int e = min(x1 - off, steps);
+      st0 = max(x0 - off, 0);
+      nst = e - st0;
+      if (nst <= 0) continue;
+      slot = nst == steps ? -1 : 2 * (int)blockIdx.x + (st0 == 0);
+      if (st0 == 0 && t == 0 && h == 0)
+        d.meta[b] = make_int2((int)blockIdx.x >> 1, share_of(ltotal, lnsh, off + steps - 1));
+    }
+  } else {
+    const int S = d.splits, wg = blockIdx.x >> 1, s = wg % S;
+    if (__builtin_amdgcn_readfirstlane(li)) return;
+    __syncthreads();
+    if (threadIdx.x == 0) li = 1;
+    b = wg / S;
+    nk = d.seqlens[b];
+    const int steps = req_steps(nk), per = steps / S, rem = steps % S;
+    st0 = s * per + min(s, rem);
+    nst = per + (s < rem ? 1 : 0);
+    slot = S > 1 ? (b * kKVH + h) * S + s : -1;
+  }
+  const int tid = run_tid(), lane = tid & 63, l16 = lane & 15, lg = lane >> 4, NT = d.NT;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: LDS bases stay scalar
-  const int NT = d.NT, nk = d.seqlens[b], npre = nk - NT;
-  // steps of the request, the split's share (contiguous), the wave's share of that
-  const int steps = nk > 0 ? (nk + kST - 1) / kST : 0, per = steps / S, rem = steps % S;
-  const int st0 = s * per + min(s, rem), nst = per + (s < rem ? 1 : 0);
+  const int npre = nk - NT;
+  // the wave's share of the run, contiguous
   const int ws0 = st0 + (wave * nst) / 4, ws1 = st0 + ((wave + 1) * nst) / 4;
   const int kbeg = ws0 * kST, kend = min(ws1 * kST, nk);  // the wave's keys [kbeg, kend)
-  const int npad = (ws1 - ws0 + NS - 1) / NS * NS;        // steps run (a multiple of the stages)
   const int kfull = min(kend - 1, npre);  // keys up to here are visible to every query row
-  const int grp = (b * kKVH + h) * S + s;
+  const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc((void*)d.kc, (short)0, (int)d.kv_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc((void*)d.vc, (short)0, (int)d.kv_bytes, 0x00020000);
+  // the request's page-table row through a bounded buffer (an entry past the row reads as slot 0)
+  const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(d.pt + (size_t)b * d.pt_stride), (short)0, 4 * d.pt_stride, 0x00020000);
+  int32_t* ring = &ptl[wave][0][0];
+  // Page-table entries of step j into ring entry j % 8 (lanes 32..63 repeat lanes 0..31).  Keys past
+  // the wave's range take the slot of its last key: their loads are repeats that stay in L2, their
+  // scores are masked and their values are real cache rows (finite), so 0 * V stays 0.
+  auto pt_dma = [&](int j) {
+    const int key = max(min(kbeg + kST * j + (lane & 31), kend - 1), 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(prs, ring + (j & (kPTR - 1)) * 64, 4, 4 * key, 0, 0, 0);
+  };
+  // the entries of the prologue's steps first: the query rows below come with them in one round trip
+  for (int j = 0; j <= PTD - NS; ++j) pt_dma(j);
   // query fragments (score operand B): column 16 rt + l16 = query row (token row / 8, head
   // h * 8 + row % 8), dims 128 kb + 32 lg .. +31 rounded to e4m3; rows of tokens past NT are zero
   v8i qb[RT][2];
@@ -181,19 +366,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
       qb[rt][kb] = v8i{w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7]};
     }
   }
-  const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc((void*)d.kc, (short)0, (int)d.kv_bytes, 0x00020000);
-  const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc((void*)d.vc, (short)0, (int)d.kv_bytes, 0x00020000);
-  // the request's page-table row through a bounded buffer (an entry past the row reads as slot 0)
-  const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(d.pt + (size_t)b * d.pt_stride), (short)0, 4 * d.pt_stride, 0x00020000);
-  int32_t* ring = &ptl[wave][0][0];
-  // Page-table entries of step j into ring entry j % 8 (lanes 32..63 repeat lanes 0..31).  Keys past
-  // the wave's range take the slot of its last key: their loads are repeats that stay in L2, their
-  // scores are masked and their values are real cache rows (finite), so 0 * V stays 0.
-  auto pt_dma = [&](int j) {
-    const int key = max(min(kbeg + kST * j + (lane & 31), kend - 1), 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(prs, ring + (j & (kPTR - 1)) * 64, 4, 4 * key, 0, 0, 0);
-  };
   // Step j into stage Q: the 32 keys' rows as score operand A (kf[Q][kt]: key 16 kt + l16, dims
   // 128 half + 32 lg ..), and the 32 value rows into the wave's LDS rows: DMA call m writes rows
   // 4 m .. 4 m + 3 with key 16 (m & 1) + 4 (m >> 1) + (row % 4), so rows 8 g .. 8 g + 7 hold keys
@@ -340,9 +512,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
       for (int rt = 0; rt < RT; ++rt) o[rt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv, pb[rt], o[rt][dt], 0, 0, 0);
     }
   };
-  // prologue: entries of steps 0 .. PTD - NS, then the first NS - 1 steps' requests, each
+  // prologue: the entries of steps 0 .. PTD - NS have landed; the first NS - 1 steps' requests, each
   // followed by the page-table DMA PTD steps ahead (the order every step keeps)
-  for (int j = 0; j <= PTD - NS; ++j) pt_dma(j);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   fetch(0, std::integral_constant<int, 0>{});
   pt_dma(PTD - NS + 1);
@@ -362,11 +533,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
     compute(j, qc);
     __builtin_amdgcn_sched_barrier(0);  // and the next step's requests stay after it
   };
-  for (int j = 0; j < npad; j += NS) {
+  const int nj = ws1 - ws0;
+  for (int j = 0; j < nj; j += NS) {
     step(j, std::integral_constant<int, 0>{});
+    if (j + 1 >= nj) break;
     step(j + 1, std::integral_constant<int, 1>{});
-    if constexpr (NS >= 3) step(j + 2, std::integral_constant<int, 2>{});
-    if constexpr (NS == 4) step(j + 3, std::integral_constant<int, 3>{});
+    if constexpr (NS >= 3) {
+      if (j + 2 >= nj) break;
+      step(j + 2, std::integral_constant<int, 2>{});
+    }
+    if constexpr (NS == 4) {
+      if (j + 3 >= nj) break;
+      step(j + 3, std::integral_constant<int, 3>{});
+    }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   // merge the four waves: M = max of the waves' maxima, L = sum of exp2(m_w - M) l_w; per row
@@ -383,19 +562,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
     }
   }
   __syncthreads();
-  if (tid < kDRows) {
+  if (tid < kRows) {
     const int row = tid;
-    float M = -1e30f, L = 0.f;
-    if (row < 16 * RT) {
-      M = fmaxf(fmaxf(mw[0][row], mw[1][row]), fmaxf(mw[2][row], mw[3][row]));
+    const float M = fmaxf(fmaxf(mw[0][row], mw[1][row]), fmaxf(mw[2][row], mw[3][row]));
+    float L = 0.f;
 #pragma unroll
-      for (int w = 0; w < 4; ++w) L += __builtin_amdgcn_exp2f(mw[w][row] - M) * lwv[w][row];
-    }
+    for (int w = 0; w < 4; ++w) L += __builtin_amdgcn_exp2f(mw[w][row] - M) * lwv[w][row];
     rowM[row] = M;
     rowL[row] = L;
-    if (S > 1) {
-      d.ws_ml[(size_t)grp * 2 * kDRows + row] = M;
-      d.ws_ml[(size_t)grp * 2 * kDRows + kDRows + row] = L;
+    if (slot >= 0) {
+      d.ws_ml[(size_t)slot * 2 * kRows + row] = M;
+      d.ws_ml[(size_t)slot * 2 * kRows + kRows + row] = L;
     }
   }
   __syncthreads();
@@ -404,7 +581,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
   const float* o1 = reinterpret_cast<const float*>(vs0 + kVS / 2);
   const float* o2 = reinterpret_cast<const float*>(vs1);
   const float* o3 = reinterpret_cast<const float*>(vs1 + kVS / 2);
-  float* wo = d.ws_o + (size_t)grp * kDRows * kDD;
+  float* wo = d.ws_o + (size_t)(slot >= 0 ? slot : 0) * kRows * kDD;
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
     if (rt > 0) __syncthreads();  // the previous tile's sums have read the buffers
@@ -419,7 +596,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
       const int r = e / (kDD / 4), c = e % (kDD / 4), at = r * kDD + 4 * (c ^ r), row = 16 * rt + r;
       const v4f a = (*reinterpret_cast<const v4f*>(o0 + at) + *reinterpret_cast<const v4f*>(o1 + at)) +
                     (*reinterpret_cast<const v4f*>(o2 + at) + *reinterpret_cast<const v4f*>(o3 + at));
-      if (S > 1) {
+      if (slot >= 0) {
         *reinterpret_cast<v4f*>(wo + row * kDD + 4 * c) = a;
       } else {
         const float L = rowL[row], il = L > 0.f ? 1.f / L : 0.f;
@@ -431,43 +608,91 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
       }
     }
   }
+  __syncthreads();  // every wave has read the buffers before the next run's requests write them
+  }
 }
 
-// out = bf16(sum_s exp2(m_s - M) o_s / L), L = sum_s exp2(m_s - M) l_s, splits in order; one
-// thread per 4 dims of one query row (rows b, t, head over the batch)
-__global__ __launch_bounds__(256) void decode_combine_kernel(DecodeDev d) {
-  const int e = blockIdx.x * 256 + threadIdx.x, NT = d.NT, S = d.splits;
-  if (e >= d.B * NT * kQH * (kDD / 4)) return;
-  const int c = e % (kDD / 4), qr = e / (kDD / 4);  // qr = (b * NT + t) * 16 + head
-  const int head = qr % kQH, bt = qr / kQH, t = bt % NT, b = bt / NT;
-  const int h = head / kGQ, gr = t * kGQ + head % kGQ, g0 = (b * kKVH + h) * S;
-  float M = -1e30f;  // the split kernel's maxima are finite (-1e30 for a split with no visible key)
-  for (int s = 0; s < S; ++s) M = fmaxf(M, d.ws_ml[(size_t)(g0 + s) * 2 * kDRows + gr]);
+// out = bf16(sum_p exp2(m_p - M) o_p / L), L = sum_p exp2(m_p - M) l_p over the pieces of a request.
+// WPR waves per query row (b, t, head), each lane 4 dims: wave v adds pieces v, v + WPR, ... with four
+// loads in flight, and the waves' sums meet in LDS in wave order.  Latency-bound: one wave a row where a
+// request has a few pieces; 4 or 16 where a call of few requests has them in tens (3 requests of 42
+// splits: 23.3 us for one thread per 4 dims walking the splits, 5.5 us for 16 waves).  kRows: rows of a slot.
+template <int WPR>
+__global__ __launch_bounds__(WPR == 4 ? 256 : 1024) void decode_combine_kernel(DecodeDev d, int kRows) {
+  constexpr int RPB = WPR > 1 ? 1 : 16;  // rows a workgroup (one token's)
+  __shared__ v4f sums[WPR > 1 ? WPR : 1][64];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, c = lane;
+  const int qr = blockIdx.x * RPB + (WPR > 1 ? 0 : wave), wv = WPR > 1 ? wave : 0;  // qr = (b * NT + t) * 16 + head
+  const int NT = d.NT, head = qr % kQH, bt = qr / kQH, t = bt % NT, b = bt / NT;
+  if (b >= d.B) return;
+  const int h = head / kGQ, gr = t * kGQ + head % kGQ;
+  int n, g0, gstep;  // piece p of the request is at slot g0 + p * gstep, the first at g0 + first
+  int first = 0;
+  if (d.splits > 0) {
+    n = d.splits, g0 = (b * kKVH + h) * n, gstep = 1;
+  } else {
+    const int2 w = d.meta[b];
+    n = w.y - w.x + 1;
+    if (n <= 1) return;  // written by the split kernel
+    g0 = 2 * (2 * w.x + h), gstep = 4, first = 1;
+  }
+  auto slot = [&](int p) { return (size_t)(g0 + p * gstep + (p == 0 ? first : 0)); };
+  float M = -1e30f;  // the pieces' maxima are finite (-1e30 for one with no visible key)
+  for (int p = lane; p < n; p += 64) M = fmaxf(M, d.ws_ml[slot(p) * 2 * kRows + gr]);
+  M = wave_max(M);
   float L = 0.f;
   v4f a = {0.f, 0.f, 0.f, 0.f};
-  for (int s = 0; s < S; ++s) {
-    const float ms = d.ws_ml[(size_t)(g0 + s) * 2 * kDRows + gr];
-    const float w = exp2f(ms - M);
-    L += w * d.ws_ml[(size_t)(g0 + s) * 2 * kDRows + kDRows + gr];
-    a += w * *reinterpret_cast<const v4f*>(d.ws_o + ((size_t)(g0 + s) * kDRows + gr) * kDD + 4 * c);
+  for (int p0 = 0; p0 < n; p0 += 64) {
+    const int pl = min(p0 + lane, n - 1);
+    const float w = p0 + lane < n ? exp2f(d.ws_ml[slot(pl) * 2 * kRows + gr] - M) : 0.f;
+    L += w * d.ws_ml[slot(pl) * 2 * kRows + kRows + gr];
+    const int m = min(64, n - p0);
+    for (int q0 = wv; q0 < m; q0 += 4 * WPR) {
+      v4f o[4];
+      float wq[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int q = q0 + k * WPR, qc = min(q, m - 1);
+        o[k] = *reinterpret_cast<const v4f*>(d.ws_o + (slot(p0 + qc) * kRows + gr) * kDD + 4 * c);
+        const float r = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), qc));
+        wq[k] = q < m ? r : 0.f;
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) a += wq[k] * o[k];
+    }
+  }
+  L = wave_sum_bfly(L);
+  if constexpr (WPR > 1) {
+    sums[wave][lane] = a;
+    __syncthreads();
+    if (wave != 0) return;
+#pragma unroll
+    for (int v = 1; v < WPR; ++v) a += sums[v][lane];
   }
   const float il = L > 0.f ? 1.f / L : 0.f;
   const uint32_t o01 = pack_bf2(a[0] * il, a[1] * il), o23 = pack_bf2(a[2] * il, a[3] * il);
   *reinterpret_cast<uint2*>(d.out + (size_t)qr * kDD + 4 * c) = make_uint2(o01, o23);
-  // 64 consecutive threads are one row (the row count is whole waves): lanes 0-31 / 32-63 its groups
-  if (d.oq) gated_e4m3(d, qr / kQH, head, c, o01, o23);
+  // the wave holds the row: lanes 0-31 / 32-63 its two 128-groups
+  if (d.oq) gated_e4m3(d, bt, head, c, o01, o23);
 }
 
-int decode_splits(int B, int splits) {
-  if (splits > 0) return min(splits, 64);
+int decode_cus() {
   int cus = 256, dev = 0;
   if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  return max(1, min(64, cus / (B * kKVH)));
+  return cus;
 }
-size_t decode_ws_bytes(int B, int S) {
-  return align_up(sizeof(float) * (size_t)B * kKVH * S * kDRows * kDD, 256) +
-         align_up(sizeof(float) * (size_t)B * kKVH * S * 2 * kDRows, 256);
+// Equal splits per request: as asked for, or (a workspace too small for the balanced form) enough to
+// give every CU a workgroup.
+int decode_splits(int B, int splits) {
+  if (splits > 0) return min(splits, 64);
+  return max(1, min(64, decode_cus() / (B * kKVH)));
 }
+size_t decode_slots_bytes(size_t slots) {  // slots of kDRows rows (or twice as many of half the rows)
+  return align_up(sizeof(float) * slots * kDRows * kDD, 256) + align_up(sizeof(float) * slots * 2 * kDRows, 256);
+}
+size_t decode_ws_bytes(int B, int S) { return decode_slots_bytes((size_t)B * kKVH * S); }
+// Balanced: two slots a workgroup, one workgroup a CU of kDRows rows or two a CU of half the rows
+size_t decode_bal_bytes(int B) { return decode_slots_bytes(2 * (size_t)decode_cus()) + align_up(sizeof(int2) * (size_t)B, 256); }
 
 }  // namespace
 }  // namespace q36
@@ -475,7 +700,8 @@ size_t decode_ws_bytes(int B, int S) {
 using namespace q36;
 
 extern "C" size_t q36_attn_decode_workspace_bytes(int32_t B, int32_t splits) {
-  return decode_ws_bytes(B, decode_splits(B, splits));
+  return splits > 0 ? decode_ws_bytes(B, decode_splits(B, splits))
+                    : std::max(decode_bal_bytes(B), decode_ws_bytes(B, decode_splits(B, 0)));
 }
 
 extern "C" int q36_attn_decode(const q36_decode_args* a, q36_stream_t stream) {
@@ -498,8 +724,13 @@ extern "C" int q36_attn_decode(const q36_decode_args* a, q36_stream_t stream) {
   Q36_REQUIRE(!a->oq || ((reinterpret_cast<uintptr_t>(a->gate) & 7u) == 0 &&
                          (reinterpret_cast<uintptr_t>(a->oq) & 3u) == 0 && (reinterpret_cast<uintptr_t>(a->oqs) & 3u) == 0),
               "q36_attn_decode: gate must be 8-byte, oq and oqs 4-byte aligned");
-  const int S = decode_splits(a->B, a->splits);
-  const size_t need = decode_ws_bytes(a->B, S);
+  // balanced unless a split count was asked for (or the workspace holds only the equal splits', or the
+  // line's length might not fit 31 bits)
+  const int max_steps = (a->pt_stride - 1) / kST + 1;
+  const bool bal = a->splits <= 0 && a->workspace_bytes >= decode_bal_bytes(a->B) &&
+                   (int64_t)a->B * ((int64_t)max_steps + ovh(2)) < (1 << 30);
+  const int S = bal ? 0 : decode_splits(a->B, a->splits);
+  const size_t need = bal ? decode_bal_bytes(a->B) : decode_ws_bytes(a->B, S);
   Q36_REQUIRE(a->workspace_bytes >= need, "q36_attn_decode: workspace of %zu bytes < %zu required", a->workspace_bytes,
               need);
   hipStream_t st = static_cast<hipStream_t>(stream);
@@ -510,17 +741,35 @@ extern "C" int q36_attn_decode(const q36_decode_args* a, q36_stream_t stream) {
                                                             static_cast<const uint8_t*>(a->v_new), a->out_loc, T, a->num_slots,
                                                             static_cast<uint8_t*>(a->k_cache),
                                                             static_cast<uint8_t*>(a->v_cache));
-  DecodeDev d{a->B, a->NT, S, a->pt_stride,
+  const bool one = a->NT <= 2;  // one row tile, two workgroups a CU
+  const int cus = decode_cus(), slots = bal ? 2 * cus : a->B * kKVH * S;  // of kDRows rows
+  // balanced: as many workgroups per KV head as the chip holds at once, and no more than pieces of a
+  // table of this width; a table so narrow that no request is cut needs no combine
+  const int nocut = max_steps <= kMinPiece;
+  const int64_t pieces = (int64_t)a->B * ((max_steps - 1) / kMinPiece + 1);
+  const int shares = (int)std::min<int64_t>(std::max(1, (one ? kDecWPE1 : 1) * cus / kKVH), pieces);
+  DecodeDev d{a->B, a->NT, a->pt_stride, S, nocut, max_steps,
               static_cast<const uint16_t*>(a->q), static_cast<const uint8_t*>(a->k_cache),
               static_cast<const uint8_t*>(a->v_cache), (int64_t)a->num_slots * kKVH * kDD, a->page_table, a->seqlens,
               a->scale * 1.44269504088896340736f, reinterpret_cast<float*>(ws),
-              reinterpret_cast<float*>(ws + align_up(sizeof(float) * (size_t)a->B * kKVH * S * kDRows * kDD, 256)),
+              reinterpret_cast<float*>(ws + align_up(sizeof(float) * (size_t)slots * kDRows * kDD, 256)),
+              reinterpret_cast<int2*>(ws + decode_slots_bytes(slots)),
               static_cast<uint16_t*>(a->out), static_cast<const uint16_t*>(a->gate), static_cast<uint8_t*>(a->oq),
               a->oqs};
-  if (a->NT <= 2)
-    decode_split_kernel<1, kDecNS1, kDecWPE1><<<dim3(S, kKVH, a->B), 256, 0, st>>>(d);
+  const unsigned grid = kKVH * (unsigned)(bal ? shares : a->B * S);
+  if (one)
+    decode_split_kernel<1, kDecNS1, kDecWPE1><<<grid, 256, 0, st>>>(d);
   else
-    decode_split_kernel<2, kDecNS2, 1><<<dim3(S, kKVH, a->B), 256, 0, st>>>(d);
-  if (S > 1) decode_combine_kernel<<<(a->B * a->NT * kQH * (kDD / 4) + 255) / 256, 256, 0, st>>>(d);
+    decode_split_kernel<2, kDecNS2, 1><<<grid, 256, 0, st>>>(d);
+  if (bal ? !nocut : S > 1) {
+    // waves per query row by the pieces an average request has
+    const int rows = T * kQH, slot_rows = one ? 16 : kDRows, per = bal ? shares / a->B : S;
+    if (per >= 32)
+      decode_combine_kernel<16><<<rows, 1024, 0, st>>>(d, slot_rows);
+    else if (per >= 4)
+      decode_combine_kernel<4><<<rows, 256, 0, st>>>(d, slot_rows);
+    else
+      decode_combine_kernel<1><<<T, 1024, 0, st>>>(d, slot_rows);
+  }
   return check_launch("q36_attn_decode");
 }

@@ -146,9 +146,9 @@ def attn_oproj(attn, gate, w: AttnWeights, ws: Workspace, out=None, stream=None,
 
 
 class DecodeWorkspace:
-    """Split partials of q36_attn_decode for up to B_max requests at a fixed split count
-    (0 = the library's default min(64, CUs / (B * 2)), resolved per call: the buffer is sized for
-    the largest count any B <= B_max can take)."""
+    """Partials of q36_attn_decode for up to B_max requests: splits 0 (the default) deals the keys of
+    all requests evenly over the chip, a positive count cuts each request into that many.  The buffer is
+    sized for the most any B <= B_max can take."""
 
     def __init__(self, B_max: int, device, splits: int = 0):
         L = _lib.lib()

@@ -195,3 +195,50 @@ def test_decode_rejects_bad_shapes(attn, dev):
         attn.attn_decode(q8, d["kc"], d["vc"], d["pt"], d["seqlens"], 8, SCALE, ws)
     with pytest.raises(RuntimeError, match="HQ=8"):
         attn.attn_decode(d["q"][:, :8].contiguous(), d["kc"], d["vc"], d["pt"], d["seqlens"], 4, SCALE, ws)
+
+
+def _ragged(B, lo, hi, longs, seed):
+    g = torch.Generator().manual_seed(seed)
+    n = torch.randint(lo, hi + 1, (B,), generator=g).tolist()
+    for i, v in enumerate(longs):
+        n[(7 + 31 * i) % B] = v
+    return n
+
+
+@pytest.mark.parametrize("NT,seqlens", [
+    (4, [4]),                                            # one key step
+    (1, [128]), (1, [129]),                              # the widest table with no cut, and one key more
+    (2, [2, 40, 256, 257, 3000]),                        # pieces of one request over many workgroups
+    (4, _ragged(64, 4, 700, [2500, 3000], 1)),           # pieces, most requests one piece
+    (4, _ragged(128, 200, 260, [4000], 2)),              # as many requests as workgroups, one long: the line
+    (3, _ragged(140, 3, 520, [2100, 900], 3)),           # more requests than workgroups
+    (1, _ragged(300, 1, 300, [1700, 2000, 1025], 4)),    # more requests than one scan holds
+], ids=["1step", "128", "129", "5", "64", "128long", "140", "300"])
+def test_decode_balanced_shares(attn, oracle_mod, dev, NT, seqlens):
+    """The default dealing of the keys to the workgroups (no split count given), within the bar of the
+    fixed splits: same arithmetic, another order of the fp32 sums."""
+    print(f"attn_decode balanced NT={NT} B={len(seqlens)}", flush=True)
+    h = _make(len(seqlens), NT, seqlens, seed=3 * NT + len(seqlens))
+    h["pt"] = h["pt"][:, :max(seqlens)].contiguous()     # (the 128-key table: exactly its four steps wide)
+    out, _ = _run(attn, h, NT, dev)
+    _check(out, _oracle(oracle_mod, h, NT), f"balanced NT={NT} B={len(seqlens)}")
+    # a workspace that holds only the fixed splits' partials is still served
+    ws = attn.DecodeWorkspace(len(seqlens), dev, splits=1)
+    ws.splits = 0
+    d = {k: h[k].to(dev) for k in ("q", "kc", "vc", "pt", "seqlens")}
+    if ws.buf.numel() >= 66048 * len(seqlens) * max(1, min(64, 128 // len(seqlens))):
+        out2 = attn.attn_decode(d["q"], d["kc"], d["vc"], d["pt"], d["seqlens"], NT, SCALE, ws)
+        assert_bf16_close(bits16(out2).reshape(-1, D), bits16(out).reshape(-1, D), 2e-3, "fixed splits")
+
+
+def test_decode_balanced_empty_requests(attn, oracle_mod, dev):
+    """Requests without keys (a padded batch's) give zeros and leave the others as they are."""
+    NT, seqlens = 2, [70, 0, 900, 0, 2, 1500]
+    h = _make(6, NT, [max(n, NT) for n in seqlens], seed=41)
+    ref = _oracle(oracle_mod, h, NT).reshape(6, -1, D)
+    h["seqlens"] = torch.tensor(seqlens, dtype=torch.int32)
+    out, _ = _run(attn, h, NT, dev)
+    got = bits16(out).reshape(6, -1, D)
+    assert not got[[1, 3]].any()
+    keep = [0, 2, 4, 5]
+    assert_bf16_close(got[keep].reshape(-1, D), ref[keep].reshape(-1, D), 1e-2, "beside empty requests")
