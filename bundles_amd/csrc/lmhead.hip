@@ -12,19 +12,16 @@
 // Kernels:
 //   lmh_prep   one wave per row: norm (sum of squares in the fixed 64-lane order), int8 quant,
 //              and the row's argmax key reset to 0.
-//   lmh_gemm   persistent, one 512-thread workgroup per CU walking 256 x 256 output tiles (8 waves,
-//              two a SIMD, each 128 vocab rows x 64 tokens, 32x32x32 int8 MFMAs with the weights as
-//              operand A, int32 accumulators); K in 64-byte steps through LDS rings filled by
-//              buffer loads straight into LDS (weights 6 stages, loaded by four waves six steps
-//              ahead; activations 3 stages, loaded by the other four), fragments double-buffered
-//              in registers, and the next tile's first steps requested before the epilogue.
-//              Epilogue: bf16 logits, the
-//              first column of each row's largest value folded into an order-preserving key, and one
-//              64-bit atomic max per row and tile: the result does not depend on the order the
-//              workgroups finish in.  lmh_gemm_logits: the same, writing the bf16 logits too.
+//   lmh_gemm   persistent, two workgroups of 4 waves a CU walking tiles of 256 (or 128) vocab rows x 128
+//              activation rows: 16x16x64 int8 MFMAs with the weights as operand A, int32 accumulators;
+//              the weights stream into registers, the activations through an LDS ring.  Epilogue: bf16
+//              logits (written out when asked for), the first column of each row's largest value
+//              folded into an order-preserving key, and one 64-bit atomic max per row and tile: the
+//              result does not depend on the order the workgroups finish in.
 //   lmh_ids    key -> token id.
-// Tile order: two row groups of XCDs (see lmh_gemm_body); the row tiles of one vocab tile run side
+// Tile order: two row groups of XCDs (see lmh_gemm); the row tiles of one vocab tile run side
 // by side on one XCD, whose L2 serves them the weight tile and keeps their activations resident.
+#include <algorithm>
 #include <type_traits>
 
 #include "q36_device.h"
@@ -35,14 +32,17 @@ namespace q36 {
 namespace {
 
 constexpr int kLH = 2048;       // hidden (K)
-constexpr int kBM = 256, kBN = 256, kBK = 64, kNK = kLH / kBK;  // 32 K steps
-constexpr int kLmhWaves = 8;  // waves of the GEMM workgroup: two a SIMD
-constexpr int kNSA = 3, kNSB = 6;  // LDS ring stages of the activations and of the weights
+constexpr int kNK = kLH / 64;  // 32 K steps of 64 columns
+constexpr int kNS = 4;         // LDS ring stages of the activations, two steps each
+// Cache policy of the logits' stores: the default (non-temporal: 2048 rows 652 against 626 us with bf16
+// logits, 823 against 755 us with fp32 ones)
+constexpr int kLogitAux = 0;
 
 struct LmhDev {
   int R, V;
-  int Rs;   // activation rows in xq: R (one term) or 64 * ceil(R / 32) (two terms, see act_row)
+  int Rs;   // activation rows in xq: R (one term) or two terms' rows in whole groups (see act_row)
   int x2;   // two activation terms (Q36_LMH_W8A8X2)
+  int tiled;  // wq (and then xq) in the tile order
   int w16;  // W8A16: the prep writes the (normed) bf16 rows to xq instead of quantizing them
   const uint16_t* h;
   const uint16_t* norm_w;
@@ -57,13 +57,20 @@ struct LmhDev {
   unsigned long long* keys;
 };
 
-// Row of the activation codes holding term `term` of token r.  One term: row r.  Two terms: the
-// tokens go in groups of 32, each group's term-1 rows followed by its term-2 rows (row 64 (r / 32) +
-// 32 term + r % 32), so one lane of the GEMM holds both terms of the same token in its accumulators.
-__host__ __device__ __forceinline__ int act_row(int r, int term, int x2) {
-  return x2 ? 64 * (r >> 5) + 32 * term + (r & 31) : r;
+// Row of the activation codes holding term `term` of token r.  One term: row r.  Two terms: the tokens go
+// in groups of G (16 for the tile-order codes' GEMM, 32 for the row-major ones': its MFMA's rows), each
+// group's term-1 rows followed by its term-2 rows, so one lane of the GEMM holds both terms of the same
+// token in its accumulators.
+__host__ __device__ __forceinline__ int act_row(int r, int term, int x2, int G) {
+  return x2 ? 2 * G * (r / G) + G * term + r % G : r;
 }
-__host__ __device__ __forceinline__ int act_rows(int R, int x2) { return x2 ? 64 * ((R + 31) >> 5) : R; }
+__host__ __device__ __forceinline__ int act_rows(int R, int x2, int G) { return x2 ? 2 * G * ((R + G - 1) / G) : R; }
+// Byte of the activation codes (row, column c): row-major, or the tile order of q36_tile_w16, each 16-row x
+// 64-column piece 1 KB contiguous (the 16x16x64 MFMA's operand layout).
+__device__ __forceinline__ size_t act_at(int row, int c, int tiled) {
+  return tiled ? ((size_t)(row >> 4) * kNK + (c >> 6)) * 1024 + 16 * ((row & 15) + 16 * ((c >> 4) & 3)) + (c & 15)
+               : (size_t)row * kLH + c;
+}
 
 // one wave (and workgroup) per row: a batch's rows spread over as many CUs
 __global__ __launch_bounds__(64) void lmh_prep_kernel(LmhDev d) {
@@ -120,7 +127,7 @@ __global__ __launch_bounds__(64) void lmh_prep_kernel(LmhDev d) {
       for (int i = 0; i < 8; ++i) m = fmaxf(m, fabsf(y[j][i]));
     m = wave_max(m);
     const float sc = m / 127.f, safe = m > 0.f ? sc : 1.f;
-    const int row = act_row(r, term, d.x2);
+    const int row = act_row(r, term, d.x2, d.tiled ? 16 : 32);
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
       uint32_t wd[2] = {0u, 0u};
@@ -130,18 +137,12 @@ __global__ __launch_bounds__(64) void lmh_prep_kernel(LmhDev d) {
         wd[i >> 2] |= ((uint32_t)qv & 0xffu) << (8 * (i & 3));
         y[j][i] = __builtin_fmaf(-(float)qv, sc, y[j][i]);
       }
-      *reinterpret_cast<uint2*>(d.xq + (size_t)row * kLH + 8 * (lane + 64 * j)) = make_uint2(wd[0], wd[1]);
+      *reinterpret_cast<uint2*>(d.xq + act_at(row, 8 * (lane + 64 * j), d.tiled)) = make_uint2(wd[0], wd[1]);
     }
     if (lane == 0) d.xs[row] = sc;
   }
   if (lane == 0) d.keys[r] = 0ull;
 }
-
-// LDS position of 16-byte chunk kc (0..3) of tile row c in one K step: rows are 64 bytes, unpadded,
-// with the chunk order xor-swizzled by ((c >> 1) & 3) ^ ((c >> 3) & 1).  A fragment read takes chunk
-// kc of consecutive rows; LDS serves a 16-byte read 16 lanes at a time over 64 banks, and with this
-// swizzle any 16 consecutive rows (and any 8) land in distinct 16-byte bank windows.
-__device__ __forceinline__ int bswz(int c, int kc) { return c * kBK + ((kc ^ ((c >> 1) & 3) ^ ((c >> 3) & 1)) << 4); }
 
 template <int N>
 using ic = std::integral_constant<int, N>;
@@ -167,6 +168,284 @@ __device__ __forceinline__ void wait_vm() {
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
 
+// 16 bytes a lane straight into LDS (a function of its own: the host pass does not know the size)
+__device__ __forceinline__ void lds_dma16(__amdgpu_buffer_rsrc_t rs, void* lds, int voff, int soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, lds, 16, voff, soff, 0, 0);
+}
+// row groups of XCDs: two when there are at least 8 row tiles, evenly split
+__host__ __device__ __forceinline__ int lmh_groups(int nrt) { return nrt >= 8 && nrt % 2 == 0 ? 2 : 1; }
+
+// The codes in the tile order (what the logits node keeps).
+// Persistent GEMM + argmax: workgroups of 4 waves, two a CU, walk their XCD's tiles of 64 VT vocab rows x 16 TB
+// activation rows.  A wave owns 16 VT vocab rows (VT 16-row MFMA tiles) against every row of the tile
+// (TB tiles): VT TB accumulators of v_mfma_i32_16x16x64_i8 with the weights as operand A.
+//
+// K goes in 64-column steps, two a stage.  The weights stream straight into registers, WD steps ahead
+// (in the tile order a fragment is 1 KB contiguous, and no other wave of the workgroup needs it); the
+// activations, which lmh_prep writes in the same order, go through an LDS ring of kNS stages filled by
+// buffer loads straight into LDS, each fragment read by the four waves as 1 KB contiguous.  A wave
+// reads its fragments three tiles ahead of their MFMAs.  Nothing drains at a tile's end: the loads of
+// the next tile's first steps are in flight while the epilogue runs, and the CU's other workgroup keeps the
+// matrix cores busy.  One barrier a stage, in its middle: before it each wave waits for its own loads
+// of the next stage, after it every wave may read that stage and the one before the current is free.
+//
+// Why this split: with both operands in LDS (8 waves, 128 x 64 a wave) a step's 96 KB of fragment reads and
+// 32 KB of writes took as long as its MFMAs; with the weights in registers a CU reads 64 KB and writes 16.
+// What bounds it now, at 2048 rows: the power the MFMAs draw (a loop of these MFMAs alone with one LDS
+// read per four runs at 3.5 POP/s on random codes and 4.6 on zeros: 367 us for this product), the
+// epilogue (about 30 us) and the weights' latency behind the logits' stores.  Measured, us a call
+// (before -> now): 2048 rows with bf16 logits 743 -> 585, fp32 800 -> 705, none 548 -> 503; 256 rows two
+// terms 175 -> 153 bf16, 153 -> 139 none; 150 rows two terms fp32 168 -> 133; 64 rows 93 -> 70; 300 rows
+// one term 139 -> 114.  A token's 64 logits of a wave go out as 64-byte runs (16-byte pieces before).
+//
+// The XCDs form ngrp row groups (2 when the row tiles split evenly, else 1): XCD x serves the rpg = nrt / ngrp
+// row tiles of group x % ngrp and the vocab tiles v = x / ngrp (mod 8 / ngrp).  Its workgroups take
+// tiles j = loc, loc + nloc, ... (loc = blockIdx / 8, nloc = gridDim / 8), tile j being row tile
+// (x % ngrp) * rpg + j % rpg of vocab tile (j / rpg) * (8 / ngrp) + x / ngrp: the row tiles of one
+// vocab tile run side by side on one XCD (its weight tile comes from HBM once per XCD), and an
+// XCD's activations (2 MB at 2048 rows) stay resident in its L2 while the weights stream through.
+//
+// STORE: 0 no logits, 1 bf16 logits, 2 fp32 logits (the bf16-rounded values widened).
+constexpr int lmh_wd(int VT, int TB) { return VT * TB <= 16 ? 8 : 4; }  // weight steps in flight (divides the 32 steps)
+// Whether step k requests the weights of step k + WD: past the tile's end only the first half of the
+// next tile's first WD steps (the rest after the epilogue, across which they would spill).
+constexpr bool lmh_loads(int k, int WD) { return k + WD < kNK || k + WD - kNK < WD / 2; }
+// Vector-memory operations of a wave that are at least newer than its loads of stage k / 2 + 1 at the barrier
+// of (even) step k: those loads went out after the barrier of step k - 4; since then, per step, VT weight
+// loads before the barrier and C activation loads after it (even steps), and between two tiles the
+// weights that waited for the epilogue.  (More, never fewer: the epilogue's stores, and the first tile's
+// weights, which are all requested ahead.  Counting the stores too, with a branch for the first tile,
+// made the K loop spill: 2048 rows with bf16 logits 578 -> 632 us.)
+constexpr int lmh_newer(int k, int VT, int WD, int C) {
+  int n = 0;
+  for (int j = k - 3; j <= k; ++j) n += lmh_loads((j + kNK) % kNK, WD) ? VT : 0;
+  return n + C + (k < 4 ? VT * (WD / 2) : 0);
+}
+static_assert(lmh_newer(8, 4, 4, 4) == 20 && lmh_newer(30, 4, 4, 4) == 16 && lmh_newer(0, 4, 4, 4) == 20, "counts");
+
+template <int VT, int TB, bool X2, int STORE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void lmh_gemm_kernel(LmhDev d) {
+  constexpr int kTN = 64 * VT, WD = lmh_wd(VT, TB), C = TB / 2, TR = 16 * TB, kStage = TB * 2048;
+  static_assert(TB % 2 == 0 && kNK % WD == 0 && (kNK / 2) % kNS == 0 && kNS == 4, "shape");
+  __shared__ __align__(1024) int8_t s0[kStage], s1[kStage], s2[kStage], s3[kStage];
+  __shared__ __align__(16) float wsc[256], xsc[256];
+  __shared__ uint32_t rkey[4][TR];
+  auto stage = [&](auto st) -> int8_t* {
+    constexpr int S = decltype(st)::value & (kNS - 1);
+    return S == 0 ? s0 : S == 1 ? s1 : S == 2 ? s2 : s3;
+  };
+  const int nvt = (d.V + kTN - 1) / kTN, nrt = (d.Rs + TR - 1) / TR;
+  const int xcd = blockIdx.x & 7, loc = blockIdx.x >> 3, nloc = gridDim.x >> 3;
+  const int ngrp = lmh_groups(nrt), rpg = nrt / ngrp, vstep = 8 / ngrp;
+  const int rbase = (xcd % ngrp) * rpg, vres = xcd / ngrp;
+  const int ntile = rpg * ((nvt - vres + vstep - 1) / vstep);  // the XCD's
+  int j = loc;
+  if (j >= ntile) return;
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  // A tile's first activation row and vocab row, and the last of its 16-row tiles of each that exists: a load
+  // past it reads that one again (what comes of it is masked), and a tile past the last loads
+  // nothing (empty descriptors).  Scalars, so that the descriptors made from them stay in SGPRs; the tile
+  // and step offsets ride in the scalar offset.
+  struct Tile {
+    int r0, v0, nt, na, k0;
+    __device__ __forceinline__ __amdgpu_buffer_rsrc_t a(const LmhDev& d) const {
+      return __builtin_amdgcn_make_buffer_rsrc((void*)(d.xq + (int64_t)r0 * kLH), (short)0, (nt + 1) * (16 * kLH), 0x00020000);
+    }
+    __device__ __forceinline__ __amdgpu_buffer_rsrc_t w(const LmhDev& d, int wv) const {
+      return __builtin_amdgcn_make_buffer_rsrc((void*)(d.wq + (int64_t)(v0 + 16 * VT * wv) * kLH), (short)0,
+                                               (na + 1) * (16 * kLH), 0x00020000);
+    }
+  };
+  auto tile = [&](int jj) {
+    const bool in = jj < ntile;
+    const int rt = jj % rpg, r0 = in ? (rbase + rt) * TR : 0, v0 = in ? (jj / rpg * vstep + vres) * kTN : 0;
+    const int nt = in ? min((d.Rs - r0 + 15) / 16, TB) - 1 : -1;
+    const int na = in ? max(min((d.V - v0 - 16 * VT * wv) / 16, VT), 0) - 1 : -1;
+    // the row tiles of a vocab tile run side by side: each starts two steps further into K than the one
+    // before (the sums are exact in any order), so that not all of them wait for the same line
+    return Tile{__builtin_amdgcn_readfirstlane(r0), __builtin_amdgcn_readfirstlane(v0), __builtin_amdgcn_readfirstlane(nt),
+                __builtin_amdgcn_readfirstlane(na), __builtin_amdgcn_readfirstlane(2 * rt)};
+  };
+  v4i w[WD][VT];
+  auto load_w = [&](const Tile& t, auto kc) {  // the wave's weights of step k
+    constexpr int k = decltype(kc)::value;
+#pragma unroll
+    for (int a = 0; a < VT; ++a)
+      w[k % WD][a] = __builtin_amdgcn_raw_buffer_load_b128(t.w(d, wv), 16 * lane,
+                                                          max(min(a, t.na), 0) * (16 * kLH) + ((k + t.k0) & (kNK - 1)) * 1024, 0);
+  };
+  auto dma = [&](const Tile& t, auto sc) {  // the wave's share of stage s: C of its 2 TB pieces of 1 KB
+    constexpr int s = decltype(sc)::value;
+#pragma unroll
+    for (int i = 0; i < C; ++i) {
+      const int c = wv * C + i, u = c >= TB ? 1 : 0, tt = c - TB * u;
+      lds_dma16(t.a(d), stage(ic<s>{}) + c * 1024, 16 * lane, max(min(tt, t.nt), 0) * (16 * kLH) + ((2 * s + u + t.k0) & (kNK - 1)) * 1024);
+    }
+  };
+  v4i f[4];
+  auto read_f = [&](auto nc) {  // fragment n = k TB + t of the tile
+    constexpr int n = decltype(nc)::value, k = n / TB, t = n % TB;
+    f[n & 3] = *reinterpret_cast<const v4i*>(stage(ic<k / 2>{}) + ((k & 1) * TB + t) * 1024 + 16 * lane);
+  };
+  v4i acc[VT][TB];  // [vocab tile][row tile]
+  Tile cur = tile(j), nxt = tile(j + nloc);
+  dma(cur, ic<0>{});
+  dma(cur, ic<1>{});
+  dma(cur, ic<2>{});
+  for_steps([&](auto kc) { load_w(cur, kc); }, std::make_integer_sequence<int, WD>{});
+  wait_vm<2 * C + VT * WD>();  // stage 0
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  for (;;) {
+    read_f(ic<0>{});
+    read_f(ic<1>{});
+    read_f(ic<2>{});
+    for_steps(
+        [&](auto kc) {
+          constexpr int k = decltype(kc)::value;
+          for_steps(
+              [&](auto tc) {
+                constexpr int t = decltype(tc)::value, n = k * TB + t;
+                if constexpr (n + 3 < kNK * TB) read_f(ic<n + 3>{});
+#pragma unroll
+                for (int a = 0; a < VT; ++a)
+                  acc[a][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w[k % WD][a], f[n & 3], k == 0 ? v4i{} : acc[a][t], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+              },
+              std::make_integer_sequence<int, TB>{});
+          if constexpr (k + WD < kNK) load_w(cur, ic<k + WD>{});
+          else if constexpr (lmh_loads(k, WD)) load_w(nxt, ic<k + WD - kNK>{});
+          if constexpr ((k & 1) == 0) {
+            // stage k / 2 + 1 has landed; after the barrier every wave may read it, and stage k / 2 - 1 is free
+            wait_vm<lmh_newer(k, VT, WD, C)>();
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            if constexpr (k / 2 + kNS - 1 < kNK / 2) dma(cur, ic<k / 2 + kNS - 1>{});
+            else dma(nxt, ic<k / 2 + kNS - 1 - kNK / 2>{});
+            if constexpr (k == 2) {
+              // the tile's weight and row scales (every wave is past the previous tile's epilogue)
+              const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
+                  (void*)(d.ws + cur.v0), (short)0, min(d.V - cur.v0, kTN) * 4, 0x00020000);
+              const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+                  (void*)(d.xs + cur.r0), (short)0, min(d.Rs - cur.r0, TR) * 4, 0x00020000);
+              __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, &wsc[64 * wv], 4, 4 * lane + 256 * wv, 0, 0, 0);
+              __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, &xsc[64 * wv], 4, 4 * lane + 256 * wv, 0, 0, 0);
+            }
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        },
+        std::make_integer_sequence<int, kNK>{});
+    // Epilogue: lane l holds tokens 16 t + l % 16 and, per token, vocab columns vb + 16 a + 4 (l / 16) + q,
+    // visited in increasing order.  Each logit (acc * xs) * ws is rounded to bf16 once (hardware
+    // round-to-nearest-even); the lane keeps the first column of its largest value (-0 and +0 compare
+    // equal, as in the bf16 argmax), folds it into a 32-bit key (order-preserving bf16 bits << 16 |
+    // 0xffff - column in the tile), exchanges it with the lanes of the same token and the other waves
+    // through LDS, and the tile's best per row goes out as one 64-bit atomic max.  V % 16 == 0 keeps a
+    // vocab tile all in or all out.
+    const int et = opaque_tid(), el = et & 63, l16 = el & 15, lg = el >> 4;
+    constexpr int NT = X2 ? TB / 2 : TB;  // token tiles (two terms: row tiles 2 b and 2 b + 1 are the terms of tile b)
+    const int vb = 16 * VT * wv, nva = 16 * (cur.na + 1);  // the wave's first column of the tile, its columns in range
+    const int tok0 = X2 ? cur.r0 / 2 : cur.r0, ntok = min(d.R - tok0, 16 * NT);
+    float4 w4[VT];
+#pragma unroll
+    for (int a = 0; a < VT; ++a) w4[a] = *reinterpret_cast<const float4*>(&wsc[vb + 16 * a + 4 * lg]);
+#pragma unroll
+    for (int b = 0; b < NT; ++b) {
+      const int t = X2 ? 2 * b : b;
+      // the logits through a buffer of the token tile's rows in range (a row past it is not written)
+      constexpr int es = STORE == 2 ? 4 : 2;
+      const int64_t lbytes = ((int64_t)min(ntok - 16 * b, 16) * d.V - cur.v0) * es;
+      uint8_t* lbase = STORE == 0 ? nullptr
+                                  : (STORE == 2 ? reinterpret_cast<uint8_t*>(d.logits32) : reinterpret_cast<uint8_t*>(d.logits)) +
+                                        ((size_t)(tok0 + 16 * b) * d.V + cur.v0) * es;
+      const __amdgpu_buffer_rsrc_t lrs =
+          __builtin_amdgcn_make_buffer_rsrc((void*)lbase, (short)0, (int)max(lbytes, (int64_t)0), 0x00020000);
+      const float x1 = xsc[16 * t + l16], x2 = X2 ? xsc[16 * (t + 1) + l16] : 0.f;
+      float bv = -__builtin_inff();
+      int bi = 0;
+      uint32_t pk[VT][2];
+#pragma unroll
+      for (int a = 0; a < VT; ++a) {
+        const bool in = 16 * a < nva;  // uniform
+        const float wq[4] = {w4[a].x, w4[a].y, w4[a].z, w4[a].w};
+        float lg4[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          if constexpr (X2)
+            lg4[q] = rbf_hw(__builtin_fmaf((float)acc[a][t][q], x1, (float)acc[a][t + 1][q] * x2) * wq[q]);
+          else
+            lg4[q] = rbf_hw(((float)acc[a][t][q] * x1) * wq[q]);
+          if (in && lg4[q] > bv) bv = lg4[q], bi = 16 * a + q;
+        }
+        if constexpr (STORE == 1) {
+          pk[a][0] = (__float_as_uint(lg4[0]) >> 16) | (__float_as_uint(lg4[1]) & 0xffff0000u);
+          pk[a][1] = (__float_as_uint(lg4[2]) >> 16) | (__float_as_uint(lg4[3]) & 0xffff0000u);
+        }
+        if constexpr (STORE == 2) {
+          // a token's 16 columns of the tile are 64 contiguous bytes over its four lanes
+          const v4i o = {(int)__float_as_uint(lg4[0]), (int)__float_as_uint(lg4[1]), (int)__float_as_uint(lg4[2]),
+                         (int)__float_as_uint(lg4[3])};
+          const int at = (l16 * d.V + vb + 16 * a + 4 * lg) * 4;
+          __builtin_amdgcn_raw_buffer_store_b128(o, lrs, in ? at : 0x7fffff00, 0, kLogitAux);
+        }
+      }
+      if constexpr (STORE == 1) {
+        // Lanes 16 apart exchange halves of two vocab tiles, so that a lane holds 8 consecutive columns and
+        // the four lanes of a token 32 (64 contiguous bytes): lane group (s1, s0) with tiles (a1, a0) ends
+        // with columns 32 a1 + 16 s0 + 8 s1 .. + 7.
+#pragma unroll
+        for (int a1 = 0; a1 < VT / 2; ++a1) {
+          const auto p0 = __builtin_amdgcn_permlane16_swap(pk[2 * a1][0], pk[2 * a1 + 1][0], false, false);
+          const auto p1 = __builtin_amdgcn_permlane16_swap(pk[2 * a1][1], pk[2 * a1 + 1][1], false, false);
+          const v4i o = {(int)p0[0], (int)p1[0], (int)p0[1], (int)p1[1]};
+          const int cl = 32 * a1 + 16 * (lg & 1) + 8 * (lg >> 1);
+          const int at = (l16 * d.V + vb + cl) * 2;
+          __builtin_amdgcn_raw_buffer_store_b128(o, lrs, cl < nva ? at : 0x7fffff00, 0, kLogitAux);
+        }
+      }
+      uint32_t b16 = __float_as_uint(bv + 0.f) >> 16;
+      b16 = (b16 & 0x8000u) ? (~b16 & 0xffffu) : (b16 | 0x8000u);
+      uint32_t best = (b16 << 16) | (0xffffu - (uint32_t)(vb + 4 * lg + bi));
+      const auto q16 = __builtin_amdgcn_permlane16_swap(best, best, false, false);
+      best = max(q16[0], q16[1]);
+      const auto q32 = __builtin_amdgcn_permlane32_swap(best, best, false, false);
+      best = max(q32[0], q32[1]);
+      if (lg == 0) rkey[wv][16 * b + l16] = nva > 0 ? best : 0u;
+    }
+    // LDS-only barrier for the key exchange: a full __syncthreads also waits for the next tile's
+    // loads in flight
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (et < ntok) {
+      const uint32_t k = max(max(rkey[0][et], rkey[1][et]), max(rkey[2][et], rkey[3][et]));
+      const uint32_t col = (uint32_t)cur.v0 + (0xffffu - (k & 0xffffu));
+      atomicMax(&d.keys[tok0 + et], ((unsigned long long)(k >> 16) << 32) | (unsigned long long)(0xffffffffu - col));
+    }
+    j += nloc;
+    if (j >= ntile) break;
+    cur = nxt;
+    nxt = tile(j + nloc);
+    // the later half of the first weights in flight, only now: kept across the epilogue they would spill
+    for_steps([&](auto kc) { load_w(cur, ic<decltype(kc)::value + WD / 2>{}); }, std::make_integer_sequence<int, WD / 2>{});
+  }
+  wait_vm<0>();  // no load into LDS outlives the workgroup
+}
+
+// ---- Row-major codes (a caller that keeps no tile-order copy): both operands through LDS, so that each weight
+// byte is fetched once a CU.  The kernel above reads row-major codes as 16 rows x 64 bytes an instruction,
+// twice a CU, and took longer there: 2048 rows 695 against 600 us, 256 rows two terms 193 against 163.
+constexpr int kBM = 256, kBN = 256, kBK = 64;
+constexpr int kLmhWaves = 8;  // waves of the workgroup: two a SIMD
+constexpr int kNSA = 3, kNSB = 6;  // LDS ring stages of the activations and of the weights
+
+// LDS position of 16-byte chunk kc (0..3) of tile row c in one K step: rows are 64 bytes, unpadded,
+// with the chunk order xor-swizzled by ((c >> 1) & 3) ^ ((c >> 3) & 1).  A fragment read takes chunk
+// kc of consecutive rows; LDS serves a 16-byte read 16 lanes at a time over 64 banks, and with this
+// swizzle any 16 consecutive rows (and any 8) land in distinct 16-byte bank windows.
+__device__ __forceinline__ int bswz(int c, int kc) { return c * kBK + ((kc ^ ((c >> 1) & 3) ^ ((c >> 3) & 1)) << 4); }
+
 // Persistent GEMM + argmax: one 512-thread workgroup per CU walks its XCD's tiles.  The XCDs form
 // ngrp row groups (2 when the row tiles split evenly, else 1): XCD x serves the rpg = nrt / ngrp
 // row tiles of group x % ngrp and the vocab tiles v = x / ngrp (mod 8 / ngrp).  Its workgroups take
@@ -188,11 +467,11 @@ __device__ __forceinline__ void wait_vm() {
 // stages the loads issued after the barrier overwrite).  The next tile's scales and first steps go
 // out before the epilogue, so it runs while they land.  The LDS reads, 96 KB a step besides the
 // 32 KB the loads write, keep the matrix cores below full rate: the ring depth changes little.
-// row groups of XCDs (see lmh_gemm_body): two when there are at least 4 row tiles, evenly split
-__host__ __device__ __forceinline__ int lmh_groups(int nrt) { return nrt >= 4 && nrt % 2 == 0 ? 2 : 1; }
+// row groups of XCDs: two when there are at least 4 row tiles, evenly split
+__host__ __device__ __forceinline__ int lmr_groups(int nrt) { return nrt >= 4 && nrt % 2 == 0 ? 2 : 1; }
 
 // LDS of the GEMM workgroup, declared once in the kernel and shared by both load roles
-struct LmhLds {
+struct LmrLds {
   int8_t* a[kNSA];  // activation stages
   int8_t* b[kNSB];  // weight stages
   float (*sc)[2][kBN];
@@ -203,8 +482,8 @@ struct LmhLds {
 // loads this wave issues (0: weights, waves 0-3; 1: activations, waves 4-7); everything else is the
 // same in both.  Each role is its own instantiation, so the compiler's wait counting sees only the
 // wave's own operand in flight.
-template <int STORE, bool X2, int NW, int ROLE, bool WT>
-__device__ __forceinline__ void lmh_gemm_body(const LmhDev& d, const LmhLds& L) {
+template <int STORE, bool X2, int NW, int ROLE>
+__device__ __forceinline__ void lmr_gemm_body(const LmhDev& d, const LmrLds& L) {
   // NW waves: two vocab halves (wn) x NW / 2 token groups (wm); a wave owns 128 vocab columns (VB = 4
   // blocks of 32) x TW tokens (TB blocks of 32)
   constexpr int WM = NW / 2, TW = kBM / WM, TB = TW / 32, VB = 4;
@@ -219,7 +498,7 @@ __device__ __forceinline__ void lmh_gemm_body(const LmhDev& d, const LmhLds& L) 
   uint32_t (*rkey)[kBM] = L.rkey;
   const int nvt = (d.V + kBN - 1) / kBN, nrt = (d.Rs + kBM - 1) / kBM;
   const int xcd = blockIdx.x & 7, loc = blockIdx.x >> 3, nloc = gridDim.x >> 3;
-  const int ngrp = lmh_groups(nrt), rpg = nrt / ngrp, vstep = 8 / ngrp;
+  const int ngrp = lmr_groups(nrt), rpg = nrt / ngrp, vstep = 8 / ngrp;
   const int rbase = (xcd % ngrp) * rpg, vres = xcd / ngrp;
   auto vt_of = [&](int jj) { return (jj / rpg) * vstep + vres; };
   int j = loc;
@@ -251,11 +530,10 @@ __device__ __forceinline__ void lmh_gemm_body(const LmhDev& d, const LmhLds& L) 
   int vrow[CPL];
 #pragma unroll
   for (int i = 0; i < CPL; ++i)
-    vrow[i] = ROLE == 0 && WT ? 16 * lane + (CPL * (wv & 3) + i) * 16 * kLH : voff + (CPL * (wv & 3) + i) * 16 * kLH;
+    vrow[i] = voff + (CPL * (wv & 3) + i) * 16 * kLH;
   auto issue_to = [&](const Tile& t, int ks, int8_t* s, int i) {
     const int q = (wv & 3) * CPL + i;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(ROLE == 0 ? t.b : t.a, s + q * 1024, 16, vrow[i],
-                                             ROLE == 0 && WT ? ks * 1024 : ks * kBK, 0, 0);
+    lds_dma16(ROLE == 0 ? t.b : t.a, s + q * 1024, vrow[i], ks * kBK);
   };
   // load i of step KS (its stage KS % NS of the wave's operand)
   auto issue_one = [&](const Tile& t, auto ksc, int i) {
@@ -279,11 +557,7 @@ __device__ __forceinline__ void lmh_gemm_body(const LmhDev& d, const LmhLds& L) 
   // 8 (j / 4) + 4 (l / 32) + j % 4 of register j.
   const int l32 = lane & 31, lh = lane >> 5;
   const int fx0 = bswz(wm * TW + l32, lh), fx1 = bswz(wm * TW + l32, 2 + lh);  // + 32 kBK per t
-  // WT (weights in the tile order, each 16-row x 64-byte piece 1 KB contiguous): the DMA puts lane l's
-  // 16 bytes (row 16 q + l % 16, K chunk l / 16 of the step) at 16 l of chunk q, and a fragment read's
-  // 16 lanes take 256 contiguous bytes
-  const int fw0 = WT ? ((wn * 128 + l32) >> 4) * 1024 + ((l32 & 15) + 16 * lh) * 16 : bswz(wn * 128 + l32, lh);
-  const int fw1 = WT ? fw0 + 512 : bswz(wn * 128 + l32, 2 + lh);
+  const int fw0 = bswz(wn * 128 + l32, lh), fw1 = bswz(wn * 128 + l32, 2 + lh);
   v16i acc[VB][TB];     // [vocab block][token block]
   v4i fx[2][2][TB], fw[2][2][VB];  // [register set][half step][block]
   auto read_one = [&](auto ksc, auto fb, int k) {  // fragment k (0..NRD-1) of step KS
@@ -469,35 +743,20 @@ __device__ __forceinline__ void lmh_gemm_body(const LmhDev& d, const LmhLds& L) 
   }
 }
 
-// The GEMM's LDS: kNSA activation and kNSB weight stages, the scales and the row keys
-#define LMH_GEMM_LDS                                                                                  \
-  __shared__ __align__(1024) int8_t a_s0[kBM * kBK], a_s1[kBM * kBK], a_s2[kBM * kBK];               \
-  __shared__ __align__(1024) int8_t b_s0[kBN * kBK], b_s1[kBN * kBK], b_s2[kBN * kBK], b_s3[kBN * kBK], \
-      b_s4[kBN * kBK], b_s5[kBN * kBK];                                                               \
-  __shared__ __align__(16) float sc_l[2][2][kBN];                                                     \
-  __shared__ uint32_t rkey[2][kBM];                                                                   \
-  static_assert(kNSA == 3 && kNSB == 6, "the stage arrays above");                                   \
-  const LmhLds L{{a_s0, a_s1, a_s2}, {b_s0, b_s1, b_s2, b_s3, b_s4, b_s5}, sc_l, rkey};
-
-// WT: the weights in the tile order (q36_lmhead_args.wq_t) instead of row-major
-template <bool X2, bool WT>
+template <bool X2, int STORE>
 __global__ __launch_bounds__(64 * kLmhWaves) __attribute__((amdgpu_waves_per_eu(kLmhWaves / 4, kLmhWaves / 4))) void
-lmh_gemm_kernel(LmhDev d) {
-  LMH_GEMM_LDS
+lmr_gemm_kernel(LmhDev d) {
+  __shared__ __align__(1024) int8_t a_s0[kBM * kBK], a_s1[kBM * kBK], a_s2[kBM * kBK];
+  __shared__ __align__(1024) int8_t b_s0[kBN * kBK], b_s1[kBN * kBK], b_s2[kBN * kBK], b_s3[kBN * kBK],
+      b_s4[kBN * kBK], b_s5[kBN * kBK];
+  __shared__ __align__(16) float sc_l[2][2][kBN];
+  __shared__ uint32_t rkey[2][kBM];
+  static_assert(kNSA == 3 && kNSB == 6, "the stage arrays above");
+  const LmrLds L{{a_s0, a_s1, a_s2}, {b_s0, b_s1, b_s2, b_s3, b_s4, b_s5}, sc_l, rkey};
   if (__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) < kLmhWaves / 2)
-    lmh_gemm_body<0, X2, kLmhWaves, 0, WT>(d, L);
+    lmr_gemm_body<STORE, X2, kLmhWaves, 0>(d, L);
   else
-    lmh_gemm_body<0, X2, kLmhWaves, 1, WT>(d, L);
-}
-// the same with the logits written out (F32: as fp32)
-template <bool X2, bool F32, bool WT>
-__global__ __launch_bounds__(64 * kLmhWaves) __attribute__((amdgpu_waves_per_eu(kLmhWaves / 4, kLmhWaves / 4))) void
-lmh_gemm_logits_kernel(LmhDev d) {
-  LMH_GEMM_LDS
-  if (__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) < kLmhWaves / 2)
-    lmh_gemm_body<F32 ? 2 : 1, X2, kLmhWaves, 0, WT>(d, L);
-  else
-    lmh_gemm_body<F32 ? 2 : 1, X2, kLmhWaves, 1, WT>(d, L);
+    lmr_gemm_body<STORE, X2, kLmhWaves, 1>(d, L);
 }
 
 __global__ __launch_bounds__(256) void lmh_ids_kernel(LmhDev d) {
@@ -528,7 +787,7 @@ LmhWs lmh_ws(int R) {
     o = align_up(o + b, 256);
     return r;
   };
-  const size_t rows = (size_t)act_rows(R, 1);  // room for two activation terms, whatever the mode
+  const size_t rows = (size_t)act_rows(R, 1, 32);  // room for two activation terms, whatever the mode and the order
   w.xq = take(rows * kLH);
   w.xs = take(sizeof(float) * rows);
   w.keys = take(sizeof(unsigned long long) * (size_t)R);
@@ -547,7 +806,8 @@ extern "C" int q36_lmhead_argmax(const q36_lmhead_args* a, q36_stream_t stream) 
   Q36_REQUIRE(a != nullptr, "q36_lmhead_argmax: null args");
   Q36_REQUIRE(a->H == kLH, "q36_lmhead_argmax: H=%d unsupported (this build is specialised to 2048)", a->H);
   Q36_REQUIRE(a->R >= 1 && a->R <= (1 << 20), "q36_lmhead_argmax: R=%d out of range", a->R);
-  Q36_REQUIRE(a->V >= 16 && a->V % 16 == 0, "q36_lmhead_argmax: V=%d must be a positive multiple of 16", a->V);
+  Q36_REQUIRE(a->V >= 16 && a->V % 16 == 0 && (!a->wq_t || a->V < (1 << 25)),
+              "q36_lmhead_argmax: V=%d must be a positive multiple of 16 (below 2^25 in the tile order)", a->V);
   Q36_REQUIRE(a->mode == Q36_LMH_W8A8 || a->mode == Q36_LMH_W8A8X2 || a->mode == Q36_LMH_W8A16,
               "q36_lmhead_argmax: mode %d unknown", a->mode);
   Q36_REQUIRE(a->mode != Q36_LMH_W8A16 || (a->R <= 64 && a->V % 32 == 0),
@@ -565,7 +825,7 @@ extern "C" int q36_lmhead_argmax(const q36_lmhead_args* a, q36_stream_t stream) 
   Q36_REQUIRE(!a->logits_f32 || a->logits, "q36_lmhead_argmax: logits_f32 set without a logits buffer");
   Q36_REQUIRE(aligned16(a->logits), "q36_lmhead_argmax: logits must be 16-byte aligned");
   const bool f32 = a->logits && a->logits_f32;
-  LmhDev d{a->R, a->V, act_rows(a->R, x2), x2, w16, static_cast<const uint16_t*>(a->h), static_cast<const uint16_t*>(a->norm_w), a->eps,
+  LmhDev d{a->R, a->V, act_rows(a->R, x2, a->wq_t ? 16 : 32), x2, a->wq_t != nullptr, w16, static_cast<const uint16_t*>(a->h), static_cast<const uint16_t*>(a->norm_w), a->eps,
            a->wq_t ? a->wq_t : static_cast<const int8_t*>(a->wq), a->ws, a->ids, f32 ? nullptr : static_cast<uint16_t*>(a->logits),
            f32 ? static_cast<float*>(a->logits) : nullptr, reinterpret_cast<int8_t*>(ws + L.xq), reinterpret_cast<float*>(ws + L.xs),
            reinterpret_cast<unsigned long long*>(ws + L.keys)};
@@ -589,32 +849,55 @@ extern "C" int q36_lmhead_argmax(const q36_lmhead_args* a, q36_stream_t stream) 
     lmh_ids_kernel<<<(a->R + 255) / 256, 256, 0, st>>>(d);
     return check_launch("q36_lmhead_argmax");
   }
-  const int nvt = (a->V + kBN - 1) / kBN, nrt = (d.Rs + kBM - 1) / kBM;
-  // persistent: one workgroup per CU (a multiple of 8, one XCD in eight), never more than the
-  // busiest XCD's tiles
-  const int ngrp = lmh_groups(nrt), vstep = 8 / ngrp;
-  const int blocks = 8 * std::max(1, std::min(lmh_cus() / 8, ((nvt + vstep - 1) / vstep) * (nrt / ngrp)));
-  // the weights' tile order: their DMA reads 1 KB contiguous pieces (2048 rows 697-702 -> 674-683 us,
-  // 256 rows two terms 171-178 -> 164-166 us against the row-major codes)
-  auto go = [&](auto wt) {
-    constexpr bool WT = decltype(wt)::value;
-    if (d.logits32 && x2)
-      lmh_gemm_logits_kernel<true, true, WT><<<blocks, 64 * kLmhWaves, 0, st>>>(d);
-    else if (d.logits32)
-      lmh_gemm_logits_kernel<false, true, WT><<<blocks, 64 * kLmhWaves, 0, st>>>(d);
-    else if (d.logits && x2)
-      lmh_gemm_logits_kernel<true, false, WT><<<blocks, 64 * kLmhWaves, 0, st>>>(d);
+  const int cus = lmh_cus();
+  if (!d.tiled) {
+    const int nvt = (a->V + kBN - 1) / kBN, nrt = (d.Rs + kBM - 1) / kBM, ngrp = lmr_groups(nrt), vstep = 8 / ngrp;
+    // persistent: one workgroup per CU (a multiple of 8, one XCD in eight), never more than the
+    // busiest XCD's tiles
+    const int blocks = 8 * std::max(1, std::min(cus / 8, ((nvt + vstep - 1) / vstep) * (nrt / ngrp)));
+    auto go = [&](auto x2c) {
+      constexpr bool X2 = decltype(x2c)::value;
+      if (d.logits32)
+        lmr_gemm_kernel<X2, 2><<<blocks, 64 * kLmhWaves, 0, st>>>(d);
+      else if (d.logits)
+        lmr_gemm_kernel<X2, 1><<<blocks, 64 * kLmhWaves, 0, st>>>(d);
+      else
+        lmr_gemm_kernel<X2, 0><<<blocks, 64 * kLmhWaves, 0, st>>>(d);
+    };
+    if (x2) go(std::true_type{});
+    else go(std::false_type{});
+    lmh_ids_kernel<<<(a->R + 255) / 256, 256, 0, st>>>(d);
+    return check_launch("q36_lmhead_argmax");
+  }
+  // Tiles of 256 vocab rows x 128 activation rows, two workgroups a CU at a time, 1024 clk of the matrix cores a
+  // K step for both; or of 128 x 128 (about 640 clk: the fragment reads from LDS bound them) where the
+  // last round would otherwise be mostly empty (64 rows two terms: 594 tiles for 512 places, 71.6 -> 69.5
+  // us; 150 rows 127 -> 131 us, 2048 one term 491 -> 551 us, so not there).
+  const int64_t nrt8 = (d.Rs + 127) / 128, nv4 = (a->V + 255) / 256, nv2 = (a->V + 127) / 128, slots = 2 * cus;
+  const bool small = (nv2 * nrt8 + slots - 1) / slots * 640 < (nv4 * nrt8 + slots - 1) / slots * 1024;
+  auto go = [&](auto vtc, auto x2c) {
+    constexpr int VT = decltype(vtc)::value, TB = 8;
+    constexpr bool X2 = decltype(x2c)::value;
+    const int nvt = (a->V + 64 * VT - 1) / (64 * VT), nrt = (d.Rs + 16 * TB - 1) / (16 * TB), ngrp = lmh_groups(nrt),
+              vstep = 8 / ngrp;
+    // persistent: two workgroups per CU (a multiple of 8, one XCD in eight), never more than the
+    // busiest XCD's tiles
+    const int blocks = 8 * (int)std::max<int64_t>(1, std::min<int64_t>(2 * cus / 8, (int64_t)((nvt + vstep - 1) / vstep) * (nrt / ngrp)));
+    if (d.logits32)
+      lmh_gemm_kernel<VT, TB, X2, 2><<<blocks, 256, 0, st>>>(d);
     else if (d.logits)
-      lmh_gemm_logits_kernel<false, false, WT><<<blocks, 64 * kLmhWaves, 0, st>>>(d);
-    else if (x2)
-      lmh_gemm_kernel<true, WT><<<blocks, 64 * kLmhWaves, 0, st>>>(d);
+      lmh_gemm_kernel<VT, TB, X2, 1><<<blocks, 256, 0, st>>>(d);
     else
-      lmh_gemm_kernel<false, WT><<<blocks, 64 * kLmhWaves, 0, st>>>(d);
+      lmh_gemm_kernel<VT, TB, X2, 0><<<blocks, 256, 0, st>>>(d);
   };
-  if (a->wq_t)
-    go(std::true_type{});
+  auto by_tile = [&](auto x2c) {
+    if (small) go(ic<2>{}, x2c);
+    else go(ic<4>{}, x2c);
+  };
+  if (x2)
+    by_tile(std::true_type{});
   else
-    go(std::false_type{});
+    by_tile(std::false_type{});
   lmh_ids_kernel<<<(a->R + 255) / 256, 256, 0, st>>>(d);
   return check_launch("q36_lmhead_argmax");
 }
