@@ -9,12 +9,12 @@
 //     (q36_dense8_linear).
 //
 // Layout of the work: a wave owns 16 RT weight rows (RT 16-row MFMA tiles) over a chunk of K, against
-// every token (up to 64: NTT tiles of 16).  K advances 64 columns a step: lane l loads
+// a group of 16 NTT tokens (the lm_head: every token, up to 64).  K advances 64 columns a step: lane l loads
 // 16 int8 of row l % 16 at column 64 s + 16 (l / 16) (four lanes cover 64 contiguous bytes of a row),
 // and the 16 bf16 of its token at the same columns; the low and high 8 of each feed two
 // v_mfma_f32_16x16x32_bf16 (the same column split on both operands, so every product is formed once).
 // int8 -> bf16 is exact: v_cvt_f32_i32 with a sign-extended byte select, then the high half of the f32.
-// The weights stream from HBM kDepth steps ahead in registers, the activations (a few hundred KB at
+// The weights stream from HBM D steps ahead in registers, the activations (a few hundred KB at
 // most, read from L2) with them.  With the weights as the first operand a lane ends with token l % 16 and four
 // consecutive rows 4 (l / 16) .. + 3 of each tile.
 #include <hip/hip_fp16.h>
@@ -29,8 +29,6 @@ namespace q36 {
 namespace {
 
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-
-constexpr int kDepth = 4;      // weight steps in flight per wave
 
 // 16 int8 (one v4i) -> two fragments of 8 bf16 (low 8 bytes, high 8 bytes)
 __device__ __forceinline__ void widen16(v4i w, v8bf& lo, v8bf& hi) {
@@ -56,12 +54,10 @@ __device__ __forceinline__ v4f mfma_bf16(v8bf a, v8bf b, v4f c) {
 // One workgroup: WAVES waves in RG = WAVES / KS row groups of 16 RT rows; the KS waves of a row group
 // split K into KS contiguous chunks (a multiple of 128 columns each) and their fp32 partial sums meet in
 // LDS, added in chunk order by the first wave of the group, which runs the epilogue.
-template <int NTT, int RT, int KS, int WAVES, int MODE, int K>
+template <int NTT, int RT, int KS, int WAVES, int MODE, int K, int D>
 __global__ __launch_bounds__(64 * WAVES) void w8a16_kernel(W16Dev d) {
   constexpr int RG = WAVES / KS;
   constexpr int RW = 16 * RT;      // rows per wave
-  // steps in flight: weights, activations (and mode 1's group scales); four token tiles hold half as many
-  constexpr int D = NTT >= 4 || RT >= 8 ? kDepth / 2 : kDepth;
   constexpr int NACC = RT * NTT * 4;
   __shared__ float red[KS > 1 ? WAVES - RG : 1][KS > 1 ? NACC : 1][KS > 1 ? 64 : 1];
   __shared__ uint32_t rkey[MODE == 0 ? RG : 1][64];
@@ -70,6 +66,7 @@ __global__ __launch_bounds__(64 * WAVES) void w8a16_kernel(W16Dev d) {
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, lr = lane & 15,
             lg = lane >> 4;
   const int ks = wave % KS, rg = wave / KS;
+  const int t0 = MODE == 1 ? 16 * NTT * blockIdx.y : 0;  // the workgroup's first token (the lm_head takes them all)
   const int r0 = blockIdx.x * (RG * RW) + rg * RW;  // N % RW == 0: a wave's rows are all in or all out
   const bool active = r0 < d.N;
   // K is a template argument so the step loop unrolls completely: with a loop edge the compiler waits for
@@ -93,7 +90,7 @@ __global__ __launch_bounds__(64 * WAVES) void w8a16_kernel(W16Dev d) {
   int xv[NTT];
 #pragma unroll
   for (int tt = 0; tt < NTT; ++tt) {
-    const int t = 16 * tt + lr;
+    const int t = t0 + 16 * tt + lr;
     xv[tt] = t < d.T ? (t * K + k0 + 16 * lg) * 2 : d.T * K * 2;
   }
   v4f acc[RT][NTT], part[RT][NTT];
@@ -256,7 +253,7 @@ __global__ __launch_bounds__(64 * WAVES) void w8a16_kernel(W16Dev d) {
     // column segments (four columns never straddle a boundary: the boundaries are multiples of 4)
 #pragma unroll
     for (int tt = 0; tt < NTT; ++tt) {
-      const int t = 16 * tt + lr;
+      const int t = t0 + 16 * tt + lr;
       if (t >= d.T) continue;
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
@@ -270,70 +267,73 @@ __global__ __launch_bounds__(64 * WAVES) void w8a16_kernel(W16Dev d) {
   }
 }
 
-// The launch shape: token tiles NTT (T <= 16 NTT), row tiles per wave RT, K split KS, waves per
-// workgroup WAVES.  Every shape the policy can pick is instantiated here.
-#define Q36_W16_SHAPES_0(X) X(1, 2, 1, 4) X(1, 4, 1, 2) X(2, 2, 1, 4) X(2, 4, 1, 2) X(2, 8, 1, 2) X(4, 2, 1, 4) X(4, 4, 1, 2)
-#define Q36_W16_SHAPES_1(X) \
-  X(1, 2, 4, 8) X(2, 2, 4, 8) X(4, 2, 4, 8) \
-  X(1, 1, 8, 8) X(2, 1, 8, 8) X(4, 1, 8, 8)
-
-struct W16Shape {
-  int ntt, rt, ks, waves;
-};
-
+// The launch shape: token tiles a workgroup NTT, row tiles per wave RT, K split KS, waves per workgroup
+// WAVES, steps in flight D.
+template <int NTT, int RT, int KS, int WAVES, int MODE, int D>
+void launch_shape(const W16Dev& d, hipStream_t st) {
+  constexpr int rows_wg = (WAVES / KS) * 16 * RT;
+  const dim3 grid((d.N + rows_wg - 1) / rows_wg, MODE == 1 ? (d.T + 16 * NTT - 1) / (16 * NTT) : 1);
+  if constexpr (MODE == 1) {
+    if (d.K == 4096) {
+      w8a16_kernel<NTT, RT, KS, WAVES, MODE, 4096, D><<<grid, 64 * WAVES, 0, st>>>(d);
+      return;
+    }
+  }
+  w8a16_kernel<NTT, RT, KS, WAVES, MODE, 2048, D><<<grid, 64 * WAVES, 0, st>>>(d);
+}
 // Measured on MI355X (the lm_head, N = 151936, codes in the tile order, graph-timed): the lm_head
 // streams whole rows, 32 a wave in four-wave workgroups up to 8 tokens (61 us; 64-row waves 63 us,
 // too few loads in flight); from 9 tokens on the activation fragments each wave reads from L2 weigh
 // more, so wider waves serve more weight rows with each: 64 rows a wave in two-wave workgroups up to
 // 24 tokens (16: 62.7 against 66.1 us), 128 rows from 25 to 32 tokens (32: 73.6 against 78.0 us), and
 // 64 rows with four token tiles (48: 99 against 138 us for 32-row waves, 63: 112 against 160 us).
-// The projections split K so that every CU has waves: in quarters for the 9216- and 12352-row
-// in_proj / qkv, in eighths for the 2048-row o_proj / out_proj.
-W16Shape w16_shape(const W16Dev& d, int mode) {
+// (A wave's rows are all in or all out: 64-row waves need N % 64 == 0, 128-row waves N % 128 == 0.)
+void launch_lmhead(const W16Dev& d, hipStream_t st) {
   const int ntt = d.T <= 16 ? 1 : d.T <= 32 ? 2 : 4;
-  // (a wave's rows are all in or all out: 64-row waves need N % 64 == 0, 128-row waves N % 128 == 0)
-  if (mode == 0) {
-    if (d.T <= 8 || d.N % 64 != 0) return W16Shape{ntt, 2, 1, 4};
-    if (ntt == 2 && d.T > 24 && d.N % 128 == 0) return W16Shape{ntt, 8, 1, 2};
-    return W16Shape{ntt, 4, 1, 2};
-  }
-  return d.N >= 8192 ? W16Shape{ntt, 2, 4, 8} : W16Shape{ntt, 1, 8, 8};
-}
-
-template <int NTT, int RT, int KS, int WAVES, int MODE>
-void launch_shape(const W16Dev& d, hipStream_t st) {
-  constexpr int rows_wg = (WAVES / KS) * 16 * RT;
-  const int grid = (d.N + rows_wg - 1) / rows_wg;
-  if constexpr (MODE == 1) {
-    if (d.K == 4096) {
-      w8a16_kernel<NTT, RT, KS, WAVES, MODE, 4096><<<grid, 64 * WAVES, 0, st>>>(d);
-      return;
-    }
-  }
-  w8a16_kernel<NTT, RT, KS, WAVES, MODE, 2048><<<grid, 64 * WAVES, 0, st>>>(d);
-}
-
-template <int MODE>
-int launch_mode(const W16Dev& d, hipStream_t st) {
-  const W16Shape s = w16_shape(d, MODE);
-#define Q36_W16_CASE(NTT, RT, KS, W)                                              \
-  if (s.ntt == NTT && s.rt == RT && s.ks == KS && s.waves == W) {                 \
-    launch_shape<NTT, RT, KS, W, MODE>(d, st);                                    \
-    return Q36_OK;                                                                \
-  }
-  if constexpr (MODE == 0) {
-    Q36_W16_SHAPES_0(Q36_W16_CASE)
+  if (d.T <= 8 || d.N % 64 != 0) {
+    if (ntt == 1) launch_shape<1, 2, 1, 4, 0, 4>(d, st);
+    else if (ntt == 2) launch_shape<2, 2, 1, 4, 0, 4>(d, st);
+    else launch_shape<4, 2, 1, 4, 0, 2>(d, st);
+  } else if (ntt == 1) {
+    launch_shape<1, 4, 1, 2, 0, 4>(d, st);
+  } else if (ntt == 2 && d.T > 24 && d.N % 128 == 0) {
+    launch_shape<2, 8, 1, 2, 0, 2>(d, st);
+  } else if (ntt == 2) {
+    launch_shape<2, 4, 1, 2, 0, 4>(d, st);
   } else {
-    Q36_W16_SHAPES_1(Q36_W16_CASE)
+    launch_shape<4, 4, 1, 2, 0, 2>(d, st);
   }
-#undef Q36_W16_CASE
-  return Q36_EINVAL;
+}
+// The projections split K so that every CU has waves, in quarters for the 9216- and 12352-row in_proj / qkv and
+// in eighths for the 2048-row o_proj / out_proj (the split sets the order of a sum; the rest does not).
+// Latency-bound, and past 16 tokens bound by the activation rows, which every wave reads from L2: 64 rows a
+// wave halve them for the wide projections, and the narrow ones, whose row groups alone leave CUs
+// idle, give each 16-token group its own workgroups (the second reading of the weights hits L2).
+// Cold weights, graph-timed, us a call before -> now at 16 / 32 / 64 tokens: 12352 x 2048 9.0 -> 8.4 / 13.0 ->
+// 10.7 / 21.6 -> 16.1, 9216 x 2048 8.6 -> 7.9 / 12.6 -> 10.4 / 17.0 -> 15.6, 2048 x 4096 7.1 / 10.7 -> 7.1 / 18.4
+// -> 8.0.  (Eight waves of 64 rows a workgroup, two tokens groups a narrow workgroup or all steps in
+// flight at once: slower.)
+void launch_linear(const W16Dev& d, hipStream_t st) {
+  const int ntt = d.T <= 16 ? 1 : d.T <= 32 ? 2 : 4;
+  if (d.N >= 8192) {
+    if (ntt == 1 && (d.T <= 8 || d.N % 64 != 0)) launch_shape<1, 2, 4, 8, 1, 4>(d, st);
+    else if (ntt == 1) launch_shape<1, 4, 4, 4, 1, 4>(d, st);
+    else if (d.N % 64 != 0) launch_shape<2, 2, 4, 4, 1, 4>(d, st);
+    else if (ntt == 2) launch_shape<2, 4, 4, 4, 1, 4>(d, st);
+    else launch_shape<4, 4, 4, 4, 1, 2>(d, st);
+  } else if (d.N / 16 * ((d.T + 15) / 16) <= 256) {  // a workgroup a CU at most
+    launch_shape<1, 1, 8, 8, 1, 4>(d, st);
+  } else {
+    launch_shape<1, 2, 8, 8, 1, 4>(d, st);
+  }
 }
 
 }  // namespace
 
 int launch_w8a16(const W16Dev& d, int mode, hipStream_t st) {
-  return mode == 0 ? launch_mode<0>(d, st) : launch_mode<1>(d, st);
+  if (mode == 0) launch_lmhead(d, st);
+  else launch_linear(d, st);
+  return Q36_OK;
 }
 
 }  // namespace q36

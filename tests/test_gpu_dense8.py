@@ -187,3 +187,18 @@ def test_dense8_tiled_copy_same_bits(dev, T, N, K):
     torch.cuda.synchronize()
     assert torch.equal(qt, want)
     assert torch.equal(y0.view(torch.int16), y1.view(torch.int16))
+
+
+@pytest.mark.parametrize("N,K", [(12352, 2048), (9216, 2048), (8224, 2048), (2048, 4096), (2048, 2048), (4096, 2048), (32, 4096)])
+def test_dense8_rows_do_not_depend_on_the_batch(dev, N, K):
+    """Every launch shape (wide and narrow N, whole and odd 64-row groups, one to four token groups) adds a
+    row's products in the same order: a batch of T rows is its rows run 8 at a time, bit for bit."""
+    from bundles_amd.qwen36_layer import formats, glue
+    g = torch.Generator(device=dev).manual_seed(N + K)
+    q, s = formats.quant_dense8((torch.randn((N, K), generator=g, device=dev) * 0.02).to(torch.bfloat16))
+    qt = formats.tile_w16(q)
+    x = torch.randn((64, K), generator=g, device=dev).to(torch.bfloat16)
+    want = torch.cat([glue.dense8_linear(x[i:i + 8].contiguous(), q, s) for i in range(0, 64, 8)])
+    for T in (1, 9, 16, 17, 31, 32, 33, 48, 49, 64):
+        print(f"dense8 N={N} K={K} T={T}", flush=True)
+        assert torch.equal(glue.dense8_linear(x[:T].contiguous(), qt, s, tiled=True), want[:T])
