@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import struct
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libq36.so")
@@ -100,37 +101,59 @@ class DecodeArgs(C.Structure):
                 ("workspace", P), ("workspace_bytes", SZ), ("gate", P), ("oq", P), ("oqs", P)]
 
 
+def _packer(st):
+    """struct.pack of a structure's fields in order (nested arrays flattened): the bytes of the filled structure, which a
+    void pointer argument takes as they are.  Filling the ctypes structure itself took longer than the launch it describes
+    (45 fields: 5 us against 1)."""
+    code = {P: "P", I32: "i", SZ: "N", I64: "q", C.c_float: "f"}
+    fmt = "@"
+    for _, t in st._fields_:
+        if t in code:
+            fmt += code[t]
+        else:  # an array of structures of 8-byte alignment
+            fmt += "0q" + "".join(code[f] for _, f in t._type_._fields_) * t._length_
+    s = struct.Struct(fmt + "0q")
+    assert s.size == C.sizeof(st), st
+    return s.pack
+
+
+pack_moe, pack_gdn, pack_ring, pack_attn = map(_packer, (MoeArgs, GdnArgs, GdnRingArgs, AttnArgs))
+pack_oproj, pack_lmhead, pack_fp8, pack_dense8 = map(_packer, (OprojArgs, LmheadArgs, Fp8LinearArgs, Dense8LinearArgs))
+pack_addnorm, pack_decode = map(_packer, (AddNormArgs, DecodeArgs))
+
+
 _lib = None
 
-# (name, restype, argtypes) of every exported symbol; tests check that each one resolves.
+# (name, restype, argtypes) of every exported symbol; tests check that each one resolves.  The argument structures
+# go as void pointers, to a structure (byref) or to the bytes a pack_* function makes.
 SYMBOLS = [
     ("q36_abi_version", I32, []),
     ("q36_last_error", C.c_char_p, []),
     ("q36_moe_workspace_bytes", SZ, [I32, I32, I32, I32, I32, I32]),
     ("q36_moe_workspace_layout", I32, [I32, I32, I32, I32, I32, I32, C.POINTER(MoeWsLayout)]),
-    ("q36_moe_route", I32, [C.POINTER(MoeArgs), P]),
-    ("q36_moe_up", I32, [C.POINTER(MoeArgs), P]),
-    ("q36_moe_down", I32, [C.POINTER(MoeArgs), P]),
-    ("q36_moe_combine", I32, [C.POINTER(MoeArgs), P]),
-    ("q36_moe_forward", I32, [C.POINTER(MoeArgs), P]),
-    ("q36_moe_forward_static", I32, [C.POINTER(MoeArgs), P]),
-    ("q36_gdn_verify", I32, [C.POINTER(GdnArgs), P]),
-    ("q36_gdn_verify_ring", I32, [C.POINTER(GdnRingArgs), P]),
+    ("q36_moe_route", I32, [P, P]),
+    ("q36_moe_up", I32, [P, P]),
+    ("q36_moe_down", I32, [P, P]),
+    ("q36_moe_combine", I32, [P, P]),
+    ("q36_moe_forward", I32, [P, P]),
+    ("q36_moe_forward_static", I32, [P, P]),
+    ("q36_gdn_verify", I32, [P, P]),
+    ("q36_gdn_verify_ring", I32, [P, P]),
     ("q36_attn_act_frag", I32, [I32]),
     ("q36_attn_workspace_bytes", SZ, [I32]),
     ("q36_oproj_workspace_bytes", SZ, [I32]),
-    ("q36_attn_proj", I32, [C.POINTER(AttnArgs), P]),
-    ("q36_attn_oproj", I32, [C.POINTER(OprojArgs), P]),
+    ("q36_attn_proj", I32, [P, P]),
+    ("q36_attn_oproj", I32, [P, P]),
     ("q36_fp8_linear_act_frag", I32, [I32, I32]),
     ("q36_fp8_linear_workspace_bytes", SZ, [I32, I32]),
-    ("q36_fp8_linear", I32, [C.POINTER(Fp8LinearArgs), P]),
-    ("q36_add_rmsnorm", I32, [C.POINTER(AddNormArgs), P]),
-    ("q36_dense8_linear", I32, [C.POINTER(Dense8LinearArgs), P]),
+    ("q36_fp8_linear", I32, [P, P]),
+    ("q36_add_rmsnorm", I32, [P, P]),
+    ("q36_dense8_linear", I32, [P, P]),
     ("q36_tile_w16", I32, [P, C.c_int64, I32, P, P]),
     ("q36_attn_decode_workspace_bytes", SZ, [I32, I32]),
-    ("q36_attn_decode", I32, [C.POINTER(DecodeArgs), P]),
+    ("q36_attn_decode", I32, [P, P]),
     ("q36_lmhead_workspace_bytes", SZ, [I32]),
-    ("q36_lmhead_argmax", I32, [C.POINTER(LmheadArgs), P]),
+    ("q36_lmhead_argmax", I32, [P, P]),
     ("q36_quant_rows_i8", I32, [P, C.c_int64, I32, P, P, P]),
     ("q36_q8_block_v1_bytes", SZ, [I32, I32]),
     ("q36_quant_q8_block_v1", I32, [P, P, I32, I32, I32, I32, P, P]),
@@ -164,12 +187,17 @@ def check(rc: int, what: str) -> None:
         raise RuntimeError(f"{what}: {kind}: {msg}")
 
 
-def ptr(t) -> int | None:
-    """Device (or host) address of a torch tensor, None for None."""
-    return None if t is None else t.data_ptr()
+def ptr(t) -> int:
+    """Device (or host) address of a torch tensor, 0 for None."""
+    return 0 if t is None else t.data_ptr()
 
 
-def stream_handle(stream=None) -> int | None:
+def stream_handle(stream=None) -> int:
+    """The given stream's handle, or the current device's current stream's."""
+    if stream is not None:
+        return stream.cuda_stream
     import torch
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return s.cuda_stream
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # the handle without a Stream object around it
+    if raw is None or not torch.cuda.is_initialized():
+        return torch.cuda.current_stream().cuda_stream
+    return raw(torch._C._cuda_getDevice())

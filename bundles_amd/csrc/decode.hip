@@ -29,6 +29,7 @@
 //                   workgroup holds whole is written by the split kernel itself).
 #include <math.h>
 
+#include <atomic>
 #include <type_traits>
 
 #include "q36_device.h"
@@ -677,8 +678,13 @@ __global__ __launch_bounds__(WPR == 4 ? 256 : 1024) void decode_combine_kernel(D
 }
 
 int decode_cus() {
+  static std::atomic<int> known[64];  // per device, 0: not asked yet
   int cus = 256, dev = 0;
-  if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  if (hipGetDevice(&dev) != hipSuccess) return cus;
+  const bool slot = dev >= 0 && dev < 64;
+  if (slot && known[dev].load(std::memory_order_relaxed)) return known[dev].load(std::memory_order_relaxed);
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && slot)
+    known[dev].store(cus, std::memory_order_relaxed);
   return cus;
 }
 // Equal splits per request: as asked for, or (a workspace too small for the balanced form) enough to

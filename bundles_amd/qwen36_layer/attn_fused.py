@@ -9,13 +9,12 @@ scales (prepare_weights).
 """
 from __future__ import annotations
 
-import ctypes as C
 from dataclasses import dataclass
 
 import torch
 
 from .. import _lib
-from .._lib import AttnArgs, DecodeArgs, OprojArgs, check, ptr
+from .._lib import check, pack_attn, pack_decode, pack_oproj, ptr
 from .moe import quantize_blocks_e4m3
 
 N_Q_HEADS, N_KV_HEADS, HEAD_DIM, HIDDEN = 16, 2, 256, 2048
@@ -103,30 +102,28 @@ def attn_proj(x, w: AttnWeights, q_norm_w, k_norm_w, eps, cos_sin, positions, ws
     if T > ws.T_max:
         raise ValueError(f"attn_proj: {T} tokens exceed the workspace's {ws.T_max}")
     dev = x.device if x is not None else xq.codes.device
-    o = out or dict(q=torch.empty((T, N_Q_HEADS, HEAD_DIM), dtype=torch.bfloat16, device=dev),
-                    gate=torch.empty((T, N_Q_HEADS, HEAD_DIM), dtype=torch.bfloat16, device=dev),
-                    k=torch.empty((T, N_KV_HEADS, HEAD_DIM), dtype=torch.bfloat16, device=dev),
-                    v=torch.empty((T, N_KV_HEADS, HEAD_DIM), dtype=torch.bfloat16, device=dev),
-                    k8=torch.empty((T, N_KV_HEADS, HEAD_DIM), dtype=torch.uint8, device=dev),
-                    v8=torch.empty((T, N_KV_HEADS, HEAD_DIM), dtype=torch.uint8, device=dev))
+    bf = dict(dtype=torch.bfloat16, device=dev)
+    u8 = dict(dtype=torch.uint8, device=dev)
+    o = out or dict(q=torch.empty((T, N_Q_HEADS, HEAD_DIM), **bf), gate=torch.empty((T, N_Q_HEADS, HEAD_DIM), **bf),
+                    k=torch.empty((T, N_KV_HEADS, HEAD_DIM), **bf), v=torch.empty((T, N_KV_HEADS, HEAD_DIM), **bf),
+                    k8=torch.empty((T, N_KV_HEADS, HEAD_DIM), **u8), v8=torch.empty((T, N_KV_HEADS, HEAD_DIM), **u8))
     kc = vc = loc = None
     slots = 0
     if cache is not None:
         kc, vc, loc = cache
         for name, t in (("k_cache", kc), ("v_cache", vc)):
-            if t.dtype != torch.uint8 or not t.is_contiguous() or t.dim() != 3 or tuple(t.shape[1:]) != (N_KV_HEADS,
-                                                                                                      HEAD_DIM):
+            if t.dtype != torch.uint8 or not t.is_contiguous() or t.shape[1:] != (N_KV_HEADS, HEAD_DIM):
                 raise ValueError(f"attn_proj: {name} must be contiguous uint8 [slots, {N_KV_HEADS}, {HEAD_DIM}]")
         if kc.shape != vc.shape:
             raise ValueError("attn_proj: k_cache and v_cache differ in shape")
         if loc.dtype != torch.int64 or not loc.is_contiguous() or loc.numel() < T:
             raise ValueError(f"attn_proj: out_loc must be contiguous int64 with at least {T} entries")
         slots = kc.shape[0]
-    a = AttnArgs(T, cos_sin.shape[0], ptr(x), ptr(w.wqkv_p), ptr(w.sqkv), ptr(q_norm_w), ptr(k_norm_w), eps,
+    a = pack_attn(T, cos_sin.shape[0], ptr(x), ptr(w.wqkv_p), ptr(w.sqkv), ptr(q_norm_w), ptr(k_norm_w), eps,
                  ptr(cos_sin), ptr(positions), ptr(o["q"]), ptr(o["gate"]), ptr(o["k"]), ptr(o["v"]), ptr(o["k8"]),
                  ptr(o["v8"]), ptr(ws.proj), ws.proj.numel(), ptr(None if xq is None else xq.codes),
                  ptr(None if xq is None else xq.scales), ptr(loc), ptr(kc), ptr(vc), slots)
-    check(_lib.lib().q36_attn_proj(C.byref(a), _lib.stream_handle(stream)), "q36_attn_proj")
+    check(_lib.lib().q36_attn_proj(a, _lib.stream_handle(stream)), "q36_attn_proj")
     return o
 
 
@@ -139,9 +136,9 @@ def attn_oproj(attn, gate, w: AttnWeights, ws: Workspace, out=None, stream=None,
         raise ValueError("attn_oproj: aq must be row-major rows of this token count (oproj_rows)")
     dev = attn.device if attn is not None else aq.codes.device
     out = torch.empty((T, HIDDEN), dtype=torch.bfloat16, device=dev) if out is None else out
-    a = OprojArgs(T, ptr(attn), ptr(gate), ptr(w.wo_p), ptr(w.so), ptr(out), ptr(ws.oproj), ws.oproj.numel(),
+    a = pack_oproj(T, ptr(attn), ptr(gate), ptr(w.wo_p), ptr(w.so), ptr(out), ptr(ws.oproj), ws.oproj.numel(),
                   ptr(None if aq is None else aq.codes), ptr(None if aq is None else aq.scales))
-    check(_lib.lib().q36_attn_oproj(C.byref(a), _lib.stream_handle(stream)), "q36_attn_oproj")
+    check(_lib.lib().q36_attn_oproj(a, _lib.stream_handle(stream)), "q36_attn_oproj")
     return out
 
 
@@ -186,9 +183,9 @@ def attn_decode(q, k_cache, v_cache, page_table, seqlens, NT: int, scale: float,
                            or gate.numel() != T * N_Q_HEADS * HEAD_DIM):
         raise ValueError("attn_decode: gate must be contiguous bf16 [T, 4096] and oq row-major rows (oproj_rows)")
     out = torch.empty_like(q) if out is None else out
-    a = DecodeArgs(B, NT, q.shape[1], k_cache.shape[1], q.shape[2], ws.splits, ptr(q), ptr(k_cache), ptr(v_cache),
+    a = pack_decode(B, NT, q.shape[1], k_cache.shape[1], q.shape[2], ws.splits, ptr(q), ptr(k_cache), ptr(v_cache),
                    k_cache.shape[0], ptr(page_table), page_table.shape[1], ptr(seqlens), ptr(out_loc), ptr(k_new),
                    ptr(v_new), scale, ptr(out), ptr(ws.buf), ws.buf.numel(), ptr(gate),
                    ptr(None if oq is None else oq.codes), ptr(None if oq is None else oq.scales))
-    check(_lib.lib().q36_attn_decode(C.byref(a), _lib.stream_handle(stream)), "q36_attn_decode")
+    check(_lib.lib().q36_attn_decode(a, _lib.stream_handle(stream)), "q36_attn_decode")
     return out

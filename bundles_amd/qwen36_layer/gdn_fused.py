@@ -10,19 +10,17 @@ Mirrors the reference's glue (R = qwen36_nodes_kb34, L = R/qwen36_layer): gdn_ve
 """
 from __future__ import annotations
 
-import ctypes as C
-
 import torch
 
 from .. import _lib
-from .._lib import GdnArgs, GdnRingArgs, check, ptr
+from .._lib import check, pack_gdn, pack_ring, ptr
 
 HEAD_K, HEAD_V, N_K_HEADS, N_V_HEADS = 128, 128, 16, 32
 QKV_DIM = 2 * N_K_HEADS * HEAD_K + N_V_HEADS * HEAD_V  # 8192
 
 
 def _req(t, name, dtype, shape):
-    if t.dtype != dtype or not t.is_contiguous() or tuple(t.shape) != tuple(shape):
+    if t.dtype != dtype or t.shape != shape or not t.is_contiguous():
         raise ValueError(f"gdn_verify_fused: {name} must be contiguous {dtype} {tuple(shape)}, got "
                          f"{t.dtype} {tuple(t.shape)}")
 
@@ -50,9 +48,9 @@ def gdn_verify_fused(mixed, z, a, b, conv_state, conv_w, A_log, dt_bias, S0, nor
     snaps = torch.empty((B, T, N_V_HEADS, HEAD_V, HEAD_K), dtype=torch.float32, device=dev) if snaps is None \
         else snaps
     conv_state_out = torch.empty_like(conv_state) if conv_state_out is None else conv_state_out
-    args = GdnArgs(B, T, ptr(mixed), ptr(z), ptr(a), ptr(b), ptr(conv_state), ptr(conv_state_out), ptr(conv_w),
+    args = pack_gdn(B, T, ptr(mixed), ptr(z), ptr(a), ptr(b), ptr(conv_state), ptr(conv_state_out), ptr(conv_w),
                    ptr(A_log), ptr(dt_bias), ptr(S0), ptr(norm_w), eps, ptr(out), ptr(snaps))
-    check(_lib.lib().q36_gdn_verify(C.byref(args), _lib.stream_handle(stream)), "q36_gdn_verify")
+    check(_lib.lib().q36_gdn_verify(args, _lib.stream_handle(stream)), "q36_gdn_verify")
     return out, snaps, conv_state_out
 
 
@@ -62,8 +60,8 @@ RING = 16
 def _pool(t, name, dtype, tail, inner_strides):
     """A slot pool [slots, *tail] with the given innermost strides (the slot stride is free but a
     multiple of 8 elements), as the reference's host checks require (L/qk_gdn_verify.cu:872-904)."""
-    if t.dtype != dtype or t.dim() != 1 + len(tail) or tuple(t.shape[1:]) != tuple(tail) or \
-            tuple(t.stride()[1:]) != tuple(inner_strides) or t.stride(0) % 8 != 0:
+    st = t.stride()
+    if t.dtype != dtype or t.shape[1:] != tail or st[1:] != inner_strides or st[0] % 8 != 0:
         raise ValueError(f"gdn_verify_ring: {name} must be a {dtype} [slots, {', '.join(map(str, tail))}] pool with "
                          f"contiguous heads, got {t.dtype} {tuple(t.shape)} strides {t.stride()}")
 
@@ -100,7 +98,7 @@ def gdn_verify_ring(mixed, z, a, b, conv_state, conv_w, window, A_log, dt_bias, 
     _pool(conv_state, "conv_state", torch.bfloat16, (QKV_DIM, 3), (3, 1))
     _req(conv_w, "conv_weights", torch.bfloat16, (QKV_DIM, 4))
     if window.dim() == 4:  # the deduplicated [wslots, T, 8192, 3] view of [wslots, 8192, T + 2]
-        if tuple(window.shape[1:]) != (T, QKV_DIM, 3) or tuple(window.stride()[1:]) != (1, T + 2, 1):
+        if window.shape[1:] != (T, QKV_DIM, 3) or window.stride()[1:] != (1, T + 2, 1):
             raise ValueError("gdn_verify_ring: conv windows must be the deduplicated [slots, T, 8192, 3] view of "
                              "[slots, 8192, T + 2]")
         if window.stride(0) % 8:
@@ -111,15 +109,15 @@ def gdn_verify_ring(mixed, z, a, b, conv_state, conv_w, window, A_log, dt_bias, 
     if dt_bias.dtype not in (torch.float32, torch.bfloat16) or dt_bias.numel() != N_V_HEADS or \
             not dt_bias.is_contiguous():
         raise ValueError("gdn_verify_ring: dt_bias must hold 32 fp32 or bf16 values")
-    if h0.dtype != torch.float32 or h0.dim() != 4 or tuple(h0.shape[1:]) != (N_V_HEADS, HEAD_V, HEAD_K) or \
+    if h0.dtype != torch.float32 or h0.shape[1:] != (N_V_HEADS, HEAD_V, HEAD_K) or \
             not h0.is_contiguous():
         raise ValueError("gdn_verify_ring: the checkpoint must be a contiguous fp32 [slots, 32, 128, 128] pool")
     for t, n in ((d_ring, "d ring"), (dlo_ring, "d ring (low parts)")):
         _pool(t, n, torch.bfloat16, (N_V_HEADS, RING, HEAD_V), (RING * HEAD_V, HEAD_V, 1))
     for t, n in ((k_ring, "k ring"), (klo_ring, "k ring (low parts)")):
         _pool(t, n, torch.bfloat16, (N_K_HEADS, RING, HEAD_K), (RING * HEAD_K, HEAD_K, 1))
-    if g_ring.dtype != torch.float32 or tuple(g_ring.shape[1:]) != (N_V_HEADS, RING) or \
-            tuple(g_ring.stride()[1:]) != (RING, 1) or g_ring.stride(0) % 4:
+    if g_ring.dtype != torch.float32 or g_ring.shape[1:] != (N_V_HEADS, RING) or \
+            g_ring.stride()[1:] != (RING, 1) or g_ring.stride(0) % 4:
         raise ValueError("gdn_verify_ring: g ring must be an fp32 [slots, 32, 16] pool")
     if qsl.dtype != torch.int32 or qsl.numel() < B + 1 or not qsl.is_contiguous():
         raise ValueError("gdn_verify_ring: query_start_loc must hold B + 1 int32 offsets")
@@ -134,7 +132,7 @@ def gdn_verify_ring(mixed, z, a, b, conv_state, conv_w, window, A_log, dt_bias, 
     _req(out, "out", torch.bfloat16, (rows, N_V_HEADS * HEAD_V))
     if oq is not None and (oq.T != rows or oq.frag or oq.codes.shape[1] != N_V_HEADS * HEAD_V):
         raise ValueError("gdn_verify_ring: oq must be row-major rows of the verify batch (glue.linear_rows)")
-    args = GdnRingArgs(
+    args = pack_ring(
         B, T, rows, min(conv_state.shape[0], h0.shape[0]), rslots, window.shape[0],
         ptr(mixed), ptr(z), ptr(a), ptr(b), ptr(conv_state), conv_state.stride(0), ptr(conv_w), ptr(window),
         window.stride(0), ptr(A_log), ptr(dt_bias), int(dt_bias.dtype == torch.float32), ptr(h0),
@@ -142,5 +140,5 @@ def gdn_verify_ring(mixed, z, a, b, conv_state, conv_w, window, A_log, dt_bias, 
         k_ring.stride(0), klo_ring.stride(0), ptr(g_ring), g_ring.stride(0), ptr(qsl), ptr(state_idx),
         ptr(replay_idx), ptr(win_idx), flags, ptr(write_pos), ptr(cache_base), ptr(norm_w), eps, scale, ptr(out),
         ptr(None if oq is None else oq.codes), ptr(None if oq is None else oq.scales))
-    check(_lib.lib().q36_gdn_verify_ring(C.byref(args), _lib.stream_handle(stream)), "q36_gdn_verify_ring")
+    check(_lib.lib().q36_gdn_verify_ring(args, _lib.stream_handle(stream)), "q36_gdn_verify_ring")
     return out

@@ -10,13 +10,12 @@ add-norm and the add-norm itself (L/proj.py:60-112 project_add_norm).  The weigh
 """
 from __future__ import annotations
 
-import ctypes as C
 from dataclasses import dataclass
 
 import torch
 
 from .. import _lib
-from .._lib import AddNormArgs, Dense8LinearArgs, Fp8LinearArgs, check, ptr
+from .._lib import check, pack_addnorm, pack_dense8, pack_fp8, ptr
 from .moe import pack_frag8, quantize_blocks_e4m3
 
 
@@ -92,26 +91,28 @@ def fp8_linear(x: torch.Tensor, w: Fp8Weight, ws: LinearWorkspace, segments=None
     else:
         ret = None
     segs = _segments("fp8_linear", T, w.n, segments)
-    a = Fp8LinearArgs(T, w.qp.shape[0], K, w.n, ptr(x), ptr(w.qp), ptr(w.s), len(segments), segs,
-                      ptr(ws.buf), ws.buf.numel(), ptr(None if xq is None else xq.codes),
-                      ptr(None if xq is None else xq.scales))
-    check(_lib.lib().q36_fp8_linear(C.byref(a), _lib.stream_handle(stream)), "q36_fp8_linear")
+    a = pack_fp8(T, w.qp.shape[0], K, w.n, ptr(x), ptr(w.qp), ptr(w.s), len(segments), *segs,
+                 ptr(ws.buf), ws.buf.numel(), ptr(None if xq is None else xq.codes),
+                 ptr(None if xq is None else xq.scales))
+    check(_lib.lib().q36_fp8_linear(a, _lib.stream_handle(stream)), "q36_fp8_linear")
     return ret
 
 
 def _segments(fn: str, T: int, n: int, segments):
+    """The checked segments as the structure's 4 x (col0, ld, out), unused ones zero."""
     if not 1 <= len(segments) <= 4:
         raise ValueError(f"{fn}: 1 to 4 segments")
     end = 0
-    segs = (_lib.LinearSeg * 4)()
+    segs = []
     for i, (c0, o) in enumerate(segments):
-        if c0 != end or o.dtype != torch.bfloat16 or o.shape[0] != T or o.stride(1) != 1:
+        shape, st = o.shape, o.stride()
+        if c0 != end or o.dtype != torch.bfloat16 or shape[0] != T or st[1] != 1:
             raise ValueError(f"{fn}: segment {i} (col0 {c0}) must continue at column {end} as bf16 [T, w]")
-        segs[i] = _lib.LinearSeg(c0, o.stride(0), o.data_ptr())
-        end = c0 + o.shape[1]
+        segs += (c0, st[0], o.data_ptr())
+        end = c0 + shape[1]
     if end != n:
         raise ValueError(f"{fn}: segments cover {end} of {n} columns")
-    return segs
+    return segs + [0] * (12 - len(segs))
 
 
 def dense8_linear(x: torch.Tensor, q: torch.Tensor, s: torch.Tensor, segments=None, stream=None, tiled=False):
@@ -132,8 +133,8 @@ def dense8_linear(x: torch.Tensor, q: torch.Tensor, s: torch.Tensor, segments=No
     else:
         ret = None
     segs = _segments("dense8_linear", T, N, segments)
-    a = Dense8LinearArgs(T, N, K, N, ptr(x), ptr(q), ptr(s), s.stride(0), len(segments), segs, int(bool(tiled)))
-    check(_lib.lib().q36_dense8_linear(C.byref(a), _lib.stream_handle(stream)), "q36_dense8_linear")
+    a = pack_dense8(T, N, K, N, ptr(x), ptr(q), ptr(s), s.stride(0), len(segments), *segs, int(bool(tiled)))
+    check(_lib.lib().q36_dense8_linear(a, _lib.stream_handle(stream)), "q36_dense8_linear")
     return ret
 
 
@@ -145,8 +146,8 @@ def add_rmsnorm(delta, residual: torch.Tensor, norm_w: torch.Tensor, eps: float,
     out = torch.empty_like(residual) if out is None else out
     if q8 is not None and (q8.T != T or q8.codes.shape[1] != H):
         raise ValueError("add_rmsnorm: q8 rows do not match the residual")
-    a = AddNormArgs(T, H, ptr(delta), ptr(residual), ptr(norm_w), eps, ptr(out),
-                    ptr(None if q8 is None else q8.codes), ptr(None if q8 is None else q8.scales),
-                    int(q8 is not None and q8.frag))
-    check(_lib.lib().q36_add_rmsnorm(C.byref(a), _lib.stream_handle(stream)), "q36_add_rmsnorm")
+    a = pack_addnorm(T, H, ptr(delta), ptr(residual), ptr(norm_w), eps, ptr(out),
+                     ptr(None if q8 is None else q8.codes), ptr(None if q8 is None else q8.scales),
+                     int(q8 is not None and q8.frag))
+    check(_lib.lib().q36_add_rmsnorm(a, _lib.stream_handle(stream)), "q36_add_rmsnorm")
     return out

@@ -18,7 +18,7 @@ from dataclasses import dataclass
 import torch
 
 from .. import _lib
-from .._lib import MoeArgs, MoeWsLayout, Q36_MOE_FP8, Q36_MOE_INT8, check, ptr
+from .._lib import MoeArgs, MoeWsLayout, Q36_MOE_FP8, Q36_MOE_INT8, check, pack_moe, ptr
 
 MAX_TOKENS = 256  # the reference's row-batch limit (L/layer.py:50)
 
@@ -179,8 +179,13 @@ class Workspace:
             y=v(L.y, (S + M) * self.H, torch.bfloat16).view(S + M, self.H))
 
 
-def _args(x, positions, router_w, gate_w, ew, topk, ws: Workspace, out, router_bias, debug, norm=None, norm_q8=None,
-          pre_norm=None):
+def _args(*args, **kwargs) -> MoeArgs:
+    return MoeArgs.from_buffer_copy(_packed(*args, **kwargs))
+
+
+def _packed(x, positions, router_w, gate_w, ew, topk, ws: Workspace, out, router_bias, debug, norm=None, norm_q8=None,
+            pre_norm=None) -> bytes:
+    """The checked arguments as the bytes of q36_moe_args."""
     M, H = (x if x is not None else pre_norm[0]).shape
     if M > ws.max_tokens:
         raise ValueError(f"moe_row_batch: {M} rows exceed the workspace's {ws.max_tokens}")
@@ -198,7 +203,7 @@ def _args(x, positions, router_w, gate_w, ew, topk, ws: Workspace, out, router_b
     if norm is not None:
         resid, norm_w, eps, norm_out = norm
         for name, t in (("resid", resid), ("norm_out", norm_out)):
-            if t.dtype != torch.bfloat16 or not t.is_contiguous() or tuple(t.shape) != (M, H):
+            if t.dtype != torch.bfloat16 or not t.is_contiguous() or t.shape != (M, H):
                 raise ValueError(f"moe_row_batch: {name} must be contiguous bfloat16 {(M, H)}")
         if norm_w.dtype != torch.bfloat16 or not norm_w.is_contiguous() or norm_w.numel() != H:
             raise ValueError(f"moe_row_batch: norm_w must be contiguous bfloat16 [{H}]")
@@ -207,11 +212,11 @@ def _args(x, positions, router_w, gate_w, ew, topk, ws: Workspace, out, router_b
     if pre_norm is not None:
         delta, r_in, r_out, in_w, in_eps = pre_norm
         for name, t in (("delta", delta), ("resid_in", r_in), ("resid_out", r_out)):
-            if t.dtype != torch.bfloat16 or not t.is_contiguous() or tuple(t.shape) != (M, H):
+            if t.dtype != torch.bfloat16 or not t.is_contiguous() or t.shape != (M, H):
                 raise ValueError(f"moe_row_batch: pre_norm {name} must be contiguous bfloat16 {(M, H)}")
         if in_w.dtype != torch.bfloat16 or not in_w.is_contiguous() or in_w.numel() != H:
             raise ValueError(f"moe_row_batch: pre_norm norm_w must be contiguous bfloat16 [{H}]")
-    return MoeArgs(M, router_w.shape[0], H, ws.I, topk, ws.dtype, ptr(x), ptr(router_w), ptr(router_bias),
+    return pack_moe(M, router_w.shape[0], H, ws.I, topk, ws.dtype, ptr(x), ptr(router_w), ptr(router_bias),
                    ptr(positions), *(ptr(t) for t in w), ptr(gate_w), ptr(out), ptr(ws.buf), ws.buf.numel(),
                    ptr(dbg.get("acc13")), ptr(dbg.get("acc2")), ptr(dbg.get("h")), ptr(resid), ptr(norm_w),
                    float(eps), ptr(norm_out), ptr(None if norm_q8 is None else norm_q8.codes),
@@ -221,8 +226,8 @@ def _args(x, positions, router_w, gate_w, ew, topk, ws: Workspace, out, router_b
 
 def route(x, positions, router_w, topk: int, ws: Workspace, router_bias=None, stream=None):
     """Routing only (ids, weights, expert lists and quantized x in the workspace); returns ws.views(M)."""
-    a = _args(x, positions, router_w, None, None, topk, ws, None, router_bias, None)
-    check(_lib.lib().q36_moe_route(C.byref(a), _lib.stream_handle(stream)), "q36_moe_route")
+    a = _packed(x, positions, router_w, None, None, topk, ws, None, router_bias, None)
+    check(_lib.lib().q36_moe_route(a, _lib.stream_handle(stream)), "q36_moe_route")
     return ws.views(x.shape[0])
 
 
@@ -248,8 +253,8 @@ def moe_row_batch(x, positions, router_w, gate_w, ew: ExpertWeights, topk: int, 
         out = torch.empty_like(shape_src)
     if norm_q8 is not None and (norm is None or norm_q8.T != shape_src.shape[0]):
         raise ValueError("moe_row_batch: norm_q8 needs the fused add-norm and one row per token")
-    a = _args(x, positions, router_w, gate_w, ew, topk, ws, out, router_bias, debug, norm, norm_q8, pre_norm)
-    check(_lib.lib().q36_moe_forward(C.byref(a), _lib.stream_handle(stream)), "q36_moe_forward")
+    a = _packed(x, positions, router_w, gate_w, ew, topk, ws, out, router_bias, debug, norm, norm_q8, pre_norm)
+    check(_lib.lib().q36_moe_forward(a, _lib.stream_handle(stream)), "q36_moe_forward")
     return out
 
 
@@ -257,7 +262,7 @@ def moe_phases(x, positions, router_w, gate_w, ew: ExpertWeights, topk: int, ws:
                stream=None):
     """The same block as moe_row_batch as four separately launched phases (route, up, down, combine);
     returns the list of (name, callable) so a caller can schedule or time each one."""
-    a = _args(x, positions, router_w, gate_w, ew, topk, ws, out, router_bias, None)
+    a = _packed(x, positions, router_w, gate_w, ew, topk, ws, out, router_bias, None)
     L = _lib.lib()
     # the argument struct holds raw device addresses: the callables keep the tensors they point into
     # alive, so a caller that drops its own references does not leave them pointing at freed memory
@@ -265,7 +270,7 @@ def moe_phases(x, positions, router_w, gate_w, ew: ExpertWeights, topk: int, ws:
 
     def call(fn, name):
         def run(_keep=keep):
-            check(fn(C.byref(a), _lib.stream_handle(stream)), name)
+            check(fn(a, _lib.stream_handle(stream)), name)
         return run
     return [("route", call(L.q36_moe_route, "q36_moe_route")), ("up", call(L.q36_moe_up, "q36_moe_up")),
             ("down", call(L.q36_moe_down, "q36_moe_down")), ("combine", call(L.q36_moe_combine, "q36_moe_combine"))]

@@ -8,12 +8,10 @@ Mirrors the reference's lm_head glue (R = qwen36_nodes_kb34, H = R/qwen36_lmhead
 """
 from __future__ import annotations
 
-import ctypes as C
-
 import torch
 
 from .. import _lib
-from .._lib import LmheadArgs, check, ptr
+from .._lib import check, pack_lmhead, ptr
 
 
 def quantize_rows(w: torch.Tensor, stream=None):
@@ -68,14 +66,14 @@ def w8a8_lmhead_argmax(h, q, scale, ws: Workspace, norm_w=None, eps: float = 1e-
     ids = torch.empty(R, dtype=torch.int32, device=h.device) if ids is None else ids
     if want_logits and logits is None:
         logits = torch.empty((R, V), dtype=torch.bfloat16, device=h.device)
-    if logits is not None and (logits.dtype not in (torch.bfloat16, torch.float32) or tuple(logits.shape) != (R, V)
+    if logits is not None and (logits.dtype not in (torch.bfloat16, torch.float32) or logits.shape != (R, V)
                                or not logits.is_contiguous()):
         raise ValueError(f"w8a8_lmhead_argmax: logits must be contiguous bf16 or fp32 [{R}, {V}]")
-    if q_t is not None and (tuple(q_t.shape) != (V, H) or (q is not None and tuple(q.shape) != (V, H))):
+    if q_t is not None and (q_t.shape != (V, H) or (q is not None and q.shape != (V, H))):
         raise ValueError(f"w8a8_lmhead_argmax: q_t is tile_rows_w16(q), int8 [{V}, {H}]")
-    a = LmheadArgs(R, H, V, ptr(h), ptr(norm_w), eps, ptr(q), ptr(scale), ptr(ids), ptr(logits), ptr(ws.buf),
-                   ws.buf.numel(),
-                   _lib.Q36_LMH_W8A16 if w8a16 else _lib.Q36_LMH_W8A8X2 if two_term else _lib.Q36_LMH_W8A8,
-                   int(logits is not None and logits.dtype == torch.float32), ptr(q_t))
-    check(_lib.lib().q36_lmhead_argmax(C.byref(a), _lib.stream_handle(stream)), "q36_lmhead_argmax")
+    a = pack_lmhead(R, H, V, ptr(h), ptr(norm_w), eps, ptr(q), ptr(scale), ptr(ids), ptr(logits), ptr(ws.buf),
+                    ws.buf.numel(),
+                    _lib.Q36_LMH_W8A16 if w8a16 else _lib.Q36_LMH_W8A8X2 if two_term else _lib.Q36_LMH_W8A8,
+                    int(logits is not None and logits.dtype == torch.float32), ptr(q_t))
+    check(_lib.lib().q36_lmhead_argmax(a, _lib.stream_handle(stream)), "q36_lmhead_argmax")
     return (ids, logits) if (want_logits or logits is not None) else ids
