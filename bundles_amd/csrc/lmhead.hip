@@ -764,6 +764,25 @@ __global__ __launch_bounds__(256) void lmh_ids_kernel(LmhDev d) {
   if (r < d.R) d.ids[r] = (int32_t)(0xffffffffu - (uint32_t)(d.keys[r] & 0xffffffffull));
 }
 
+// The ids from the workgroups' keys (W8A16 without a norm): one workgroup a token, the largest value's
+// first row.  Bound by latency (4 bytes a workgroup of the GEMM, read once).
+__global__ __launch_bounds__(256) void lmh_ids_wg_kernel(const uint32_t* keys, int nwg, int rows, int T, int32_t* ids) {
+  __shared__ unsigned long long best[4];
+  const int t = blockIdx.x, tid = threadIdx.x;
+  unsigned long long m = 0ull;
+#pragma unroll 4
+  for (int g = tid; g < nwg; g += 256) {
+    const uint32_t k = keys[(size_t)g * T + t];
+    const uint32_t row = (uint32_t)(g * rows) + (0xffffu - (k & 0xffffu));
+    m = max(m, k ? ((unsigned long long)(k >> 16) << 32) | (0xffffffffu - row) : 0ull);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o));
+  if ((tid & 63) == 0) best[tid >> 6] = m;
+  __syncthreads();
+  if (tid == 0) ids[t] = (int32_t)(0xffffffffu - (uint32_t)(max(max(best[0], best[1]), max(best[2], best[3])) & 0xffffffffull));
+}
+
 int lmh_cus() {
   static int cached[64] = {0};
   int dev = 0;
@@ -830,13 +849,22 @@ extern "C" int q36_lmhead_argmax(const q36_lmhead_args* a, q36_stream_t stream) 
            f32 ? static_cast<float*>(a->logits) : nullptr, reinterpret_cast<int8_t*>(ws + L.xq), reinterpret_cast<float*>(ws + L.xs),
            reinterpret_cast<unsigned long long*>(ws + L.keys)};
   hipStream_t st = static_cast<hipStream_t>(stream);
-  lmh_prep_kernel<<<a->R, 64, 0, st>>>(d);
+  // W8A16 without a norm needs no prep: the GEMM reads h itself, and each workgroup leaves its best key in a
+  // place of its own, for the ids kernel, instead of meeting the others in keys that a launch has to
+  // clear first (V = 151936, us before -> now: 1 row 58.5 -> 57.6, 7 rows 60.6 -> 59.7, 16 rows 62.2 -> 60.6,
+  // 30 rows 75.6 -> 74.3).  The places lie where the prep's rows would; where they do not fit (this
+  // vocabulary at 56 rows or more, a wider one sooner), the prep stays.
+  const int wrows = w16 ? w8a16_lmhead_rows(a->R, a->V) : 0, nwg = w16 ? (a->V + wrows - 1) / wrows : 0;
+  const bool direct = w16 && !a->norm_w && (size_t)nwg * a->R * sizeof(uint32_t) <= L.xs - L.xq;
+  if (!direct) lmh_prep_kernel<<<a->R, 64, 0, st>>>(d);
   if (w16) {
     W16Dev g{};
     g.T = a->R;
     g.N = a->V;
     g.K = kLH;
-    g.x = reinterpret_cast<const uint16_t*>(d.xq);  // the prep's bf16 rows (2 R * H bytes fit in xq)
+    // the prep's bf16 rows (2 R * H bytes fit in xq), or h as it is
+    g.x = direct ? d.h : reinterpret_cast<const uint16_t*>(d.xq);
+    g.wgkeys = direct ? reinterpret_cast<uint32_t*>(d.xq) : nullptr;
     // the codes in the tile order when the caller keeps that copy: each piece the kernel loads at once
     // is then 1 KB contiguous (1 row 77 -> 61 us, 32 rows 115 -> 79 us at V = 151936)
     g.q = d.wq;
@@ -846,7 +874,10 @@ extern "C" int q36_lmhead_argmax(const q36_lmhead_args* a, q36_stream_t stream) 
     g.logits32 = d.logits32;
     g.keys = d.keys;
     launch_w8a16(g, 0, st);
-    lmh_ids_kernel<<<(a->R + 255) / 256, 256, 0, st>>>(d);
+    if (direct)
+      lmh_ids_wg_kernel<<<a->R, 256, 0, st>>>(g.wgkeys, nwg, wrows, a->R, d.ids);
+    else
+      lmh_ids_kernel<<<(a->R + 255) / 256, 256, 0, st>>>(d);
     return check_launch("q36_lmhead_argmax");
   }
   const int cus = lmh_cus();

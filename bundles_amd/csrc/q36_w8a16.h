@@ -16,6 +16,7 @@ struct W16Dev {
   uint16_t* logits;       // bf16 [T, N] or null
   float* logits32;        // fp32 [T, N] (the bf16-rounded values) or null
   unsigned long long* keys;  // [T] argmax keys (zero on entry)
+  uint32_t* wgkeys;       // or, when set, [workgroups][T]: each workgroup's best, bf16 key << 16 | 0xffff - row in it
   // mode 1
   const uint16_t* s16;    // fp16 [K / 128][s_ld]
   int64_t s_ld;
@@ -26,5 +27,7 @@ struct W16Dev {
 
 // T <= 64, N % 32 == 0, K 2048 (mode 0) or 2048 / 4096 (mode 1), checked by the callers
 int launch_w8a16(const W16Dev& d, int mode, hipStream_t st);
+// Vocab rows a workgroup of the lm_head (mode 0) takes
+int w8a16_lmhead_rows(int T, int N);
 
 }  // namespace q36

@@ -243,7 +243,9 @@ __global__ __launch_bounds__(64 * WAVES) void w8a16_kernel(W16Dev d) {
       uint32_t k = rkey[0][tid];
 #pragma unroll
       for (int j = 1; j < RG; ++j) k = max(k, rkey[j][tid]);
-      if (k != 0u) {
+      if (d.wgkeys) {
+        d.wgkeys[(size_t)blockIdx.x * d.T + tid] = k;
+      } else if (k != 0u) {
         const uint32_t row = (uint32_t)(blockIdx.x * (RG * RW)) + (0xffffu - (k & 0xffffu));
         atomicMax(&d.keys[tid], ((unsigned long long)(k >> 16) << 32) | (unsigned long long)(0xffffffffu - row));
       }
@@ -288,6 +290,7 @@ void launch_shape(const W16Dev& d, hipStream_t st) {
 // 24 tokens (16: 62.7 against 66.1 us), 128 rows from 25 to 32 tokens (32: 73.6 against 78.0 us), and
 // 64 rows with four token tiles (48: 99 against 138 us for 32-row waves, 63: 112 against 160 us).
 // (A wave's rows are all in or all out: 64-row waves need N % 64 == 0, 128-row waves N % 128 == 0.)
+// (w8a16_lmhead_rows: the rows of a workgroup, 16 RT WAVES / KS.)
 void launch_lmhead(const W16Dev& d, hipStream_t st) {
   const int ntt = d.T <= 16 ? 1 : d.T <= 32 ? 2 : 4;
   if (d.T <= 8 || d.N % 64 != 0) {
@@ -329,6 +332,8 @@ void launch_linear(const W16Dev& d, hipStream_t st) {
 }
 
 }  // namespace
+
+int w8a16_lmhead_rows(int T, int N) { return T > 24 && T <= 32 && N % 128 == 0 ? 256 : 128; }
 
 int launch_w8a16(const W16Dev& d, int mode, hipStream_t st) {
   if (mode == 0) launch_lmhead(d, st);

@@ -131,6 +131,29 @@ def test_lmhead_w8a16_tiled_copy_same_bits(mods, dev, R, V, norm):
     assert torch.equal(logits.view(torch.int16), logits2.view(torch.int16))
 
 
+# without a norm the workgroups' keys meet in the ids kernel (their places fit the workspace: all but the
+# last two); rows copied over the vocabulary make the maximum tie across workgroups and within one
+@pytest.mark.parametrize("R,V", [(1, 32), (1, 151936), (7, 4128), (8, 33024), (16, 151936), (24, 8192), (29, 4160),
+                                 (32, 4224), (64, 4096), (64, 160), (16, 1 << 19), (63, 151936)])
+def test_lmhead_w8a16_ids_of_ties(mods, dev, R, V):
+    """The ids without a norm are the first of each row's largest logits, whichever workgroups hold them."""
+    from bundles_amd import synth
+    _, _, lmh = mods
+    print(f"lmhead W8A16 ties R={R} V={V}", flush=True)
+    d = synth.lmhead_inputs(R, 4096, dev, seed=7 * R + V)
+    q, s = lmh.quantize_rows(d["w"])
+    idx = torch.arange(V, device=dev) * 37 % min(V // 2, 4096)  # every row at least twice
+    q, s = q[idx].contiguous(), s[idx].contiguous()
+    ws = lmh.Workspace(R, dev)
+    ids, logits = lmh.w8a8_lmhead_argmax(d["h"], q, s, ws, want_logits=True, w8a16=True)
+    only = lmh.w8a8_lmhead_argmax(d["h"], None, s, ws, w8a16=True, q_t=lmh.tile_rows_w16(q))
+    torch.cuda.synchronize()
+    lg = bf16_f32(bits16(logits))
+    assert np.array_equal(np_(ids), np.argmax(lg, axis=1))
+    assert np.array_equal(np_(only), np_(ids))
+    assert np.all((lg == lg.max(axis=1, keepdims=True)).sum(axis=1) > 1), "no ties"
+
+
 # the W8A8 GEMM forms on the tile-order copy: one term (ids only, bf16 and f32 logits) and two terms
 @pytest.mark.parametrize("R,V,two_term,logits", [(256, 151936, False, None), (64, 4096, False, "bf16"),
                                                  (300, 8192, True, None), (128, 4160, False, "f32"),
