@@ -68,8 +68,16 @@ struct GdnRingDev {
 };
 
 // Four waves per SIMD (two workgroups per CU): at most 128 VGPRs, of which the 16 x 4 h0 values are 64.
-// TM bounds T (4, 5 or 8): the conv's input registers are sized by it.
-template <int TM>
+// TM bounds T (4, 5 or 8): the conv's input registers are sized by it.  EXACT: T is TM, the window
+// lengths served most, with no branch around a position, so one's work fills another's latency.
+//
+// Bound by latency and, two workgroups a CU, by the vector and matrix units: a workgroup's phases take 11 us,
+// of which the checkpoint's transfer needs 4 at the CU's share of HBM.  So the matrix cores work
+// through two phases (half of the dots beside the other waves' small tiles, half beside the history), the
+// gates lie in a wave that is idle then, and bf16 rounding is one instruction.  Kernel alone, graph-timed,
+// us before -> now at B x T: 8x4 13.2 -> 11.6, 16x4 15.5 -> 13.5, 32x4 23.6 -> 22.6, 48x4 35.0 -> 34.3,
+// 64x4 43.8 -> 40.1, 64x5 46.7 -> 42.6, 64x8 54.0 -> 47.2.
+template <int TM, bool EXACT>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void gdn_ring_kernel(GdnRingDev d) {
   __shared__ __attribute__((aligned(16))) float xf[8][64][4];      // MFMA B fragments of X (step, lane)
   __shared__ __attribute__((aligned(16))) float kw[32][KW_STRIDE];  // rows 0-15 ring keys, 16-23 window keys
@@ -80,11 +88,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void g
   __shared__ __attribute__((aligned(16))) uint16_t dh[2][RL][RV];     // committed d entries, logical order
   __shared__ __attribute__((aligned(16))) uint16_t zs[RTMAX][2 * RV];  // the output gate's z
   __shared__ float nws[RV], rg[2][RL];
-  __shared__ float gg[2][RTMAX], gbeta[2][RTMAX], geg[2][RTMAX];
+  __shared__ float gbeta[2][RTMAX], geg[2][RTMAX];
   __shared__ float dec[2][RL], tdec[2];
 
   const int r = blockIdx.x >> 4, hk = blockIdx.x & 15;
-  const int T = d.T, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int T = EXACT ? TM : d.T, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // The request's row offset and its three indices (int32, or int64 as two 32-bit words), all
   // requested before any is used: one scalar round trip.
   const int f = d.idx_i64;
@@ -151,8 +159,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void g
 #pragma unroll
   for (int t = 0; t < TM; ++t) w[3 + t] = bf2f(d.mixed[(bos + min(t, T - 1)) * RQKV + ch]);
   const v2i cwr = *reinterpret_cast<const v2i*>(d.conv_w + (int64_t)ch * 4);
-  // gate inputs: thread tid < 2 T serves head tid & 1, position tid >> 1
-  const int gt = min(tid, 2 * T - 1), ghv = 2 * hk + (gt & 1);
+  // gate inputs: lane l < 2 T of wave 2 serves head l & 1, position l >> 1
+  const int gt = min(lane, 2 * T - 1), ghv = 2 * hk + (gt & 1);
   const int64_t grow = bos + (gt >> 1);
   const float av = bf2f(d.a[grow * RHV + ghv]), bv = bf2f(d.b[grow * RHV + ghv]);
   const uint32_t dtw = reinterpret_cast<const uint32_t*>(d.dt_bias)[d.dt_f32 ? ghv : ghv >> 1];
@@ -171,7 +179,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void g
   // reads row l & 15 of a tile, columns 16 s + 4 (l >> 4) .. + 3 at step s.  Its 8 steps are
   // requested two at a time through the phases below (about 64 KB in flight a CU: enough to keep
   // HBM busy, little enough that a phase's own stores, issued before its next request, do not queue
-  // behind a deep stream in the CU's in-order memory pipe)
+  // behind a deep stream in the CU's in-order memory pipe; the third and fourth pair together: 64x4
+  // 44.2 against 40.1 us, the workgroup waiting to issue them)
   const int hh = wave >> 2, rb = (wave & 3) * 32;
   const float* hp = d.h0 + ((slot * RHV + 2 * hk + hh) * RV + rb + (lane & 15)) * RK + 4 * (lane >> 4);
   v4f hr[2][8];
@@ -212,11 +221,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void g
 #pragma unroll
     for (int t = 0; t < TM; ++t) {
       if (t < T) {
-        float acc = rbf(w[t] * cw0);
-        acc = acc + rbf(w[t + 1] * cw1);
-        acc = acc + rbf(w[t + 2] * cw2);
-        acc = acc + rbf(w[t + 3] * cw3);
-        const float o = rbf(acc / (1.f + expf_q(-acc)));
+        float acc = rbf_hw(w[t] * cw0);
+        acc = acc + rbf_hw(w[t + 1] * cw1);
+        acc = acc + rbf_hw(w[t + 2] * cw2);
+        acc = acc + rbf_hw(w[t + 3] * cw3);
+        const float o = rbf_hw(acc / (1.f + expf_q(-acc)));
         if (wave < 4) qko[tid >> 7][t][tid & 127] = o;  // wave-uniform: one object per store
         else vs[(tid - 256) >> 7][t][(tid - 256) & 127] = o;
       }
@@ -226,28 +235,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void g
     uint16_t* const rec = stage + 1536 + tid * (T + 2);
 #pragma unroll
     for (int i = 0; i < TM + 2; ++i)
-      if (i < T + 2) rec[i] = (uint16_t)f2bf(w[1 + i]);
+      if (i < T + 2) rec[i] = (uint16_t)(__float_as_uint(w[1 + i]) >> 16);  // a bf16 value
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
       float v = 0.f;
 #pragma unroll
       for (int t = 0; t < TM + 3; ++t) v = t == T + i ? w[t] : v;
-      stage[3 * tid + i] = (uint16_t)f2bf(v);
+      stage[3 * tid + i] = (uint16_t)(__float_as_uint(v) >> 16);
     }
-  }
-  if (tid < 2 * T) {
-    const int h = tid & 1, t = tid >> 1;
-    // dt_bias: the fp32 word, or the bf16 half of the word that holds element ghv (shift and mask, no
-    // branch on the loaded value)
-    const uint32_t dsh = d.dt_f32 ? 0u : ((ghv & 1) ? 0u : 16u);
-    const uint32_t dmask = d.dt_f32 ? 0xffffffffu : 0xffff0000u;
-    const float dtb = __uint_as_float((dtw << dsh) & dmask);
-    const float xg = av + dtb;
-    const float sp = xg <= 20.f ? logf(1.f + expf_q(xg)) : xg;
-    const float g = -expf_q(alog) * sp;
-    gg[h][t] = g;
-    gbeta[h][t] = sigmoid_q(bv);
-    geg[h][t] = expf_q(g);
   }
   request(2);
   __syncthreads();
@@ -290,20 +285,21 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void g
       if (nv + t < RL) {
         const int ph = (cb + nv + t) & 15;
         const int64_t off = ((int64_t)hk * RL + ph) * RK + lane;
-        const uint32_t h0b = f2bf(y0), h1b = f2bf(y1);
-        d.k_ring[rp * d.k_slot + off] = (uint16_t)h0b;
-        d.k_ring[rp * d.k_slot + off + 64] = (uint16_t)h1b;
-        d.klo_ring[rp * d.klo_slot + off] = (uint16_t)f2bf(y0 - bf2f(h0b));
-        d.klo_ring[rp * d.klo_slot + off + 64] = (uint16_t)f2bf(y1 - bf2f(h1b));
-        if (lane < 2) d.g_ring[rp * d.g_slot + (2 * hk + lane) * RL + ph] = gg[lane][t];
+        const uint32_t hb = pack_bf2_hw(y0, y1);
+        const uint32_t lb = pack_bf2_hw(y0 - bf_lo(hb), y1 - bf_hi(hb));
+        d.k_ring[rp * d.k_slot + off] = (uint16_t)hb;
+        d.k_ring[rp * d.k_slot + off + 64] = (uint16_t)(hb >> 16);
+        d.klo_ring[rp * d.klo_slot + off] = (uint16_t)lb;
+        d.klo_ring[rp * d.klo_slot + off + 64] = (uint16_t)(lb >> 16);
       }
     }
   }
   request(4);
   __syncthreads();
 
-  // ---- dots that need no checkpoint row, while the early rows stream: ring keys (wave 0) and window
-  // keys (wave 1) against X, and the history's decays (32 lanes of wave 7).
+  // ---- dots that need no checkpoint row: ring keys (wave 0) and window keys (wave 1) against X; the
+  // window's gates (wave 2) and the history's decays (32 lanes of wave 7).  Then every wave its
+  // first half of the checkpoint's.
   // key rows r0 .. r0 + 15 of kw against X -> xr rows r0 .. r0 + 15 (two accumulation chains)
   auto xr_tile = [&](int r0) {
     v4f a2[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
@@ -319,6 +315,22 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void g
   };
   if (wave == 0) xr_tile(0);
   else if (wave == 1) xr_tile(16);
+  else if (wave == 2) {
+    if (lane < 2 * T) {
+      const int h = lane & 1, t = lane >> 1;
+      // dt_bias: the fp32 word, or the bf16 half of the word that holds element ghv (shift and mask, no
+      // branch on the loaded value)
+      const uint32_t dsh = d.dt_f32 ? 0u : ((ghv & 1) ? 0u : 16u);
+      const uint32_t dmask = d.dt_f32 ? 0xffffffffu : 0xffff0000u;
+      const float dtb = __uint_as_float((dtw << dsh) & dmask);
+      const float xg = av + dtb;
+      const float sp = xg <= 20.f ? logf(1.f + expf_q(xg)) : xg;
+      const float g = -expf_q(alog) * sp;
+      gbeta[h][t] = sigmoid_q(bv);
+      geg[h][t] = expf_q(g);
+      if (nv + t < RL) d.g_ring[rp * d.g_slot + ghv * RL + ((cb + nv + t) & 15)] = g;
+    }
+  }
   else if (tid >= 448 && tid < 480) {  // decay of entry c: exp(total - prefix_c), sums in logical order
     const int h = (tid - 448) >> 4, c = tid & 15;
     float tot = 0.f, pre = 0.f;
@@ -330,6 +342,19 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void g
     dec[h][c] = c < nv ? expf_q(tot - pre) : 0.f;
     if (c == 0) tdec[h] = expf_q(tot);
   }
+  v4f acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  auto dots = [&](int s0) {  // steps s0 .. s0 + 3 as they arrive
+#pragma unroll
+    for (int s = s0; s < s0 + 4; ++s) {
+      const v4f xb = *reinterpret_cast<const v4f*>(&xf[s][lane][0]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(hr[0][s][j], xb[j], acc[0], 0, 0, 0);
+        acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(hr[1][s][j], xb[j], acc[1], 0, 0, 0);
+      }
+    }
+  };
+  dots(0);
   request(6);
   __syncthreads();
   // The history's part of each row's dots: R_x = sum_c decay_c dhat_c (khat_c . x).  Lanes 2j and
@@ -348,24 +373,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void g
     }
   }
 
-  // ---- the checkpoint rows' dots, step by step as they arrive
-  {
-    v4f acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  // ---- the rest of the checkpoint rows' dots.  D: lane l, register q = row 4 (l >> 4) + q of the tile,
+  // vector l & 15
+  dots(4);
 #pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      const v4f xb = *reinterpret_cast<const v4f*>(&xf[s][lane][0]);
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(hr[0][s][j], xb[j], acc[0], 0, 0, 0);
-        acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(hr[1][s][j], xb[j], acc[1], 0, 0, 0);
-      }
-    }
-    // D: lane l, register q = row 4 (l >> 4) + q of the tile, vector l & 15
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) hx[hh][rb + 16 * i + 4 * (lane >> 4) + q][lane & 15] = acc[i][q];
-  }
+    for (int q = 0; q < 4; ++q) hx[hh][rb + 16 * i + 4 * (lane >> 4) + q][lane & 15] = acc[i][q];
   __syncthreads();
 
   // ---- per value row: P_x = td (h0 . x) + R_x = S x for the window's vectors, then the delta rule
@@ -395,12 +409,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void g
           for (int i = 0; i < 4; ++i) P[4 * x4 + i] = __builtin_fmaf(eg, P[4 * x4 + i], u * xv[i]);
         }
         if (part == 0) {
-          qko[rh][t][rv] = rbf(P[t]);  // the core output is bf16
+          qko[rh][t][rv] = rbf_hw(P[t]);  // the core output is bf16
         } else if (nv + t < RL) {
           const int ph = (cb + nv + t) & 15;
-          const uint32_t hi = f2bf(u);
-          d.d_ring[dro + ph * RV] = (uint16_t)hi;
-          d.dlo_ring[dlo + ph * RV] = (uint16_t)f2bf(u - bf2f(hi));
+          const float hi = rbf_hw(u);
+          d.d_ring[dro + ph * RV] = (uint16_t)(__float_as_uint(hi) >> 16);
+          d.dlo_ring[dlo + ph * RV] = (uint16_t)(__float_as_uint(rbf_hw(u - hi)) >> 16);
         }
       }
     }
@@ -418,13 +432,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void g
       const float rstd = 1.f / sqrtf(ss / (float)RV + d.eps);
       const float z0 = bf2f(zs[t][h * RV + lane]), z1 = bf2f(zs[t][h * RV + lane + 64]);
       uint16_t* op = d.out + (bos + t) * RZ + (2 * hk + h) * RV + lane;
-      const uint32_t y0 = f2bf(((o0 * rstd) * nws[lane]) * (z0 * sigmoid_q(z0)));
-      const uint32_t y1 = f2bf(((o1 * rstd) * nws[lane + 64]) * (z1 * sigmoid_q(z1)));
-      op[0] = (uint16_t)y0;
-      op[64] = (uint16_t)y1;
+      const uint32_t y = pack_bf2_hw(((o0 * rstd) * nws[lane]) * (z0 * sigmoid_q(z0)),
+                                     ((o1 * rstd) * nws[lane + 64]) * (z1 * sigmoid_q(z1)));
+      op[0] = (uint16_t)y;
+      op[64] = (uint16_t)(y >> 16);
       if (d.oq) {
         // the value head's 128 outputs are one e4m3 group of the out_proj's input (the wave's lanes)
-        const float f0 = bf2f(y0), f1 = bf2f(y1);
+        const float f0 = bf_lo(y), f1 = bf_hi(y);
         const float m = wave_max(fmaxf(fabsf(f0), fabsf(f1)));
         const float inv = m > 0.f ? 448.f / m : 0.f;
         const uint32_t cd = f2e4m3x2_hw(f0 * inv, f1 * inv);
@@ -485,8 +499,10 @@ extern "C" int q36_gdn_verify_ring(const q36_gdn_ring_args* a, q36_stream_t stre
                a->write_pos, a->cache_base, static_cast<const uint16_t*>(a->norm_w), a->eps, a->scale,
                static_cast<uint16_t*>(a->out), static_cast<uint8_t*>(a->oq), a->oqs};
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  if (a->T <= 4) gdn_ring_kernel<4><<<a->B * RHK, 512, 0, st>>>(d);
-  else if (a->T == 5) gdn_ring_kernel<5><<<a->B * RHK, 512, 0, st>>>(d);
-  else gdn_ring_kernel<8><<<a->B * RHK, 512, 0, st>>>(d);
+  if (a->T == 4) gdn_ring_kernel<4, true><<<a->B * RHK, 512, 0, st>>>(d);
+  else if (a->T < 4) gdn_ring_kernel<4, false><<<a->B * RHK, 512, 0, st>>>(d);
+  else if (a->T == 5) gdn_ring_kernel<5, true><<<a->B * RHK, 512, 0, st>>>(d);
+  else if (a->T == 8) gdn_ring_kernel<8, true><<<a->B * RHK, 512, 0, st>>>(d);
+  else gdn_ring_kernel<8, false><<<a->B * RHK, 512, 0, st>>>(d);
   return check_launch("q36_gdn_verify_ring");
 }

@@ -108,6 +108,13 @@ def test_ring_edges(gdn, oracle_mod, dev, T, wp):
     _case(gdn, oracle_mod, dev, 4, T, seed=3 + T, wp=wp)
 
 
+@pytest.mark.parametrize("T", [3, 4, 5, 6, 7, 8])
+def test_ring_window_lengths(gdn, oracle_mod, dev, T):
+    """The window lengths with a kernel of their own (4, 5, 8) and those that share one, with a history that
+    the appends run over and a padded request."""
+    _case(gdn, oracle_mod, dev, 3, T, seed=40 + T, wp=11, padded=(1,))
+
+
 def test_ring_int32_indices_bf16_dt_padding_and_window_view(gdn, oracle_mod, dev):
     _case(gdn, oracle_mod, dev, 6, 4, seed=9, padded=(0, 4), idx32=True, dt_bf16=True, view4=True)
 
