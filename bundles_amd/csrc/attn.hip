@@ -63,8 +63,8 @@ __global__ __launch_bounds__(256) void act_quant_kernel(const uint16_t* x, const
       const v4i gv = ldg16a(reinterpret_cast<const uint8_t*>(gate + (size_t)t * K + 8 * c));
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        f[2 * i] = rbf(f[2 * i] * sigmoid_q(bf_lo((uint32_t)gv[i])));
-        f[2 * i + 1] = rbf(f[2 * i + 1] * sigmoid_q(bf_hi((uint32_t)gv[i])));
+        f[2 * i] = rbf_hw(f[2 * i] * sigmoid_q(bf_lo((uint32_t)gv[i])));
+        f[2 * i + 1] = rbf_hw(f[2 * i + 1] * sigmoid_q(bf_hi((uint32_t)gv[i])));
       }
     }
     float m = 0.f;
@@ -247,7 +247,7 @@ __global__ __launch_bounds__(256) void proj_gemm_kernel(GemmDev g) {
         if (col < g.nout) {
           const int sg = (g.nseg > 1 && col >= g.c0[1]) + (g.nseg > 2 && col >= g.c0[2]) + (g.nseg > 3 && col >= g.c0[3]);
           *reinterpret_cast<uint2*>(g.ys[sg] + (size_t)t * g.ld[sg] + (col - g.c0[sg])) =
-              make_uint2(pack_bf2(acc[c][tt][0], acc[c][tt][1]), pack_bf2(acc[c][tt][2], acc[c][tt][3]));
+              make_uint2(pack_bf2_hw(acc[c][tt][0], acc[c][tt][1]), pack_bf2_hw(acc[c][tt][2], acc[c][tt][3]));
         }
       }
     }
@@ -381,7 +381,7 @@ ks_gemm_kernel(GemmDev g) {
     if (t < g.T && col < g.nout) {
       const int sg = (g.nseg > 1 && col >= g.c0[1]) + (g.nseg > 2 && col >= g.c0[2]) + (g.nseg > 3 && col >= g.c0[3]);
       *reinterpret_cast<uint2*>(g.ys[sg] + (size_t)t * g.ld[sg] + (col - g.c0[sg])) =
-          make_uint2(pack_bf2(v.x, v.y), pack_bf2(v.z, v.w));
+          make_uint2(pack_bf2_hw(v.x, v.y), pack_bf2_hw(v.z, v.w));
     }
   }
 }
@@ -559,7 +559,7 @@ __device__ __forceinline__ void tile_gemm_body(const GemmDev& g, const TileLds<B
         if (col < g.nout) {
           const int sg = (g.nseg > 1 && col >= g.c0[1]) + (g.nseg > 2 && col >= g.c0[2]) + (g.nseg > 3 && col >= g.c0[3]);
           *reinterpret_cast<uint2*>(g.ys[sg] + (size_t)t * g.ld[sg] + (col - g.c0[sg])) =
-              make_uint2(pack_bf2(acc[rt][tt][0], acc[rt][tt][1]), pack_bf2(acc[rt][tt][2], acc[rt][tt][3]));
+              make_uint2(pack_bf2_hw(acc[rt][tt][0], acc[rt][tt][1]), pack_bf2_hw(acc[rt][tt][2], acc[rt][tt][3]));
         }
       }
     }

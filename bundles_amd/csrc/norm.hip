@@ -64,7 +64,7 @@ __global__ __launch_bounds__(64) void add_rmsnorm_kernel(NormDev d) {
       }
       v4i nv;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) nv[q] = (int)pack_bf2(z[j][2 * q], z[j][2 * q + 1]);
+      for (int q = 0; q < 4; ++q) nv[q] = (int)pack_bf2_hw(z[j][2 * q], z[j][2 * q + 1]);
       *reinterpret_cast<v4i*>(d.residual + at) = nv;
     }
   }
@@ -81,7 +81,7 @@ __global__ __launch_bounds__(64) void add_rmsnorm_kernel(NormDev d) {
     v4i ov;
 #pragma unroll
     for (int q = 0; q < 4; ++q)
-      ov[q] = (int)pack_bf2((z[j][2 * q] * rstd) * (1.f + bf_lo((uint32_t)wv[q])),
+      ov[q] = (int)pack_bf2_hw((z[j][2 * q] * rstd) * (1.f + bf_lo((uint32_t)wv[q])),
                             (z[j][2 * q + 1] * rstd) * (1.f + bf_hi((uint32_t)wv[q])));
     *reinterpret_cast<v4i*>(d.out + (size_t)r * kNH + 8 * (lane + 64 * j)) = ov;
     if (d.q8) {
