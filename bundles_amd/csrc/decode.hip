@@ -87,8 +87,8 @@ struct DecodeDev {
 __device__ __forceinline__ void gated_e4m3(const DecodeDev& d, int tok, int head, int c, uint32_t o01, uint32_t o23) {
   const size_t at = (size_t)tok * (kQH * kDD) + head * kDD + 4 * c;
   const uint2 gv = *reinterpret_cast<const uint2*>(d.gate + at);
-  float f[4] = {rbf(bf_lo(o01) * sigmoid_q(bf_lo(gv.x))), rbf(bf_hi(o01) * sigmoid_q(bf_hi(gv.x))),
-                rbf(bf_lo(o23) * sigmoid_q(bf_lo(gv.y))), rbf(bf_hi(o23) * sigmoid_q(bf_hi(gv.y)))};
+  float f[4] = {rbf_hw(bf_lo(o01) * sigmoid_q(bf_lo(gv.x))), rbf_hw(bf_hi(o01) * sigmoid_q(bf_hi(gv.x))),
+                rbf_hw(bf_lo(o23) * sigmoid_q(bf_lo(gv.y))), rbf_hw(bf_hi(o23) * sigmoid_q(bf_hi(gv.y)))};
   float m = fmaxf(fmaxf(fabsf(f[0]), fabsf(f[1])), fmaxf(fabsf(f[2]), fabsf(f[3])));
 #pragma unroll
   for (int o = 16; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
@@ -602,7 +602,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
       } else {
         const float L = rowL[row], il = L > 0.f ? 1.f / L : 0.f;
         uint16_t* dst = d.out + (((size_t)b * NT + (row >> 3)) * kQH + h * kGQ + (row & 7)) * kDD + 4 * c;
-        const uint32_t o01 = pack_bf2(a[0] * il, a[1] * il), o23 = pack_bf2(a[2] * il, a[3] * il);
+        const uint32_t o01 = pack_bf2_hw(a[0] * il, a[1] * il), o23 = pack_bf2_hw(a[2] * il, a[3] * il);
         *reinterpret_cast<uint2*>(dst) = make_uint2(o01, o23);
         // a wave holds one row (rows * 64 threads, whole waves): its two 128-groups are its lane halves
         if (d.oq) gated_e4m3(d, b * NT + (row >> 3), h * kGQ + (row & 7), c, o01, o23);
@@ -671,7 +671,7 @@ __global__ __launch_bounds__(WPR == 4 ? 256 : 1024) void decode_combine_kernel(D
     for (int v = 1; v < WPR; ++v) a += sums[v][lane];
   }
   const float il = L > 0.f ? 1.f / L : 0.f;
-  const uint32_t o01 = pack_bf2(a[0] * il, a[1] * il), o23 = pack_bf2(a[2] * il, a[3] * il);
+  const uint32_t o01 = pack_bf2_hw(a[0] * il, a[1] * il), o23 = pack_bf2_hw(a[2] * il, a[3] * il);
   *reinterpret_cast<uint2*>(d.out + (size_t)qr * kDD + 4 * c) = make_uint2(o01, o23);
   // the wave holds the row: lanes 0-31 / 32-63 its two 128-groups
   if (d.oq) gated_e4m3(d, bt, head, c, o01, o23);

@@ -102,11 +102,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
 #pragma unroll
     for (int t = 0; t < kTMax; ++t) {
       if (t < T) {
-        float acc = rbf(w[t] * cw[0]);
-        acc = acc + rbf(w[t + 1] * cw[1]);
-        acc = acc + rbf(w[t + 2] * cw[2]);
-        acc = acc + rbf(w[t + 3] * cw[3]);
-        const float o = rbf(acc / (1.f + expf_q(-acc)));
+        float acc = rbf_hw(w[t] * cw[0]);
+        acc = acc + rbf_hw(w[t + 1] * cw[1]);
+        acc = acc + rbf_hw(w[t + 2] * cw[2]);
+        acc = acc + rbf_hw(w[t + 3] * cw[3]);
+        const float o = rbf_hw(acc / (1.f + expf_q(-acc)));
         if (part == 0) qs[t][i] = o;
         else if (part == 1) ks[t][i] = o;
         else vs[t][i] = o;
@@ -116,7 +116,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
     if (part == 2 || (hv & 1) == 0) {
       uint16_t* co = d.conv_state_out + ((size_t)bq * GQKV + ch) * 3;
 #pragma unroll
-      for (int q = 0; q < 3; ++q) co[q] = (uint16_t)f2bf(w[T + q]);
+      for (int q = 0; q < 3; ++q) co[q] = (uint16_t)(__float_as_uint(w[T + q]) >> 16);
     }
   } else {
     if (i < 16 * T) {
@@ -193,7 +193,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
       ov[h] = ov[h] + lane_xor<1>(ov[h]);
       ov[h] = ov[h] + lane_xor<2>(ov[h]);
       ov[h] = ov[h] + lane_xor<4>(ov[h]);
-      if (c8 == 0) os[t][r0 + 64 * h] = rbf(ov[h]);  // the core output is bf16
+      if (c8 == 0) os[t][r0 + 64 * h] = rbf_hw(ov[h]);  // the core output is bf16
     }
   }
   __syncthreads();
