@@ -825,8 +825,10 @@ extern "C" int q36_lmhead_argmax(const q36_lmhead_args* a, q36_stream_t stream) 
   Q36_REQUIRE(a != nullptr, "q36_lmhead_argmax: null args");
   Q36_REQUIRE(a->H == kLH, "q36_lmhead_argmax: H=%d unsupported (this build is specialised to 2048)", a->H);
   Q36_REQUIRE(a->R >= 1 && a->R <= (1 << 20), "q36_lmhead_argmax: R=%d out of range", a->R);
-  Q36_REQUIRE(a->V >= 16 && a->V % 16 == 0 && (!a->wq_t || a->V < (1 << 25)),
-              "q36_lmhead_argmax: V=%d must be a positive multiple of 16 (below 2^25 in the tile order)", a->V);
+  Q36_REQUIRE(a->V >= 16 && a->V % 16 == 0, "q36_lmhead_argmax: V=%d must be a positive multiple of 16", a->V);
+  // the tile-order GEMM addresses 16 rows of logits by 32-bit offsets
+  Q36_REQUIRE(!a->wq_t || !a->logits || a->mode == Q36_LMH_W8A16 || a->V < (1 << 25),
+              "q36_lmhead_argmax: V=%d must be below 2^25 for logits on the tile order in W8A8", a->V);
   Q36_REQUIRE(a->mode == Q36_LMH_W8A8 || a->mode == Q36_LMH_W8A8X2 || a->mode == Q36_LMH_W8A16,
               "q36_lmhead_argmax: mode %d unknown", a->mode);
   Q36_REQUIRE(a->mode != Q36_LMH_W8A16 || (a->R <= 64 && a->V % 32 == 0),
