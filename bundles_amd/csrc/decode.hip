@@ -138,7 +138,11 @@ __global__ __launch_bounds__(256) void kv_scatter_kernel(const uint8_t* k8, cons
 // How one call's keys are dealt to the workgroups of a KV head (G of them fit on the chip at once), in
 // steps of kST keys:
 //   pieces  each request in ceil(steps / c) equal pieces, one piece a workgroup, with the smallest c (from
-//           kMinPiece up) that needs no more than G pieces;
+//           kMinPiece up) that needs no more than G pieces.  The one-row-tile form, of which two workgroups
+//           fit a CU, takes no more than G / 2: one a CU reads as fast, and longer runs leave fewer
+//           partials (us, G against G / 2 pieces: 125 x 2 rows over 2580 .. 2995 keys 79.3 -> 73.4,
+//           52 x 1 over 2325 37.6 -> 35.1, 3 x 1 over 20000 .. 32000 30.1 -> 26.8, 12 x 1 over 2984 ..
+//           3471 22.2 -> 19.3);
 //   line    where there are more requests than G, or a few long ones among many would make that c much
 //           more than an equal share: a request weighs its steps plus ovh (what starting and merging a
 //           run costs beside its steps), half before and half after them, and the line of all
@@ -149,12 +153,14 @@ __global__ __launch_bounds__(256) void kv_scatter_kernel(const uint8_t* k8, cons
 // captured launch follows the lengths it finds.  With a fixed number of splits per request, as before,
 // the longest request sets a call's time.  Measured, us a call (fixed -> dealt): 64 x 4 rows over 128 ..
 // 8192 keys 86.9 -> 47.9, 256 x 1 over 20 .. 4000 107.8 -> 58.0, 150 x 4 over 300 .. 6000 134 -> 83.9, 12 x 2
-// over 3000 .. 30000 60.1 -> 41.9; equal lengths: 64 x 4 over 4096 64.5 -> 64.8, 256 x 1 over 4000 177 -> 182
-// (the combine launch, which finds nothing cut).
+// over 3000 .. 30000 60.1 -> 39.9.  Equal lengths gain nothing and pay for the dealing and for a combine that
+// may find nothing cut: 64 x 4 over 4096 64.5 -> 64.8, 256 x 1 over 4000 177 -> 182, 26 x 2 over 7656 48.8 ->
+// 53.3 (short tables keep fixed splits: see q36_attn_decode).
 // ovh: 4 / 12 / 20 / 28 steps gave 58.5 / 52.2 / 49.3 / 50.3 us on the first of these (two row tiles) and
 // 56.5 / 57.2 / 63.7 / 70.7 on the second (one).  kMinPiece: 2 / 4 / 8 steps 25.0 / 22.5 / 22.9 us for one
 // request of 4 rows over 8000 keys, 14.0 / 14.6 / 16.0 us for one of 1 row over 1000.
 constexpr int kMinPiece = 4, kWhole = 8;
+constexpr int kAlone = 12, kEven = 40;  // fixed splits: steps (see q36_attn_decode)
 constexpr int ovh(int RT) { return RT == 1 ? 8 : 16; }
 // share w of nsh begins at total * w / nsh; the share that holds position x
 __device__ __forceinline__ int share_begin(int total, int nsh, int w) { return (int)((int64_t)total * w / nsh); }
@@ -221,9 +227,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
       rkeys[t] = rk;
       __syncthreads();
       const int steps = rsum[0] + rsum[1] + rsum[2] + rsum[3], total = steps + d.B * kOvh;
-      const int c0 = max((steps + G - 1) / G, kMinPiece);
+      // pieces at most, and how much more than an equal share one may hold
+      const int Gp = RT == 1 && d.B <= G / 2 && steps >= kMinPiece * (G / 2) ? G / 2 : G;
+      constexpr int kSlack = RT == 1 ? 8 : 4;
+      const int c0 = max((steps + Gp - 1) / Gp, kMinPiece);
       int pc = 0;
-      if (d.B <= min(G, 256)) {
+      if (d.B <= min(Gp, 256)) {
         // 16 piece sizes c0 .. about 2 c0, four a wave
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
@@ -235,9 +244,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
         }
         __syncthreads();
         const int n = npiece[t & 15];
-        const uint64_t fits = __builtin_amdgcn_ballot_w64(n <= G) & 0xffffu;
+        const uint64_t fits = __builtin_amdgcn_ballot_w64(n <= Gp) & 0xffffu;
         const int k = fits ? __builtin_ctzll(fits) : 0, c = c0 + (c0 * k + 15) / 16;
-        if (fits && c <= total / G + total / (4 * G) + 2) {
+        if (fits && c <= total / Gp + total / (kSlack * Gp) + 2) {
           if (wg >= __builtin_amdgcn_readlane(n, k)) return;
           pc = c;
         }
@@ -730,12 +739,26 @@ extern "C" int q36_attn_decode(const q36_decode_args* a, q36_stream_t stream) {
   Q36_REQUIRE(!a->oq || ((reinterpret_cast<uintptr_t>(a->gate) & 7u) == 0 &&
                          (reinterpret_cast<uintptr_t>(a->oq) & 3u) == 0 && (reinterpret_cast<uintptr_t>(a->oqs) & 3u) == 0),
               "q36_attn_decode: gate must be 8-byte, oq and oqs 4-byte aligned");
+  const bool one = a->NT <= 2;  // one row tile, two workgroups a CU
+  const int cus = decode_cus(), resident = (one ? kDecWPE1 : 1) * cus;
+  const int max_steps = (a->pt_stride - 1) / kST + 1;
+  // Dealing costs about 3 us and a combine 5; where no length the table can hold makes that good, the
+  // splits are fixed: whole requests up to kAlone steps, and a few splits of at most kEven steps, in the
+  // two-row-tile form of kEven steps together (more splits gain from the dealing even at equal lengths).
+  // Measured, us a call (dealt, fixed): 84 x 1 row over 191 keys 18.4, 9.5; 56 x 1 over 646 21.7, 15.2; 101 x 2
+  // over 250 .. 877 26.0, 21.7; 39 x 1 over 1101 22.1, 17.5; 117 x 3 over 131 .. 187 19.4, 16.7; 44 x 3 over 644 .. 879 25.8, 22.2; on the other
+  // side 95 x 2 over 750 .. 2445 43.0, 48.6; 46 x 4 over 650 .. 3800 37.2, 49.1.
+  const auto fixed = [&] {
+    const int so = decode_splits(a->B, 0);
+    const int s = max_steps <= kAlone ? 1 : so <= (one ? 4 : 2) && max_steps <= kEven * (one ? so : 1) ? so : 0;
+    return (int64_t)a->B * kKVH * s <= resident && a->workspace_bytes >= decode_ws_bytes(a->B, std::max(s, 1)) ? s : 0;
+  };
+  const int s0 = a->splits > 0 ? a->splits : fixed();
   // balanced unless a split count was asked for (or the workspace holds only the equal splits', or the
   // line's length might not fit 31 bits)
-  const int max_steps = (a->pt_stride - 1) / kST + 1;
-  const bool bal = a->splits <= 0 && a->workspace_bytes >= decode_bal_bytes(a->B) &&
+  const bool bal = s0 == 0 && a->workspace_bytes >= decode_bal_bytes(a->B) &&
                    (int64_t)a->B * ((int64_t)max_steps + ovh(2)) < (1 << 30);
-  const int S = bal ? 0 : decode_splits(a->B, a->splits);
+  const int S = bal ? 0 : decode_splits(a->B, s0);
   const size_t need = bal ? decode_bal_bytes(a->B) : decode_ws_bytes(a->B, S);
   Q36_REQUIRE(a->workspace_bytes >= need, "q36_attn_decode: workspace of %zu bytes < %zu required", a->workspace_bytes,
               need);
@@ -747,13 +770,12 @@ extern "C" int q36_attn_decode(const q36_decode_args* a, q36_stream_t stream) {
                                                             static_cast<const uint8_t*>(a->v_new), a->out_loc, T, a->num_slots,
                                                             static_cast<uint8_t*>(a->k_cache),
                                                             static_cast<uint8_t*>(a->v_cache));
-  const bool one = a->NT <= 2;  // one row tile, two workgroups a CU
-  const int cus = decode_cus(), slots = bal ? 2 * cus : a->B * kKVH * S;  // of kDRows rows
+  const int slots = bal ? 2 * cus : a->B * kKVH * S;  // of kDRows rows
   // balanced: as many workgroups per KV head as the chip holds at once, and no more than pieces of a
   // table of this width; a table so narrow that no request is cut needs no combine
   const int nocut = max_steps <= kMinPiece;
   const int64_t pieces = (int64_t)a->B * ((max_steps - 1) / kMinPiece + 1);
-  const int shares = (int)std::min<int64_t>(std::max(1, (one ? kDecWPE1 : 1) * cus / kKVH), pieces);
+  const int shares = (int)std::min<int64_t>(std::max(1, resident / kKVH), pieces);
   DecodeDev d{a->B, a->NT, a->pt_stride, S, nocut, max_steps,
               static_cast<const uint16_t*>(a->q), static_cast<const uint8_t*>(a->k_cache),
               static_cast<const uint8_t*>(a->v_cache), (int64_t)a->num_slots * kKVH * kDD, a->page_table, a->seqlens,

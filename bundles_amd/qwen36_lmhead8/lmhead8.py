@@ -52,7 +52,7 @@ def w8a8_lmhead_argmax(h, q, scale, ws: Workspace, norm_w=None, eps: float = 1e-
     next_token_logits_buffer, H/node.py:68-88,136-149).  two_term: the reference's two-term activation
     form (H/w8a8.py:25-37); w8a16: the bf16 rows times the int8 weights unquantized (H/lmhead8.py:57-91;
     R <= 64, V a multiple of 32); q_t (optional): tile_rows_w16(q), read instead of q by every form, q
-    may then be None (the same bits; 3-5 % faster for W8A8, 20-30 % for W8A16)."""
+    may then be None (the same bits; 13 % faster for W8A8 at 2048 rows, 15-30 % for W8A16)."""
     R, H = h.shape
     if q is None and q_t is None:
         raise ValueError("w8a8_lmhead_argmax: q or q_t is required")

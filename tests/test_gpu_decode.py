@@ -231,6 +231,27 @@ def test_decode_balanced_shares(attn, oracle_mod, dev, NT, seqlens):
         assert_bf16_close(bits16(out2).reshape(-1, D), bits16(out).reshape(-1, D), 2e-3, "fixed splits")
 
 
+@pytest.mark.parametrize("NT,seqlens", [
+    (1, [5, 384, 0, 70]), (4, [384, 4, 129]),            # tables of up to 12 steps: whole requests
+    (2, _ragged(70, 20, 400, [1280, 0], 5)),             # one split of up to 40 steps
+    (1, _ragged(50, 300, 900, [2560], 6)),               # two
+    (3, _ragged(100, 3, 500, [1280], 7)),                # two row tiles, one split
+    (1, [9000, 8000, 4]),                                # one row tile, pieces: one workgroup a CU
+], ids=["whole1", "whole4", "70", "50", "100", "3"])
+def test_decode_default_route(attn, oracle_mod, dev, NT, seqlens):
+    """The default route by the table's width and the batch, against the oracle; requests without keys give zeros."""
+    B = len(seqlens)
+    print(f"attn_decode default NT={NT} B={B}", flush=True)
+    h = _make(B, NT, [max(n, NT) for n in seqlens], seed=5 * NT + B)
+    h["pt"] = h["pt"][:, :max(seqlens)].contiguous()
+    ref = _oracle(oracle_mod, h, NT).reshape(B, -1, D)
+    h["seqlens"] = torch.tensor(seqlens, dtype=torch.int32)
+    got = bits16(_run(attn, h, NT, dev)[0]).reshape(B, -1, D)
+    keep = [i for i, n in enumerate(seqlens) if n]
+    assert not got[[i for i, n in enumerate(seqlens) if not n]].any()
+    assert_bf16_close(got[keep].reshape(-1, D), ref[keep].reshape(-1, D), 1e-2, f"default NT={NT} B={B}")
+
+
 def test_decode_balanced_empty_requests(attn, oracle_mod, dev):
     """Requests without keys (a padded batch's) give zeros and leave the others as they are."""
     NT, seqlens = 2, [70, 0, 900, 0, 2, 1500]
