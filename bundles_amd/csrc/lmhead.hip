@@ -205,7 +205,8 @@ __host__ __device__ __forceinline__ int lmh_groups(int nrt) { return nrt >= 8 &&
 // vocab tile run side by side on one XCD (its weight tile comes from HBM once per XCD), and an
 // XCD's activations (2 MB at 2048 rows) stay resident in its L2 while the weights stream through.
 //
-// STORE: 0 no logits, 1 bf16 logits, 2 fp32 logits (the bf16-rounded values widened).
+// STORE: 0 no logits, 1 bf16 logits, 2 fp32 logits (the bf16-rounded values widened); 3 and 4: as 1 and 2
+// with 64-bit addresses, for vocabularies whose 16 rows of logits pass 32-bit offsets.
 constexpr int lmh_wd(int VT, int TB) { return VT * TB <= 16 ? 8 : 4; }  // weight steps in flight (divides the 32 steps)
 // Whether step k requests the weights of step k + WD: past the tile's end only the first half of the
 // next tile's first WD steps (the rest after the epilogue, across which they would spill).
@@ -354,13 +355,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int b = 0; b < NT; ++b) {
       const int t = X2 ? 2 * b : b;
       // the logits through a buffer of the token tile's rows in range (a row past it is not written)
-      constexpr int es = STORE == 2 ? 4 : 2;
+      constexpr bool F32 = STORE == 2 || STORE == 4, BF16 = STORE == 1 || STORE == 3, WIDE = STORE >= 3;
+      constexpr int es = F32 ? 4 : 2;
       const int64_t lbytes = ((int64_t)min(ntok - 16 * b, 16) * d.V - cur.v0) * es;
       uint8_t* lbase = STORE == 0 ? nullptr
-                                  : (STORE == 2 ? reinterpret_cast<uint8_t*>(d.logits32) : reinterpret_cast<uint8_t*>(d.logits)) +
+                                  : (F32 ? reinterpret_cast<uint8_t*>(d.logits32) : reinterpret_cast<uint8_t*>(d.logits)) +
                                         ((size_t)(tok0 + 16 * b) * d.V + cur.v0) * es;
       const __amdgpu_buffer_rsrc_t lrs =
-          __builtin_amdgcn_make_buffer_rsrc((void*)lbase, (short)0, (int)max(lbytes, (int64_t)0), 0x00020000);
+          __builtin_amdgcn_make_buffer_rsrc((void*)lbase, (short)0, WIDE ? 0 : (int)max(lbytes, (int64_t)0), 0x00020000);
+      // four words at column c of the lane's token
+      auto put = [&](v4i o, int c, bool ok) {
+        if constexpr (WIDE) {
+          if (ok && 16 * b + l16 < ntok) *reinterpret_cast<v4i*>(lbase + ((int64_t)l16 * d.V + c) * es) = o;
+        } else {
+          __builtin_amdgcn_raw_buffer_store_b128(o, lrs, ok ? (l16 * d.V + c) * es : 0x7fffff00, 0, kLogitAux);
+        }
+      };
       const float x1 = xsc[16 * t + l16], x2 = X2 ? xsc[16 * (t + 1) + l16] : 0.f;
       float bv = -__builtin_inff();
       int bi = 0;
@@ -378,19 +388,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             lg4[q] = rbf_hw(((float)acc[a][t][q] * x1) * wq[q]);
           if (in && lg4[q] > bv) bv = lg4[q], bi = 16 * a + q;
         }
-        if constexpr (STORE == 1) {
+        if constexpr (BF16) {
           pk[a][0] = (__float_as_uint(lg4[0]) >> 16) | (__float_as_uint(lg4[1]) & 0xffff0000u);
           pk[a][1] = (__float_as_uint(lg4[2]) >> 16) | (__float_as_uint(lg4[3]) & 0xffff0000u);
         }
-        if constexpr (STORE == 2) {
+        if constexpr (F32) {
           // a token's 16 columns of the tile are 64 contiguous bytes over its four lanes
           const v4i o = {(int)__float_as_uint(lg4[0]), (int)__float_as_uint(lg4[1]), (int)__float_as_uint(lg4[2]),
                          (int)__float_as_uint(lg4[3])};
-          const int at = (l16 * d.V + vb + 16 * a + 4 * lg) * 4;
-          __builtin_amdgcn_raw_buffer_store_b128(o, lrs, in ? at : 0x7fffff00, 0, kLogitAux);
+          put(o, vb + 16 * a + 4 * lg, in);
         }
       }
-      if constexpr (STORE == 1) {
+      if constexpr (BF16) {
         // Lanes 16 apart exchange halves of two vocab tiles, so that a lane holds 8 consecutive columns and
         // the four lanes of a token 32 (64 contiguous bytes): lane group (s1, s0) with tiles (a1, a0) ends
         // with columns 32 a1 + 16 s0 + 8 s1 .. + 7.
@@ -400,8 +409,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           const auto p1 = __builtin_amdgcn_permlane16_swap(pk[2 * a1][1], pk[2 * a1 + 1][1], false, false);
           const v4i o = {(int)p0[0], (int)p1[0], (int)p0[1], (int)p1[1]};
           const int cl = 32 * a1 + 16 * (lg & 1) + 8 * (lg >> 1);
-          const int at = (l16 * d.V + vb + cl) * 2;
-          __builtin_amdgcn_raw_buffer_store_b128(o, lrs, cl < nva ? at : 0x7fffff00, 0, kLogitAux);
+          put(o, vb + cl, cl < nva);
         }
       }
       uint32_t b16 = __float_as_uint(bv + 0.f) >> 16;
@@ -826,9 +834,6 @@ extern "C" int q36_lmhead_argmax(const q36_lmhead_args* a, q36_stream_t stream) 
   Q36_REQUIRE(a->H == kLH, "q36_lmhead_argmax: H=%d unsupported (this build is specialised to 2048)", a->H);
   Q36_REQUIRE(a->R >= 1 && a->R <= (1 << 20), "q36_lmhead_argmax: R=%d out of range", a->R);
   Q36_REQUIRE(a->V >= 16 && a->V % 16 == 0, "q36_lmhead_argmax: V=%d must be a positive multiple of 16", a->V);
-  // the tile-order GEMM addresses 16 rows of logits by 32-bit offsets
-  Q36_REQUIRE(!a->wq_t || !a->logits || a->mode == Q36_LMH_W8A16 || a->V < (1 << 25),
-              "q36_lmhead_argmax: V=%d must be below 2^25 for logits on the tile order in W8A8", a->V);
   Q36_REQUIRE(a->mode == Q36_LMH_W8A8 || a->mode == Q36_LMH_W8A8X2 || a->mode == Q36_LMH_W8A16,
               "q36_lmhead_argmax: mode %d unknown", a->mode);
   Q36_REQUIRE(a->mode != Q36_LMH_W8A16 || (a->R <= 64 && a->V % 32 == 0),
@@ -907,7 +912,7 @@ extern "C" int q36_lmhead_argmax(const q36_lmhead_args* a, q36_stream_t stream) 
   // last round would otherwise be mostly empty (64 rows two terms: 594 tiles for 512 places, 71.6 -> 69.5
   // us; 150 rows 127 -> 131 us, 2048 one term 491 -> 551 us, so not there).
   const int64_t nrt8 = (d.Rs + 127) / 128, nv4 = (a->V + 255) / 256, nv2 = (a->V + 127) / 128, slots = 2 * cus;
-  const bool small = (nv2 * nrt8 + slots - 1) / slots * 640 < (nv4 * nrt8 + slots - 1) / slots * 1024;
+  const bool small = a->V < 1 << 25 && (nv2 * nrt8 + slots - 1) / slots * 640 < (nv4 * nrt8 + slots - 1) / slots * 1024;
   auto go = [&](auto vtc, auto x2c) {
     constexpr int VT = decltype(vtc)::value, TB = 8;
     constexpr bool X2 = decltype(x2c)::value;
@@ -916,6 +921,16 @@ extern "C" int q36_lmhead_argmax(const q36_lmhead_args* a, q36_stream_t stream) 
     // persistent: two workgroups per CU (a multiple of 8, one XCD in eight), never more than the
     // busiest XCD's tiles
     const int blocks = 8 * (int)std::max<int64_t>(1, std::min<int64_t>(2 * cus / 8, (int64_t)((nvt + vstep - 1) / vstep) * (nrt / ngrp)));
+    // 16 rows of fp32 logits reach past 31 bits of byte offset from 2^25 columns on
+    if constexpr (VT == 4) {
+      if ((d.logits || d.logits32) && a->V >= 1 << 25) {
+        if (d.logits32)
+          lmh_gemm_kernel<VT, TB, X2, 4><<<blocks, 256, 0, st>>>(d);
+        else
+          lmh_gemm_kernel<VT, TB, X2, 3><<<blocks, 256, 0, st>>>(d);
+        return;
+      }
+    }
     if (d.logits32)
       lmh_gemm_kernel<VT, TB, X2, 2><<<blocks, 256, 0, st>>>(d);
     else if (d.logits)

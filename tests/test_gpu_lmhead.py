@@ -154,3 +154,30 @@ def test_lmhead_tile_forms_agree(lmh, dev, R, two_term, f32):
     assert torch.equal(logits.to(torch.bfloat16), want) and torch.equal(logits_r, want)
     first = (want == want.float().amax(1, keepdim=True).to(want.dtype)).to(torch.int8).argmax(1)
     assert torch.equal(ids.long(), first) and torch.equal(ids_r, ids)
+
+
+@pytest.mark.parametrize("R,two_term,f32", [(35, False, True), (20, True, False)])
+def test_lmhead_logits_past_32_bit_offsets(lmh, dev, R, two_term, f32):
+    """A vocabulary whose 16 rows of fp32 logits pass 2^31 bytes (and a tail of one 16-row tile): the logits
+    of its slices bit for bit, the ids the first largest."""
+    V = (1 << 25) + 16
+    if torch.cuda.mem_get_info()[0] < 90 << 30:
+        pytest.skip("64 GiB of codes do not fit the free memory")
+    print(f"lmhead wide R={R} two_term={two_term} f32={f32}", flush=True)
+    g = torch.Generator(device=dev)
+    g.manual_seed(R)
+    h = torch.randn((R, 2048), generator=g, device=dev).to(torch.bfloat16)
+    s = torch.rand(V, generator=g, device=dev) * 1e-3 + 1e-4
+    codes = torch.empty((V, 2048), dtype=torch.int8, device=dev)  # random codes, so in tile order as well
+    for v0 in range(0, V, 1 << 20):
+        codes[v0:v0 + (1 << 20)].random_(-127, 128, generator=g)
+    ws = lmh.Workspace(R, dev)
+    buf = torch.full((R, V), -7.0, dtype=torch.float32 if f32 else torch.bfloat16, device=dev)
+    ids, logits = lmh.w8a8_lmhead_argmax(h, None, s, ws, logits=buf, two_term=two_term, q_t=codes)
+    for v0 in (0, 1 << 20, (1 << 24) - 512, (1 << 25) - 4096, V - 272):
+        n = min(4096, V - v0)
+        _, want = lmh.w8a8_lmhead_argmax(h, None, s[v0:v0 + n].contiguous(), ws, want_logits=True, two_term=two_term,
+                                         q_t=codes[v0:v0 + n])
+        assert torch.equal(logits[:, v0:v0 + n].to(torch.bfloat16), want), v0
+    for r in range(R):
+        assert int(ids[r]) == int((logits[r] == logits[r].max()).nonzero()[0]), r
