@@ -34,12 +34,12 @@
 
 #include "q36_device.h"
 #include "q36_host.h"
+#include "q36_deal.h"
 
 namespace q36 {
 namespace {
 
 constexpr int kQH = 16, kKVH = 2, kDD = 256, kGQ = kQH / kKVH, kDNT = 4, kDRows = kGQ * kDNT;
-constexpr int kST = 32;              // keys per wave step
 // NS (kernel template): key / value stages per wave (steps in flight + 1); the page-table entries run
 // 2 NS steps ahead, so an entry's DMA is older than every key and value load a wait leaves in flight
 // The two forms' shapes (alternating builds on one box, three rounds): the one-row-tile form (decode,
@@ -136,7 +136,7 @@ __global__ __launch_bounds__(256) void kv_scatter_kernel(const uint8_t* k8, cons
 }
 
 // How one call's keys are dealt to the workgroups of a KV head (G of them fit on the chip at once), in
-// steps of kST keys:
+// steps of kST keys (the arithmetic is q36_deal.h's):
 //   pieces  each request in ceil(steps / c) equal pieces, one piece a workgroup, with the smallest c (from
 //           kMinPiece up) that needs no more than G pieces.  The one-row-tile form, of which two workgroups
 //           fit a CU, takes no more than G / 2: one a CU reads as fast, and longer runs leave fewer
@@ -146,7 +146,7 @@ __global__ __launch_bounds__(256) void kv_scatter_kernel(const uint8_t* k8, cons
 //   line    where there are more requests than G, or a few long ones among many would make that c much
 //           more than an equal share: a request weighs its steps plus ovh (what starting and merging a
 //           run costs beside its steps), half before and half after them, and the line of all
-//           weights is cut into G equal shares.  A share holds the end of one request, whole requests
+//           weights is cut into G equal shares (as many as positions if these are fewer).  A share holds the end of one request, whole requests
 //           and the start of another; requests of at most kWhole steps are not cut but belong to the
 //           share that holds their start.
 // Every workgroup works the dealing out for itself from seqlens (about 1 us, before its first key), so a
@@ -159,13 +159,7 @@ __global__ __launch_bounds__(256) void kv_scatter_kernel(const uint8_t* k8, cons
 // ovh: 4 / 12 / 20 / 28 steps gave 58.5 / 52.2 / 49.3 / 50.3 us on the first of these (two row tiles) and
 // 56.5 / 57.2 / 63.7 / 70.7 on the second (one).  kMinPiece: 2 / 4 / 8 steps 25.0 / 22.5 / 22.9 us for one
 // request of 4 rows over 8000 keys, 14.0 / 14.6 / 16.0 us for one of 1 row over 1000.
-constexpr int kMinPiece = 4, kWhole = 8;
 constexpr int kAlone = 12, kEven = 40;  // fixed splits: steps (see q36_attn_decode)
-constexpr int ovh(int RT) { return RT == 1 ? 8 : 16; }
-// share w of nsh begins at total * w / nsh; the share that holds position x
-__device__ __forceinline__ int share_begin(int total, int nsh, int w) { return (int)((int64_t)total * w / nsh); }
-__device__ __forceinline__ int share_of(int total, int nsh, int x) { return (int)((((int64_t)x + 1) * nsh - 1) / total); }
-__device__ __forceinline__ int req_steps(int nk) { return nk > 0 ? (nk + kST - 1) / kST : 0; }
 // Integer sum over the wave, and inclusive scan, without LDS (the plan runs before the first load of a key).
 __device__ __forceinline__ int wave_sum_i(int v) {
   v += (int)dpp_u32<0xB1>((uint32_t)v);
@@ -212,7 +206,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
   // so that no register holds it across a run): the share, the next request, the chunk of requests
   __shared__ int roff[256], rkeys[256], rsum[4], npiece[16];
   __shared__ int lx0, lx1, ltotal, lnsh, lpc, li, lhi, lc0, lbase;
-  constexpr int kOvh = ovh(RT);
   const int h = blockIdx.x & 1;
   {
     const int t = run_tid();
@@ -226,35 +219,34 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
       roff[t] = st;
       rkeys[t] = rk;
       __syncthreads();
-      const int steps = rsum[0] + rsum[1] + rsum[2] + rsum[3], total = steps + d.B * kOvh;
-      // pieces at most, and how much more than an equal share one may hold
-      const int Gp = RT == 1 && d.B <= G / 2 && steps >= kMinPiece * (G / 2) ? G / 2 : G;
-      constexpr int kSlack = RT == 1 ? 8 : 4;
-      const int c0 = max((steps + Gp - 1) / Gp, kMinPiece);
+      const int steps = rsum[0] + rsum[1] + rsum[2] + rsum[3], total = steps + d.B * ovh(RT);
+      const int Gp = piece_places(RT, d.B, G, steps), c0 = piece_least(steps, Gp);
       int pc = 0;
       if (d.B <= min(Gp, 256)) {
-        // 16 piece sizes c0 .. about 2 c0, four a wave
+        // the kSizes piece sizes, four a wave
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-          const int kk = 4 * (t >> 6) + k, c = c0 + (c0 * kk + 15) / 16;
+          const int kk = 4 * (t >> 6) + k, c = piece_size(c0, kk);
           int n = 0;
-          for (int q = t & 63; q < d.B; q += 64) n += max((roff[q] + c - 1) / c, 1);
+          for (int q = t & 63; q < d.B; q += 64) n += req_pieces(roff[q], c);
           n = wave_sum_i(n);
           if ((t & 63) == 0) npiece[kk] = n;
         }
         __syncthreads();
         const int n = npiece[t & 15];
         const uint64_t fits = __builtin_amdgcn_ballot_w64(n <= Gp) & 0xffffu;
-        const int k = fits ? __builtin_ctzll(fits) : 0, c = c0 + (c0 * k + 15) / 16;
-        if (fits && c <= total / Gp + total / (kSlack * Gp) + 2) {
-          if (wg >= __builtin_amdgcn_readlane(n, k)) return;
+        const int k = fits ? __builtin_ctzll(fits) : 0, c = piece_size(c0, k), nk = __builtin_amdgcn_readlane(n, k);
+        if (pieces_taken(RT, nk, c, total, Gp)) {
+          if (wg >= nk) return;
           pc = c;
         }
       }
+      const int nsh = line_shares(total, G);
+      if (!pc && wg >= nsh) return;
       if (t == 0) {
         lpc = pc;
         if (pc) lx0 = wg, lx1 = wg + 1;
-        else lx0 = share_begin(total, G, wg), lx1 = share_begin(total, G, wg + 1), ltotal = total, lnsh = G;
+        else lx0 = share_begin(total, nsh, wg), lx1 = share_begin(total, nsh, wg + 1), ltotal = total, lnsh = nsh;
       }
     }
     if (t == 0) li = 0, lhi = 0, lc0 = -256, lbase = 0;
@@ -273,7 +265,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
       if (c0 >= d.B || base >= x1) return;
       const bool in = c0 + t < d.B;
       const int rk = c0 == 0 ? rkeys[t] : in ? d.seqlens[c0 + t] : 0, st = min(req_steps(rk), d.max_steps);
-      const int w = !in ? 0 : pc ? max((st + pc - 1) / pc, 1) : st + kOvh;
+      const int w = !in ? 0 : pc ? req_pieces(st, pc) : st + ovh(RT);
       const int inc = wave_scan_i(w);
       __syncthreads();  // the state above has been read
       if ((t & 63) == 63) rsum[t >> 6] = inc;
@@ -291,32 +283,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
     }
     b = __builtin_amdgcn_readfirstlane(lc0) + i;
     nk = __builtin_amdgcn_readfirstlane(rkeys[i]);
-    const int off0 = __builtin_amdgcn_readfirstlane(roff[i]), off = off0 + kOvh / 2;  // (line) of its first step
+    const int off0 = __builtin_amdgcn_readfirstlane(roff[i]);
     const int steps = req_steps(nk);
     __syncthreads();
     if (t == 0) li = i + 1;
     __syncthreads();
+    const int wg = (int)blockIdx.x >> 1;
+    DealRun r;
+    int last;  // of the workgroups that hold a piece of the request, this one being the first
     if (pc) {
-      const int n = max((min(steps, d.max_steps) + pc - 1) / pc, 1), p = x0 - off0, per = steps / n, rem = steps % n;
-      st0 = p * per + min(p, rem);
-      nst = per + (p < rem ? 1 : 0);
-      slot = n > 1 ? 2 * (int)blockIdx.x + (p == 0) : -1;
-      if (p == 0 && t == 0 && h == 0) d.meta[b] = make_int2(x0, x0 + n - 1);
-    } else
-    // (a key count past the page table's width is not cut either: its weight is the table's)
-    if (steps <= kWhole || steps > d.max_steps || d.nocut) {
-      if (off0 < x0) continue;
-      st0 = 0, nst = steps, slot = -1;
-      if (t == 0 && h == 0) d.meta[b] = make_int2(0, 0);
+      const int n = req_pieces(min(steps, d.max_steps), pc), p = x0 - off0;
+      r = piece_run(steps, n, p);
+      last = wg + n - 1;
     } else {
-      const int e = min(x1 - off, steps);
-      st0 = max(x0 - off, 0);
-      nst = e - st0;
-      if (nst <= 0) continue;
-      slot = nst == steps ? -1 : 2 * (int)blockIdx.x + (st0 == 0);
-      if (st0 == 0 && t == 0 && h == 0)
-        d.meta[b] = make_int2((int)blockIdx.x >> 1, share_of(ltotal, lnsh, off + steps - 1));
+      // (a key count past the page table's width is not cut either: its weight is the table's)
+      r = line_run(steps, off0, ovh(RT) / 2, steps <= kWhole || steps > d.max_steps || d.nocut, x0, x1);
+      if (r.nst < 0) continue;
+      last = share_of(ltotal, lnsh, off0 + ovh(RT) / 2 + steps - 1);
     }
+    st0 = r.st0, nst = r.nst;
+    slot = r.part ? part_slot(wg, h, r.part) : -1;
+    if (r.part != 1 && t == 0 && h == 0) d.meta[b] = r.part ? make_int2(wg, last) : make_int2(0, 0);
   } else {
     const int S = d.splits, wg = blockIdx.x >> 1, s = wg % S;
     if (__builtin_amdgcn_readfirstlane(li)) return;
@@ -644,7 +631,7 @@ __global__ __launch_bounds__(WPR == 4 ? 256 : 1024) void decode_combine_kernel(D
     const int2 w = d.meta[b];
     n = w.y - w.x + 1;
     if (n <= 1) return;  // written by the split kernel
-    g0 = 2 * (2 * w.x + h), gstep = 4, first = 1;
+    g0 = part_slot(w.x, h, 1), gstep = part_slot(1, 0, 1), first = part_slot(0, 0, 2);
   }
   auto slot = [&](int p) { return (size_t)(g0 + p * gstep + (p == 0 ? first : 0)); };
   float M = -1e30f;  // the pieces' maxima are finite (-1e30 for one with no visible key)
@@ -741,7 +728,7 @@ extern "C" int q36_attn_decode(const q36_decode_args* a, q36_stream_t stream) {
               "q36_attn_decode: gate must be 8-byte, oq and oqs 4-byte aligned");
   const bool one = a->NT <= 2;  // one row tile, two workgroups a CU
   const int cus = decode_cus(), resident = (one ? kDecWPE1 : 1) * cus;
-  const int max_steps = (a->pt_stride - 1) / kST + 1;
+  const int max_steps = table_steps(a->pt_stride);
   // Dealing costs about 3 us and a combine 5; where no length the table can hold makes that good, the
   // splits are fixed: whole requests up to kAlone steps, and a few splits of at most kEven steps, in the
   // two-row-tile form of kEven steps together (more splits gain from the dealing even at equal lengths).
@@ -773,9 +760,8 @@ extern "C" int q36_attn_decode(const q36_decode_args* a, q36_stream_t stream) {
   const int slots = bal ? 2 * cus : a->B * kKVH * S;  // of kDRows rows
   // balanced: as many workgroups per KV head as the chip holds at once, and no more than pieces of a
   // table of this width; a table so narrow that no request is cut needs no combine
-  const int nocut = max_steps <= kMinPiece;
-  const int64_t pieces = (int64_t)a->B * ((max_steps - 1) / kMinPiece + 1);
-  const int shares = (int)std::min<int64_t>(std::max(1, resident / kKVH), pieces);
+  const int nocut = table_uncut(max_steps);
+  const int shares = deal_groups(a->B, max_steps, resident / kKVH);
   DecodeDev d{a->B, a->NT, a->pt_stride, S, nocut, max_steps,
               static_cast<const uint16_t*>(a->q), static_cast<const uint8_t*>(a->k_cache),
               static_cast<const uint8_t*>(a->v_cache), (int64_t)a->num_slots * kKVH * kDD, a->page_table, a->seqlens,

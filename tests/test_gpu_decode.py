@@ -263,3 +263,67 @@ def test_decode_balanced_empty_requests(attn, oracle_mod, dev):
     assert not got[[1, 3]].any()
     keep = [0, 2, 4, 5]
     assert_bf16_close(got[keep].reshape(-1, D), ref[keep].reshape(-1, D), 1e-2, "beside empty requests")
+
+
+def _widen(h, width, fill=0):
+    """The same batch with an engine-wide page table: columns past a request's keys are never read for them."""
+    pt = torch.full((h["pt"].shape[0], width), fill, dtype=torch.int32)
+    pt[:, :h["pt"].shape[1]] = h["pt"]
+    return dict(h, pt=pt)
+
+
+@pytest.mark.parametrize("width", [4096, 32768])
+@pytest.mark.parametrize("NT,seqlens", [
+    (1, [300]), (1, [1000]), (1, [3000]), (1, [3800, 3800]), (1, [600, 1700, 900, 1400]), (1, [680] * 8),
+    (1, _ragged(14, 264, 500, [], 8)), (2, [1000, 3500]), (3, [700, 64, 900]), (4, [1000]), (4, [3500]), (4, [1450, 1200]),
+    (4, _ragged(5, 264, 700, [], 9)), (1, _ragged(90, 100, 300, [], 10)), (3, _ragged(200, 3, 300, [900], 11)),
+    (1, _ragged(300, 1, 200, [4000], 12)),
+], ids=lambda v: f"{len(v)}x{max(v)}" if isinstance(v, list) else str(v))
+def test_decode_table_wider_than_the_requests(attn, oracle_mod, dev, NT, seqlens, width):
+    """The page table as wide as an engine's, whatever the lengths: against the oracle, with a workspace that holds
+    NaN everywhere and one that holds another call's partials.  Only what the call itself wrote may count."""
+    B = len(seqlens)
+    print(f"attn_decode wide table NT={NT} B={B} longest {max(seqlens)} width {width}", flush=True)
+    h = _widen(_make(B, NT, seqlens, seed=11 * NT + B), width)
+    ref = _oracle(oracle_mod, h, NT)
+    other = _make(B, NT, [4000 - 50 * (i % 8) for i in range(B)] if B < 20 else [n + 200 for n in seqlens], seed=3, qscale=4.0)
+    ws = attn.DecodeWorkspace(B, dev)
+    outs = []
+    for prefill in ("nan", "partials"):
+        if prefill == "nan":
+            ws.buf.fill_(0xFF)
+        else:
+            d = {k: other[k].to(dev) for k in ("q", "kc", "vc", "pt", "seqlens")}
+            attn.attn_decode(d["q"], d["kc"], d["vc"], d["pt"], d["seqlens"], NT, SCALE, ws)
+        d = {k: h[k].to(dev) for k in ("q", "kc", "vc", "pt", "seqlens")}
+        outs.append(attn.attn_decode(d["q"], d["kc"], d["vc"], d["pt"], d["seqlens"], NT, SCALE, ws))
+        _check(outs[-1], ref, f"wide table, workspace of {prefill}")
+    assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("NT", [1, 4])
+def test_decode_graph_follows_the_lengths(attn, oracle_mod, dev, NT):
+    """One captured launch over an engine-wide table, replayed with the lengths changed between the replays:
+    each replay gives the bits of an eager call with a workspace of NaN, and the oracle's values."""
+    print(f"attn_decode graph, lengths changed, NT={NT}", flush=True)
+    h = _widen(_make(3, NT, [3000, 700, 1800], seed=51 + NT), 32768)
+    d = {k: h[k].to(dev) for k in ("q", "kc", "vc", "pt", "seqlens")}
+    ws, fresh, out = attn.DecodeWorkspace(3, dev), attn.DecodeWorkspace(3, dev), torch.empty_like(d["q"])
+
+    def call(w, o):
+        return attn.attn_decode(d["q"], d["kc"], d["vc"], d["pt"], d["seqlens"], NT, SCALE, w, out=o)
+
+    call(ws, out)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        call(ws, out)
+    for lens in ([3000, 700, 1800], [300, 40, 270], [NT, 600, 33], [1000, 700, 1000], [2999, NT, 4], [400, 400, 400]):
+        print(f"replay {lens}", flush=True)
+        d["seqlens"].copy_(torch.tensor(lens, dtype=torch.int32))
+        out.view(torch.int16).fill_(0x5A5A)
+        g.replay()
+        torch.cuda.synchronize()
+        fresh.buf.fill_(0xFF)
+        assert torch.equal(call(fresh, None), out)
+        _check(out, _oracle(oracle_mod, dict(h, seqlens=torch.tensor(lens, dtype=torch.int32)), NT), f"replay {lens}")
