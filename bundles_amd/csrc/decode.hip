@@ -63,7 +63,8 @@ typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 struct DecodeDev {
   int B, NT, pt_stride;
   int splits;               // > 0: every request in this many equal splits; 0: balanced (see decode_split)
-  int nocut;                // balanced: no request is cut (the launch is followed by no combine)
+  int groups, per;          // balanced: workgroups of a KV head the keys are dealt to, and these over B
+  int even;                 // balanced: the pieces of every request where the lengths allow it (0: none)
   int max_steps;            // steps the page table's width holds: the most a request weighs
   const uint16_t* q;        // bf16 [B*NT, 16, 256]
   const uint8_t* kc;        // e4m3 [slots, 2, 256]
@@ -137,6 +138,7 @@ __global__ __launch_bounds__(256) void kv_scatter_kernel(const uint8_t* k8, cons
 
 // How one call's keys are dealt to the workgroups of a KV head (G of them fit on the chip at once), in
 // steps of kST keys (the arithmetic is q36_deal.h's):
+//   even    batches of short or equal requests: every request whole, or in the same few pieces, one a workgroup;
 //   pieces  each request in ceil(steps / c) equal pieces, one piece a workgroup, with the smallest c (from
 //           kMinPiece up) that needs no more than G pieces.  The one-row-tile form, of which two workgroups
 //           fit a CU, takes no more than G / 2: one a CU reads as fast, and longer runs leave fewer
@@ -146,20 +148,21 @@ __global__ __launch_bounds__(256) void kv_scatter_kernel(const uint8_t* k8, cons
 //   line    where there are more requests than G, or a few long ones among many would make that c much
 //           more than an equal share: a request weighs its steps plus ovh (what starting and merging a
 //           run costs beside its steps), half before and half after them, and the line of all
-//           weights is cut into G equal shares (as many as positions if these are fewer).  A share holds the end of one request, whole requests
-//           and the start of another; requests of at most kWhole steps are not cut but belong to the
-//           share that holds their start.
-// Every workgroup works the dealing out for itself from seqlens (about 1 us, before its first key), so a
-// captured launch follows the lengths it finds.  With a fixed number of splits per request, as before,
-// the longest request sets a call's time.  Measured, us a call (fixed -> dealt): 64 x 4 rows over 128 ..
-// 8192 keys 86.9 -> 47.9, 256 x 1 over 20 .. 4000 107.8 -> 58.0, 150 x 4 over 300 .. 6000 134 -> 83.9, 12 x 2
-// over 3000 .. 30000 60.1 -> 39.9.  Equal lengths gain nothing and pay for the dealing and for a combine that
-// may find nothing cut: 64 x 4 over 4096 64.5 -> 64.8, 256 x 1 over 4000 177 -> 182, 26 x 2 over 7656 48.8 ->
-// 53.3 (short tables keep fixed splits: see q36_attn_decode).
+//           weights is cut into G equal shares (as many as positions if these are fewer).  A share
+//           holds the end of one request, whole requests and the start of another; requests of at most kWhole
+//           steps are not cut but belong to the share that holds their start.
+// Every workgroup works the dealing out for itself from seqlens before its first key, so a captured launch follows the
+// lengths it finds.  That takes 0.5 us more than one load where it is even, 2 to 3 us else, and the combine launch
+// 1.5 to 2.5 us where it finds nothing cut; a call whose page table holds no long request is spared both (see
+// q36_attn_decode).  Measured, us a call (a fixed number of splits per request -> dealt): 64 x 4 rows over 128 .. 8192
+// keys 85.4 -> 45.4, 256 x 1 over 20 .. 4000 96 -> 51, 150 x 4 over 300 .. 6000 130 -> 87, 12 x 2 over 3000 ..
+// 30000 53.7 -> 36.6, 1 x 1 over 1000 42.9 -> 11.0.  Equal lengths have only that to lose: 64 x 4 over 4096 60.1 ->
+// 62.3, 256 x 1 over 4096 181.6 -> 184.1; so have short ones in a table of 32768 entries: 84 x 1 over 191 8.9 -> 11.1,
+// 56 x 1 over 646 14.8 -> 16.0, 117 x 3 over 131 .. 187 16.1 -> 16.4, 300 x 1 over 100 .. 300 20.9 -> 23.3, 1000 x 1 over 50 .. 300
+// 48.6 -> 54.9 (by pieces and line as the others: 18.0, 18.5, 19.0, 32.0 and 60.0).
 // ovh: 4 / 12 / 20 / 28 steps gave 58.5 / 52.2 / 49.3 / 50.3 us on the first of these (two row tiles) and
 // 56.5 / 57.2 / 63.7 / 70.7 on the second (one).  kMinPiece: 2 / 4 / 8 steps 25.0 / 22.5 / 22.9 us for one
 // request of 4 rows over 8000 keys, 14.0 / 14.6 / 16.0 us for one of 1 row over 1000.
-constexpr int kAlone = 12, kEven = 40;  // fixed splits: steps (see q36_attn_decode)
 // Integer sum over the wave, and inclusive scan, without LDS (the plan runs before the first load of a key).
 __device__ __forceinline__ int wave_sum_i(int v) {
   v += (int)dpp_u32<0xB1>((uint32_t)v);
@@ -170,6 +173,22 @@ __device__ __forceinline__ int wave_sum_i(int v) {
   v = (int)(p16[0] + p16[1]);
   const auto p32 = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false);
   return (int)(p32[0] + p32[1]);
+}
+__device__ __forceinline__ int wave_rows_sum_i(int v) {  // over the wave's four rows of 16 lanes
+  const auto p16 = __builtin_amdgcn_permlane16_swap((uint32_t)v, (uint32_t)v, false, false);
+  v = (int)(p16[0] + p16[1]);
+  const auto p32 = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false);
+  return (int)(p32[0] + p32[1]);
+}
+__device__ __forceinline__ int wave_max_i(int v) {
+  v = max(v, (int)dpp_u32<0xB1>((uint32_t)v));
+  v = max(v, (int)dpp_u32<0x4E>((uint32_t)v));
+  v = max(v, (int)dpp_u32<0x141>((uint32_t)v));
+  v = max(v, (int)dpp_u32<0x140>((uint32_t)v));
+  const auto p16 = __builtin_amdgcn_permlane16_swap((uint32_t)v, (uint32_t)v, false, false);
+  v = max((int)p16[0], (int)p16[1]);
+  const auto p32 = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false);
+  return max((int)p32[0], (int)p32[1]);
 }
 __device__ __forceinline__ int wave_scan_i(int v) {
   v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr 1, 2, 4, 8: within rows of 16
@@ -204,80 +223,137 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
   __shared__ float mw[4][kRows], lwv[4][kRows], rowM[kRows], rowL[kRows];
   // balanced: offset and key count of each of 256 requests, the waves' sums, and the loop's state (in LDS,
   // so that no register holds it across a run): the share, the next request, the chunk of requests
-  __shared__ int roff[256], rkeys[256], rsum[4], npiece[16];
-  __shared__ int lx0, lx1, ltotal, lnsh, lpc, li, lhi, lc0, lbase;
+  __shared__ int roff[256], rkeys[256], rsum[4], rmax[4], npiece[64];
+  __shared__ int lx0, lx1, li, lhi, lc0, lbase;
   const int h = blockIdx.x & 1;
-  {
-    const int t = run_tid();
-    if (d.splits == 0) {
-      const int wg = blockIdx.x >> 1, G = gridDim.x >> 1;
-      const int rk = t < d.B ? d.seqlens[t] : 0, st = min(req_steps(rk), d.max_steps);
-      int w = st;
-      for (int q = t + 256; q < d.B; q += 256) w += min(req_steps(d.seqlens[q]), d.max_steps);
-      w = wave_sum_i(w);
-      if ((t & 63) == 0) rsum[t >> 6] = w;
-      roff[t] = st;
-      rkeys[t] = rk;
-      __syncthreads();
-      const int steps = rsum[0] + rsum[1] + rsum[2] + rsum[3], total = steps + d.B * ovh(RT);
-      const int Gp = piece_places(RT, d.B, G, steps), c0 = piece_least(steps, Gp);
-      int pc = 0;
-      if (d.B <= min(Gp, 256)) {
-        // the kSizes piece sizes, four a wave
+  // The run's request and key count; of a call dealt in pieces also the request's pieces and which of them (pn 0: not)
+  int b = 0, nk = 0, pn = 0, pp = 0;
+  if (d.splits == 0) {
+    const int t = run_tid(), lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), wg = blockIdx.x >> 1, G = d.groups;
+    // Up to 256 requests every wave reads all lengths (request 64 j + lane), so that a call dealt evenly is dealt with no
+    // exchange between waves.
+    int len[4] = {0, 0, 0, 0}, steps = 0, longest = 0;
+    const bool few = d.B <= 256;
+    if (few) {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const int kk = 4 * (t >> 6) + k, c = piece_size(c0, kk);
-          int n = 0;
-          for (int q = t & 63; q < d.B; q += 64) n += req_pieces(roff[q], c);
-          n = wave_sum_i(n);
-          if ((t & 63) == 0) npiece[kk] = n;
-        }
-        __syncthreads();
-        const int n = npiece[t & 15];
-        const uint64_t fits = __builtin_amdgcn_ballot_w64(n <= Gp) & 0xffffu;
-        const int k = fits ? __builtin_ctzll(fits) : 0, c = piece_size(c0, k), nk = __builtin_amdgcn_readlane(n, k);
-        if (pieces_taken(RT, nk, c, total, Gp)) {
-          if (wg >= nk) return;
-          pc = c;
-        }
+      for (int j = 0; j < 4; ++j) len[j] = d.seqlens[min(64 * j + lane, d.B - 1)];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (64 * j + lane >= d.B) len[j] = 0;
+        const int v = min(req_steps(len[j]), d.max_steps);
+        steps += v, longest = max(longest, v);
       }
-      const int nsh = line_shares(total, G);
-      if (!pc && wg >= nsh) return;
-      if (t == 0) {
-        lpc = pc;
-        if (pc) lx0 = wg, lx1 = wg + 1;
-        else lx0 = share_begin(total, nsh, wg), lx1 = share_begin(total, nsh, wg + 1), ltotal = total, lnsh = nsh;
+    } else {
+#pragma unroll 4
+      for (int q = t; q < d.B; q += 256) {
+        const int v = min(req_steps(d.seqlens[q]), d.max_steps);
+        steps += v, longest = max(longest, v);
       }
     }
-    if (t == 0) li = 0, lhi = 0, lc0 = -256, lbase = 0;
-    __syncthreads();
+    steps = wave_sum_i(steps), longest = wave_max_i(longest);
+    if (!few) {
+      if (lane == 0) rsum[wv] = steps, rmax[wv] = longest;
+      __syncthreads();
+      steps = rsum[0] + rsum[1] + rsum[2] + rsum[3], longest = max(max(rmax[0], rmax[1]), max(rmax[2], rmax[3]));
+    }
+    steps = __builtin_amdgcn_readfirstlane(steps), longest = __builtin_amdgcn_readfirstlane(longest);
+    pn = even_pieces(RT, d.B, G, d.per, d.even, steps, longest);
+    if (pn) {
+      if (wg >= d.B * pn) return;
+      b = pn == 1 ? wg : wg / pn, pp = wg - b * pn;
+      nk = few ? __builtin_amdgcn_readlane(b < 64 ? len[0] : b < 128 ? len[1] : b < 192 ? len[2] : len[3], b & 63)
+               : d.seqlens[b];
+    } else {
+      // (rolled loops: the plan's code is fetched cold on every launch, and longer code took longer)
+      const int total = steps + d.B * ovh(RT), Gp = piece_places(RT, d.B, G, steps);
+      if (few) {
+        const int rk = wv == 0 ? len[0] : wv == 1 ? len[1] : wv == 2 ? len[2] : len[3];
+        rkeys[t] = rk;
+        roff[t] = min(req_steps(rk), d.max_steps);
+      }
+      __syncthreads();
+      // (no search where the requests longer than the largest piece taken are too many already)
+      const int most = piece_most(RT, total, Gp);
+      int longs = 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        longs += __builtin_popcountll(__builtin_amdgcn_ballot_w64(min(req_steps(len[j]), d.max_steps) > most));
+      if (few && d.B + longs <= Gp) {
+        // the kSizes piece sizes at once: thread t adds up size t % 16's pieces of every 16th request
+        const int c0 = piece_least(steps, Gp), ct = piece_size(c0, t & (kSizes - 1));
+        int n = 0;
+#pragma unroll 2
+        for (int q = t / kSizes; q < d.B; q += 256 / kSizes) n += req_pieces(roff[q], ct);
+        n = wave_rows_sum_i(n);
+        if (lane < kSizes) npiece[wv * kSizes + lane] = n;
+        __syncthreads();
+        n = npiece[t & 15] + npiece[16 + (t & 15)] + npiece[32 + (t & 15)] + npiece[48 + (t & 15)];
+        const uint64_t fits = __builtin_amdgcn_ballot_w64(n <= Gp) & 0xffffu;
+        const int k = fits ? __builtin_ctzll(fits) : 0, c = piece_size(c0, k), np = __builtin_amdgcn_readlane(n, k);
+        if (np <= Gp && c <= most) {
+          if (wg >= np) return;
+          // the request that piece wg belongs to
+          int end = 0;
+#pragma unroll 1
+          for (int q = 0; end <= wg; q += 64) {
+            const int w = q + lane < d.B ? req_pieces(roff[q + lane], c) : 0;
+            const int e = end + wave_scan_i(w);
+            const uint64_t at = __builtin_amdgcn_ballot_w64(wg < e);
+            end = __builtin_amdgcn_readlane(e, 63);
+            if (at == 0) continue;
+            const int l = __builtin_ctzll(at);
+            b = q + l, pn = __builtin_amdgcn_readlane(w, l), nk = rkeys[b];
+            pp = wg - __builtin_amdgcn_readlane(e, l) + pn;
+          }
+        }
+      }
+      if (!pn) {
+        const int nsh = line_shares(total, G);
+        if (wg >= nsh) return;
+        const int x0 = share_begin(total, nsh, wg), x1 = share_begin(total, nsh, wg + 1);
+        if (t == 0) lx0 = x0, lx1 = x1, li = 0, lhi = 0, lc0 = -256, lbase = 0;
+        __syncthreads();
+      }
+    }
   }
-  for (;;) {
-  // the run of steps [st0, st0 + nst) of request b, its key count, and the slot of its partial result
-  // (-1: the whole request, written out here)
-  int b, nk, st0, nst, slot;
-  if (d.splits == 0) {
+  for (bool again = false;; again = true) {
+  // the run of steps [st0, st0 + nst) of request b, and the slot of its partial result (-1: the whole request, written
+  // out here)
+  int st0, nst, slot, part;
+  const int wg = (int)blockIdx.x >> 1;
+  if (pn) {
+    if (again) {  // only whole requests can be more than workgroups
+      b += gridDim.x >> 1;
+      if (pn > 1 || b >= d.B) return;
+      nk = d.seqlens[b];
+    }
+    const DealRun r = piece_run(req_steps(nk), pn, pp);
+    st0 = r.st0, nst = r.nst;
+    part = r.part;
+  } else if (d.splits == 0) {
     const int t = run_tid(), x0 = __builtin_amdgcn_readfirstlane(lx0), x1 = __builtin_amdgcn_readfirstlane(lx1);
-    const int pc = __builtin_amdgcn_readfirstlane(lpc);
     int i = __builtin_amdgcn_readfirstlane(li);
     if (i >= __builtin_amdgcn_readfirstlane(lhi)) {  // the next 256 requests
       const int c0 = __builtin_amdgcn_readfirstlane(lc0) + 256, base = __builtin_amdgcn_readfirstlane(lbase);
       if (c0 >= d.B || base >= x1) return;
       const bool in = c0 + t < d.B;
-      const int rk = c0 == 0 ? rkeys[t] : in ? d.seqlens[c0 + t] : 0, st = min(req_steps(rk), d.max_steps);
-      const int w = !in ? 0 : pc ? req_pieces(st, pc) : st + ovh(RT);
-      const int inc = wave_scan_i(w);
+      const int rk = d.B <= 256 ? rkeys[t] : in ? d.seqlens[c0 + t] : 0;
+      const int w = in ? min(req_steps(rk), d.max_steps) + ovh(RT) : 0, inc = wave_scan_i(w), v = t >> 6;
       __syncthreads();  // the state above has been read
-      if ((t & 63) == 63) rsum[t >> 6] = inc;
+      if ((t & 63) == 63) rsum[v] = inc;
       __syncthreads();
-      int off = base + inc - w;
-#pragma unroll
-      for (int v = 0; v < 3; ++v) off += v < (t >> 6) ? rsum[v] : 0;
+      const int off = base + inc - w + (v > 0 ? rsum[0] : 0) + (v > 1 ? rsum[1] : 0) + (v > 2 ? rsum[2] : 0);
       roff[t] = off;
       rkeys[t] = rk;
       // the requests of the chunk that touch the share
-      const int lo = __syncthreads_count(in && off + w <= x0), hi = __syncthreads_count(in && off < x1);
-      if (t == 0) li = lo, lhi = hi, lc0 = c0, lbase = base + rsum[0] + rsum[1] + rsum[2] + rsum[3];
+      const int lo = __builtin_popcountll(__builtin_amdgcn_ballot_w64(in && off + w <= x0));
+      const int hi = __builtin_popcountll(__builtin_amdgcn_ballot_w64(in && off < x1));
+      if ((t & 63) == 0) npiece[v] = lo, npiece[4 + v] = hi;
+      __syncthreads();
+      if (t == 0) {
+        li = npiece[0] + npiece[1] + npiece[2] + npiece[3], lhi = npiece[4] + npiece[5] + npiece[6] + npiece[7];
+        lc0 = c0, lbase = base + rsum[0] + rsum[1] + rsum[2] + rsum[3];
+      }
       __syncthreads();
       continue;
     }
@@ -288,33 +364,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
     __syncthreads();
     if (t == 0) li = i + 1;
     __syncthreads();
-    const int wg = (int)blockIdx.x >> 1;
-    DealRun r;
-    int last;  // of the workgroups that hold a piece of the request, this one being the first
-    if (pc) {
-      const int n = req_pieces(min(steps, d.max_steps), pc), p = x0 - off0;
-      r = piece_run(steps, n, p);
-      last = wg + n - 1;
-    } else {
-      // (a key count past the page table's width is not cut either: its weight is the table's)
-      r = line_run(steps, off0, ovh(RT) / 2, steps <= kWhole || steps > d.max_steps || d.nocut, x0, x1);
-      if (r.nst < 0) continue;
-      last = share_of(ltotal, lnsh, off0 + ovh(RT) / 2 + steps - 1);
-    }
+    // (a key count past the page table's width is not cut either: its weight is the table's)
+    const DealRun r = line_run(steps, off0, ovh(RT) / 2, steps <= kWhole || steps > d.max_steps, x0, x1);
+    if (r.nst < 0) continue;
     st0 = r.st0, nst = r.nst;
-    slot = r.part ? part_slot(wg, h, r.part) : -1;
-    if (r.part != 1 && t == 0 && h == 0) d.meta[b] = r.part ? make_int2(wg, last) : make_int2(0, 0);
+    part = r.part;
   } else {
-    const int S = d.splits, wg = blockIdx.x >> 1, s = wg % S;
-    if (__builtin_amdgcn_readfirstlane(li)) return;
-    __syncthreads();
-    if (threadIdx.x == 0) li = 1;
-    b = wg / S;
+    if (again) return;
+    const int S = d.splits;
+    b = S == 1 ? wg : wg / S;
+    const int s = wg - b * S;
     nk = d.seqlens[b];
-    const int steps = req_steps(nk), per = steps / S, rem = steps % S;
-    st0 = s * per + min(s, rem);
-    nst = per + (s < rem ? 1 : 0);
+    const DealRun r = piece_run(req_steps(nk), S, s);
+    st0 = r.st0, nst = r.nst, part = 0;
     slot = S > 1 ? (b * kKVH + h) * S + s : -1;
+  }
+  // scalars: the descriptors made from them stay in SGPRs
+  b = __builtin_amdgcn_readfirstlane(b), nk = __builtin_amdgcn_readfirstlane(nk);
+  st0 = __builtin_amdgcn_readfirstlane(st0), nst = __builtin_amdgcn_readfirstlane(nst);
+  if (d.splits == 0) {
+    slot = part ? part_slot(wg, h, part) : -1;
+    if (threadIdx.x == 0 && h == 0) {  // the workgroups that hold the request's first and last piece
+      if (part == 0 || (part & kFirst)) d.meta[b].x = part ? wg : 0;
+      if (part == 0 || (part & kLast)) d.meta[b].y = part ? wg : 0;
+    }
   }
   const int tid = run_tid(), lane = tid & 63, l16 = lane & 15, lg = lane >> 4, NT = d.NT;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: LDS bases stay scalar
@@ -329,7 +402,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
   const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(
       (void*)(d.pt + (size_t)b * d.pt_stride), (short)0, 4 * d.pt_stride, 0x00020000);
   int32_t* ring = &ptl[wave][0][0];
-  // Page-table entries of step j into ring entry j % 8 (lanes 32..63 repeat lanes 0..31).  Keys past
+  // Page-table entries of step j into ring entry j % kPTR (lanes 32..63 repeat lanes 0..31).  Keys past
   // the wave's range take the slot of its last key: their loads are repeats that stay in L2, their
   // scores are masked and their values are real cache rows (finite), so 0 * V stays 0.
   auto pt_dma = [&](int j) {
@@ -609,68 +682,131 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
   }
 }
 
-// out = bf16(sum_p exp2(m_p - M) o_p / L), L = sum_p exp2(m_p - M) l_p over the pieces of a request.
-// WPR waves per query row (b, t, head), each lane 4 dims: wave v adds pieces v, v + WPR, ... with four
-// loads in flight, and the waves' sums meet in LDS in wave order.  Latency-bound: one wave a row where a
-// request has a few pieces; 4 or 16 where a call of few requests has them in tens (3 requests of 42
-// splits: 23.3 us for one thread per 4 dims walking the splits, 5.5 us for 16 waves).  kRows: rows of a slot.
-template <int WPR>
-__global__ __launch_bounds__(WPR == 4 ? 256 : 1024) void decode_combine_kernel(DecodeDev d, int kRows) {
-  constexpr int RPB = WPR > 1 ? 1 : 16;  // rows a workgroup (one token's)
-  __shared__ v4f sums[WPR > 1 ? WPR : 1][64];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, c = lane;
-  const int qr = blockIdx.x * RPB + (WPR > 1 ? 0 : wave), wv = WPR > 1 ? wave : 0;  // qr = (b * NT + t) * 16 + head
-  const int NT = d.NT, head = qr % kQH, bt = qr / kQH, t = bt % NT, b = bt / NT;
-  if (b >= d.B) return;
-  const int h = head / kGQ, gr = t * kGQ + head % kGQ;
-  int n, g0, gstep;  // piece p of the request is at slot g0 + p * gstep, the first at g0 + first
-  int first = 0;
-  if (d.splits > 0) {
-    n = d.splits, g0 = (b * kKVH + h) * n, gstep = 1;
-  } else {
-    const int2 w = d.meta[b];
-    n = w.y - w.x + 1;
-    if (n <= 1) return;  // written by the split kernel
-    g0 = part_slot(w.x, h, 1), gstep = part_slot(1, 0, 1), first = part_slot(0, 0, 2);
+// out = bf16(sum_p exp2(m_p - M) o_p / L), L = sum_p exp2(m_p - M) l_p over the pieces of a request, for each query row
+// (b, t, head).  Latency-bound (the request's pieces, then their maxima, sums and outputs at once): a request of a few
+// pieces takes one pass by one wave (decode_combine_few); 4 or 16 waves a row where a call of few requests has
+// them in tens (3 requests of 42 splits: 23.3 us for one thread per 4 dims walking the splits, 5.5 us for 16
+// waves).  kRows: rows of a slot.
+struct Pieces {
+  int n, g0, gstep, first;  // piece p of the request is at slot g0 + p * gstep, the first at g0 + first
+  __device__ __forceinline__ int at(int p) const { return p * gstep + (p == 0 ? first : 0); }
+};
+__device__ __forceinline__ Pieces req_parts(const DecodeDev& d, int b, int h) {
+  if (d.splits > 0) return Pieces{d.splits, (b * kKVH + h) * d.splits, 1, 0};
+  const int2 w = d.meta[b];
+  return Pieces{w.y - w.x + 1, part_slot(w.x, h, 0), part_slot(1, 0, 0), part_slot(0, 0, kFirst)};
+}
+__device__ __forceinline__ void put_row(const DecodeDev& d, int bt, int head, int c, v4f a, float L) {
+  const float il = L > 0.f ? 1.f / L : 0.f;
+  const uint32_t o01 = pack_bf2_hw(a[0] * il, a[1] * il), o23 = pack_bf2_hw(a[2] * il, a[3] * il);
+  *reinterpret_cast<uint2*>(d.out + ((size_t)bt * kQH + head) * kDD + 4 * c) = make_uint2(o01, o23);
+  // the wave holds the row: lanes 0-31 / 32-63 its two 128-groups
+  if (d.oq) gated_e4m3(d, bt, head, c, o01, o23);
+}
+
+// A workgroup a token, each of its 4 waves 4 query rows, each lane 4 dims of them.  Up to kNF pieces are in flight at
+// once, read through descriptors of the request's slots (a piece past the last reads zeros and costs no traffic);
+// more go in rounds, the sums rescaled to the new maximum.  Where nothing was cut the launch is pure overhead, so
+// it is kept small: a wave a row took 0.3 us more for 84 tokens and 1.5 us more for 1000.
+constexpr int kNF = 4;
+__global__ __launch_bounds__(256) void decode_combine_few_kernel(DecodeDev d, int kRows) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = threadIdx.x & 63;
+  const int bt = blockIdx.x, t = bt % d.NT, b = bt / d.NT, head = 4 * wave, h = head / kGQ, gr = t * kGQ + head % kGQ;
+  const Pieces P = req_parts(d, b, h);
+  if (d.splits == 0 && P.n <= 1) return;  // written by the split kernel
+  const int span = (P.at(P.n - 1) + P.first + 1) * kRows;
+  const __amdgpu_buffer_rsrc_t ors = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(d.ws_o + (size_t)P.g0 * kRows * kDD), (short)0, span * (kDD * 4), 0x00020000);
+  const __amdgpu_buffer_rsrc_t mrs = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(d.ws_ml + (size_t)P.g0 * 2 * kRows), (short)0, span * (2 * 4), 0x00020000);
+  v4f a[4] = {}, M = {-1e30f, -1e30f, -1e30f, -1e30f}, L = {};  // the pieces' maxima are finite (-1e30: no visible key)
+  for (int p0 = 0; p0 < P.n; p0 += kNF) {
+    v4f m[kNF], l[kNF], o[kNF][4];
+#pragma unroll
+    for (int k = 0; k < kNF; ++k) {
+      const bool in = p0 + k < P.n;
+      const int row = P.at(p0 + k) * kRows, past = 0x7fffff00;
+      const int mo = in ? (2 * row + gr) * 4 : past, oo = in ? (row + gr) * (kDD * 4) + 16 * c : past;
+      m[k] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(mrs, mo, 0, 0));
+      l[k] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(mrs, mo, kRows * 4, 0));
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        o[k][i] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(ors, oo, i * kDD * 4, 0));
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float mk[kNF], mx = M[i];
+#pragma unroll
+      for (int k = 0; k < kNF; ++k) {
+        mk[k] = p0 + k < P.n ? m[k][i] : -1e30f;
+        mx = fmaxf(mx, mk[k]);
+      }
+      if (p0) {
+        const float s = __builtin_amdgcn_exp2f(M[i] - mx);
+        L[i] *= s;
+        a[i] *= s;
+      }
+      M[i] = mx;
+#pragma unroll
+      for (int k = 0; k < kNF; ++k) {
+        const float w = __builtin_amdgcn_exp2f(mk[k] - mx);
+        L[i] += w * l[k][i];
+        a[i] += w * o[k][i];
+      }
+    }
   }
-  auto slot = [&](int p) { return (size_t)(g0 + p * gstep + (p == 0 ? first : 0)); };
-  float M = -1e30f;  // the pieces' maxima are finite (-1e30 for one with no visible key)
-  for (int p = lane; p < n; p += 64) M = fmaxf(M, d.ws_ml[slot(p) * 2 * kRows + gr]);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) put_row(d, bt, head + i, c, a[i], L[i]);
+}
+
+// A workgroup a row: wave v adds pieces v, v + WPR, ..., each lane 4 dims, four in flight, and the waves' sums meet in LDS
+// in wave order.
+template <int WPR>
+__global__ __launch_bounds__(64 * WPR) void decode_combine_kernel(DecodeDev d, int kRows) {
+  __shared__ v4f sums[WPR][64];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, c = lane;
+  const int head = blockIdx.x % kQH, bt = blockIdx.x / kQH, t = bt % d.NT, b = bt / d.NT;
+  const int h = head / kGQ, gr = t * kGQ + head % kGQ;
+  const Pieces P = req_parts(d, b, h);
+  const int n = P.n;
+  if (d.splits == 0 && n <= 1) return;  // written by the split kernel
+  auto slot = [&](int p) { return (size_t)(P.g0 + P.at(p)); };
+  v4f o[4];
+  auto fetch = [&](int p0, int q0, int m) {  // pieces p0 + q0, p0 + q0 + WPR, .. (past the m-th: the last again)
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      o[k] = *reinterpret_cast<const v4f*>(d.ws_o + (slot(p0 + min(q0 + k * WPR, m - 1)) * kRows + gr) * kDD + 4 * c);
+  };
+  auto ml = [&](int p, int what) { return d.ws_ml[(slot(p) * 2 + what) * kRows + gr]; };
+  float mp = ml(min(lane, n - 1), 0), lp = ml(min(lane, n - 1), 1);
+  fetch(0, wave, min(64, n));
+  float M = mp;
+  for (int p = lane + 64; p < n; p += 64) M = fmaxf(M, ml(p, 0));
   M = wave_max(M);
   float L = 0.f;
   v4f a = {0.f, 0.f, 0.f, 0.f};
   for (int p0 = 0; p0 < n; p0 += 64) {
-    const int pl = min(p0 + lane, n - 1);
-    const float w = p0 + lane < n ? exp2f(d.ws_ml[slot(pl) * 2 * kRows + gr] - M) : 0.f;
-    L += w * d.ws_ml[slot(pl) * 2 * kRows + kRows + gr];
+    if (p0) mp = ml(min(p0 + lane, n - 1), 0), lp = ml(min(p0 + lane, n - 1), 1);
+    const float w = p0 + lane < n ? exp2f(mp - M) : 0.f;
+    L += w * lp;
     const int m = min(64, n - p0);
-    for (int q0 = wv; q0 < m; q0 += 4 * WPR) {
-      v4f o[4];
-      float wq[4];
+    for (int q0 = wave; q0 < m; q0 += 4 * WPR) {
+      if (p0 + q0 != wave) fetch(p0, q0, m);
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         const int q = q0 + k * WPR, qc = min(q, m - 1);
-        o[k] = *reinterpret_cast<const v4f*>(d.ws_o + (slot(p0 + qc) * kRows + gr) * kDD + 4 * c);
         const float r = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), qc));
-        wq[k] = q < m ? r : 0.f;
+        a += (q < m ? r : 0.f) * o[k];
       }
-#pragma unroll
-      for (int k = 0; k < 4; ++k) a += wq[k] * o[k];
     }
   }
   L = wave_sum_bfly(L);
-  if constexpr (WPR > 1) {
-    sums[wave][lane] = a;
-    __syncthreads();
-    if (wave != 0) return;
+  sums[wave][lane] = a;
+  __syncthreads();
+  if (wave != 0) return;
 #pragma unroll
-    for (int v = 1; v < WPR; ++v) a += sums[v][lane];
-  }
-  const float il = L > 0.f ? 1.f / L : 0.f;
-  const uint32_t o01 = pack_bf2_hw(a[0] * il, a[1] * il), o23 = pack_bf2_hw(a[2] * il, a[3] * il);
-  *reinterpret_cast<uint2*>(d.out + (size_t)qr * kDD + 4 * c) = make_uint2(o01, o23);
-  // the wave holds the row: lanes 0-31 / 32-63 its two 128-groups
-  if (d.oq) gated_e4m3(d, bt, head, c, o01, o23);
+  for (int v = 1; v < WPR; ++v) a += sums[v][lane];
+  put_row(d, bt, head, c, a, L);
 }
 
 int decode_cus() {
@@ -729,15 +865,14 @@ extern "C" int q36_attn_decode(const q36_decode_args* a, q36_stream_t stream) {
   const bool one = a->NT <= 2;  // one row tile, two workgroups a CU
   const int cus = decode_cus(), resident = (one ? kDecWPE1 : 1) * cus;
   const int max_steps = table_steps(a->pt_stride);
-  // Dealing costs about 3 us and a combine 5; where no length the table can hold makes that good, the
-  // splits are fixed: whole requests up to kAlone steps, and a few splits of at most kEven steps, in the
-  // two-row-tile form of kEven steps together (more splits gain from the dealing even at equal lengths).
-  // Measured, us a call (dealt, fixed): 84 x 1 row over 191 keys 18.4, 9.5; 56 x 1 over 646 21.7, 15.2; 101 x 2
-  // over 250 .. 877 26.0, 21.7; 39 x 1 over 1101 22.1, 17.5; 117 x 3 over 131 .. 187 19.4, 16.7; 44 x 3 over 644 .. 879 25.8, 22.2; on the other
-  // side 95 x 2 over 750 .. 2445 43.0, 48.6; 46 x 4 over 650 .. 3800 37.2, 49.1.
+  // Where no length the table can hold makes the dealing good, the splits are fixed here, by the rule that the kernel
+  // applies to the lengths, and neither the dealing nor a combine that may find nothing cut is paid for.  Measured, us
+  // a call (dealt, fixed): 84 x 1 row over 191 keys 11.1, 9.0; 56 x 1 over 646 16.0, 15.3; 117 x 3 over 131 .. 187 16.4, 14.2;
+  // on the other side 95 x 2 over 750 .. 2445 43.0, 48.6; 46 x 4 over 650 .. 3800 37.2, 49.1.
+  const int so = decode_splits(a->B, 0);
+  const int even = so <= (one ? 4 : 2) && (int64_t)a->B * kKVH * so <= resident ? so : 0;
   const auto fixed = [&] {
-    const int so = decode_splits(a->B, 0);
-    const int s = max_steps <= kAlone ? 1 : so <= (one ? 4 : 2) && max_steps <= kEven * (one ? so : 1) ? so : 0;
+    const int s = even_table(one ? 1 : 2, even, max_steps);
     return (int64_t)a->B * kKVH * s <= resident && a->workspace_bytes >= decode_ws_bytes(a->B, std::max(s, 1)) ? s : 0;
   };
   const int s0 = a->splits > 0 ? a->splits : fixed();
@@ -759,10 +894,10 @@ extern "C" int q36_attn_decode(const q36_decode_args* a, q36_stream_t stream) {
                                                             static_cast<uint8_t*>(a->v_cache));
   const int slots = bal ? 2 * cus : a->B * kKVH * S;  // of kDRows rows
   // balanced: as many workgroups per KV head as the chip holds at once, and no more than pieces of a
-  // table of this width; a table so narrow that no request is cut needs no combine
+  // table of this width; a table so narrow that every request is dealt whole needs no combine
   const int nocut = table_uncut(max_steps);
   const int shares = deal_groups(a->B, max_steps, resident / kKVH);
-  DecodeDev d{a->B, a->NT, a->pt_stride, S, nocut, max_steps,
+  DecodeDev d{a->B, a->NT, a->pt_stride, S, shares, shares / a->B, even, max_steps,
               static_cast<const uint16_t*>(a->q), static_cast<const uint8_t*>(a->k_cache),
               static_cast<const uint8_t*>(a->v_cache), (int64_t)a->num_slots * kKVH * kDD, a->page_table, a->seqlens,
               a->scale * 1.44269504088896340736f, reinterpret_cast<float*>(ws),
@@ -780,10 +915,10 @@ extern "C" int q36_attn_decode(const q36_decode_args* a, q36_stream_t stream) {
     const int rows = T * kQH, slot_rows = one ? 16 : kDRows, per = bal ? shares / a->B : S;
     if (per >= 32)
       decode_combine_kernel<16><<<rows, 1024, 0, st>>>(d, slot_rows);
-    else if (per >= 4)
+    else if (per >= 3)
       decode_combine_kernel<4><<<rows, 256, 0, st>>>(d, slot_rows);
     else
-      decode_combine_kernel<1><<<T, 1024, 0, st>>>(d, slot_rows);
+      decode_combine_few_kernel<<<T, 256, 0, st>>>(d, slot_rows);
   }
   return check_launch("q36_attn_decode");
 }

@@ -451,8 +451,10 @@ int q36_add_rmsnorm(const q36_add_norm_args* a, q36_stream_t stream);
  * with gate bf16 [B*NT, HQ*D] (q36_attn_proj's gate output), oq receives the e4m3 codes row-major
  * [B*NT, HQ*D] of bf16(out * sigmoid(gate)) per 128-channel group and oqs fp32 [B*NT, HQ*D/128] the
  * group scales (amax / 448): q36_attn_oproj's aq / aqs.
- * splits: 0 = every request's keys dealt evenly over the chip's workgroups, whatever the lengths (worked
- * out on the device from seqlens; a few fixed splits where the page table is too short for that to pay); a positive count cuts each request into that many (at most 64).
+ * splits: 0 = every request's keys dealt over the chip's workgroups, worked out on the device from
+ * seqlens whatever the page table's width (equal pieces for short or equal requests, even shares for
+ * others; a few fixed splits where the table is too short for that to pay); a positive count cuts each
+ * request into that many (at most 64).
  * Constraints: HQ = 16, HKV = 2, D = 256, 1 <= NT <= 4,
  * num_slots * HKV * D < 2^31; q, caches 16-byte aligned. */
 typedef struct q36_decode_args {

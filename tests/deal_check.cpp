@@ -17,72 +17,81 @@ using namespace q36;
 
 // One KV head (h), one batch: the split kernel's steps per request and partial slots, then the combine's reads.
 static const char* walk(const std::vector<int>& len, int RT, int width, int cus, int h) {
+  // (the split count of the equal splits, as the host passes it on)
+  const int so = std::max(1, std::min(64, cus / (2 * (int)len.size())));
+  const int splits = so <= (RT == 1 ? 4 : 2) && (int)len.size() * 2 * so <= (RT == 1 ? 2 : 1) * cus ? so : 0;
   const int B = (int)len.size(), max_steps = table_steps(width), nocut = table_uncut(max_steps);
   const int G = deal_groups(B, max_steps, (RT == 1 ? 2 : 1) * cus / 2);
-  std::vector<int> st(B), first(B, -1), last(B, -1), whole(B, 0), metas(B, 0);
+  std::vector<int> st(B), first(B, -1), last(B, -1), whole(B, 0), firsts(B, 0), lasts(B, 0);
   std::vector<std::vector<int>> done(B);
-  int steps = 0;
+  int steps = 0, longest = 0;
   for (int b = 0; b < B; ++b) {
     st[b] = std::min(req_steps(len[b]), max_steps);
-    steps += st[b];
+    steps += st[b], longest = std::max(longest, st[b]);
     done[b].assign(req_steps(len[b]), 0);
   }
   const int total = steps + B * ovh(RT), Gp = piece_places(RT, B, G, steps), c0 = piece_least(steps, Gp);
-  int pc = 0, np = 0;
-  if (B <= std::min(Gp, 256)) {
-    int k = 0, n = 0, c = 0;
-    for (; k < kSizes; ++k) {
-      c = piece_size(c0, k), n = 0;
-      for (int b = 0; b < B; ++b) n += req_pieces(st[b], c);
-      if (n <= Gp) break;
+  const int even = even_pieces(RT, B, G, G / B, splits, steps, longest);
+  std::vector<int> pieces(B, even);  // of each request, where the call is dealt in pieces
+  int np = even * B;
+  if (!np && B <= std::min(Gp, 256)) {
+    for (int k = 0; k < kSizes; ++k) {
+      int n = 0;
+      for (int b = 0; b < B; ++b) n += pieces[b] = req_pieces(st[b], piece_size(c0, k));
+      if (n > Gp) continue;
+      if (piece_size(c0, k) <= piece_most(RT, total, Gp)) np = n;
+      // (the kernel does not search where this many requests are too long)
+      if (np && B + std::count_if(st.begin(), st.end(), [&](int v) { return v > piece_most(RT, total, Gp); }) > Gp)
+        return "pieces that fit are not searched for";
+      break;
     }
-    if (k < kSizes && pieces_taken(RT, n, c, total, Gp)) pc = c, np = n;
   }
   const int nsh = line_shares(total, G);
   const int slots = 4 * (RT == 1 ? cus : cus / 2);  // of 16 RT rows
   std::vector<int> owner(slots, -1);                // request that wrote the slot in this call
-  for (int w = 0; w < G; ++w) {
-    if (pc ? w >= np : w >= nsh) continue;
-    const int x0 = pc ? w : share_begin(total, nsh, w), x1 = pc ? w + 1 : share_begin(total, nsh, w + 1);
-    int off = 0;
-    for (int b = 0; b < B; ++b) {
-      const int wt = pc ? req_pieces(st[b], pc) : st[b] + ovh(RT), off0 = off, n_all = req_steps(len[b]);
-      off += wt;
-      if (off <= x0 || off0 >= x1) continue;
-      DealRun r;
-      int lst;
-      if (pc) {
-        r = piece_run(n_all, wt, x0 - off0);
-        lst = w + wt - 1;
-      } else {
-        r = line_run(n_all, off0, ovh(RT) / 2, n_all <= kWhole || n_all > max_steps || nocut, x0, x1);
-        if (r.nst < 0) continue;
-        lst = share_of(total, nsh, off0 + ovh(RT) / 2 + n_all - 1);
-      }
-      if (r.st0 < 0 || r.st0 + r.nst > n_all) return "a run outside its request";
-      for (int s = r.st0; s < r.st0 + r.nst; ++s) ++done[b][s];
-      if (r.part != 1) ++metas[b], first[b] = r.part ? w : 0, last[b] = r.part ? lst : 0;
-      if (r.part == 0) {
-        ++whole[b];
-      } else {
-        const int slot = part_slot(w, h, r.part);
-        if (slot < 0 || slot >= slots) return "a slot outside the workspace";
-        if (owner[slot] >= 0) return "a slot written twice";
-        owner[slot] = b;
+  const char* err = nullptr;
+  auto run = [&](int b, const DealRun& r, int w) {
+    if (r.st0 < 0 || r.st0 + r.nst > (int)done[b].size()) err = "a run outside its request";
+    for (int s = r.st0; !err && s < r.st0 + r.nst; ++s) ++done[b][s];
+    if (r.part == 0 || (r.part & kFirst)) first[b] = r.part ? w : 0, ++firsts[b];
+    if (r.part == 0 || (r.part & kLast)) last[b] = r.part ? w : 0, ++lasts[b];
+    if (r.part == 0) {
+      ++whole[b];
+      return;
+    }
+    const int slot = part_slot(w, h, r.part);
+    if (w >= G) err = "a piece past the workgroups";
+    else if (slot < 0 || slot >= slots) err = "a slot outside the workspace";
+    else if (owner[slot] >= 0) err = "a slot written twice";
+    else owner[slot] = b;
+  };
+  if (np) {
+    for (int b = 0, w = 0; b < B; ++b)
+      for (int p = 0; p < pieces[b]; ++p, ++w) run(b, piece_run(req_steps(len[b]), pieces[b], p), w);
+  } else {
+    for (int w = 0; w < nsh; ++w) {
+      const int x0 = share_begin(total, nsh, w), x1 = share_begin(total, nsh, w + 1);
+      for (int b = 0, off = 0; b < B; ++b) {
+        const int wt = st[b] + ovh(RT), off0 = off, n_all = req_steps(len[b]);
+        off += wt;
+        if (off <= x0 || off0 >= x1) continue;
+        const DealRun r = line_run(n_all, off0, ovh(RT) / 2, n_all <= kWhole || n_all > max_steps, x0, x1);
+        if (r.nst >= 0) run(b, r, w);
       }
     }
   }
+  if (err) return err;
   int used = 0;
   for (int b = 0; b < B; ++b) {
     for (int d : done[b])
       if (d != 1) return "a step not in exactly one run";
-    if (metas[b] != 1) return "a request whose pieces are not told to the combine once";
+    if (firsts[b] != 1 || lasts[b] != 1) return "a request whose pieces are not told to the combine once";
     const int n = last[b] - first[b] + 1;
     if ((n <= 1) != (whole[b] == 1) || whole[b] > 1) return "a request neither whole nor in pieces";
     if (n <= 1) continue;
     if (nocut) return "a cut request without a combine";
     for (int p = 0; p < n; ++p) {
-      const int slot = part_slot(first[b] + p, h, p == 0 ? 2 : 1);
+      const int slot = part_slot(first[b] + p, h, p == 0 ? kFirst : 0);
       if (slot >= slots || owner[slot] != b) return "the combine reads a slot that this call did not write";
       ++used;
     }

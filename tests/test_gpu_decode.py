@@ -237,7 +237,8 @@ def test_decode_balanced_shares(attn, oracle_mod, dev, NT, seqlens):
     (1, _ragged(50, 300, 900, [2560], 6)),               # two
     (3, _ragged(100, 3, 500, [1280], 7)),                # two row tiles, one split
     (1, [9000, 8000, 4]),                                # one row tile, pieces: one workgroup a CU
-], ids=["whole1", "whole4", "70", "50", "100", "3"])
+    (1, _ragged(300, 1, 384, [], 18)), (4, _ragged(150, 4, 384, [], 19)),  # 12 steps, more requests than workgroups
+], ids=["whole1", "whole4", "70", "50", "100", "3", "300", "150"])
 def test_decode_default_route(attn, oracle_mod, dev, NT, seqlens):
     """The default route by the table's width and the batch, against the oracle; requests without keys give zeros."""
     B = len(seqlens)
@@ -278,15 +279,22 @@ def _widen(h, width, fill=0):
     (1, _ragged(14, 264, 500, [], 8)), (2, [1000, 3500]), (3, [700, 64, 900]), (4, [1000]), (4, [3500]), (4, [1450, 1200]),
     (4, _ragged(5, 264, 700, [], 9)), (1, _ragged(90, 100, 300, [], 10)), (3, _ragged(200, 3, 300, [900], 11)),
     (1, _ragged(300, 1, 200, [4000], 12)),
+    # dealt evenly, by the lengths: whole requests, more of them than workgroups; two and three pieces each
+    # (some requests with fewer steps than pieces); equal lengths in as many as fit
+    (1, _ragged(300, 1, 384, [], 13)), (4, _ragged(150, 4, 380, [0], 14)), (1, _ragged(56, 300, 900, [2560, 1], 15)),
+    (2, _ragged(40, 33, 1200, [3800, 2], 16)), (3, _ragged(64, 3, 500, [1280], 17)), (4, [700] * 8), (1, [2000] * 30),
+    (2, [1500] * 5), (4, [4000] * 3),
 ], ids=lambda v: f"{len(v)}x{max(v)}" if isinstance(v, list) else str(v))
 def test_decode_table_wider_than_the_requests(attn, oracle_mod, dev, NT, seqlens, width):
     """The page table as wide as an engine's, whatever the lengths: against the oracle, with a workspace that holds
     NaN everywhere and one that holds another call's partials.  Only what the call itself wrote may count."""
     B = len(seqlens)
     print(f"attn_decode wide table NT={NT} B={B} longest {max(seqlens)} width {width}", flush=True)
-    h = _widen(_make(B, NT, seqlens, seed=11 * NT + B), width)
-    ref = _oracle(oracle_mod, h, NT)
-    other = _make(B, NT, [4000 - 50 * (i % 8) for i in range(B)] if B < 20 else [n + 200 for n in seqlens], seed=3, qscale=4.0)
+    h = _widen(_make(B, NT, [max(n, NT) for n in seqlens], seed=11 * NT + B), width)
+    ref = _oracle(oracle_mod, h, NT).reshape(B, NT, HQ, D)
+    h["seqlens"] = torch.tensor(seqlens, dtype=torch.int32)
+    ref[[i for i, n in enumerate(seqlens) if n == 0]] = 0  # no keys: zeros
+    other = _make(B, NT, [4000 - 50 * (i % 8) for i in range(B)] if B < 20 else [max(n, NT) + 200 for n in seqlens], seed=3, qscale=4.0)
     ws = attn.DecodeWorkspace(B, dev)
     outs = []
     for prefill in ("nan", "partials"):
