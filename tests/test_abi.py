@@ -66,6 +66,54 @@ def test_struct_layouts_match_header(tmp_path):
             assert got[(cname, fname)] == getattr(st, fname).offset, f"{cname}.{fname}"
 
 
+def _entries():
+    """(symbol, its argument structure) of every entry point that takes one."""
+    from bundles_amd import _lib
+    return [(n, a[0]._type_) for n, _, a in _lib.SYMBOLS if a and hasattr(a[0], "_type_") and
+            isinstance(a[0]._type_, type) and issubclass(a[0]._type_, C.Structure)]
+
+
+def test_entry_points_refuse_another_structure(L):
+    """Each entry takes its own argument structure; another one, raw bytes or a number never reach the library."""
+    from bundles_amd import _lib
+    entries = _entries()
+    assert {n for n, _ in entries} >= {"q36_moe_forward", "q36_gdn_verify", "q36_gdn_verify_ring", "q36_attn_proj",
+                                       "q36_attn_oproj", "q36_fp8_linear", "q36_add_rmsnorm", "q36_dense8_linear",
+                                       "q36_attn_decode", "q36_lmhead_argmax", "q36_moe_route"}
+    for name, st in entries:
+        other = _lib.MoeArgs if st is not _lib.MoeArgs else _lib.GdnArgs
+        for wrong in (C.byref(other()), other(), bytes(C.sizeof(st)), 4096):
+            with pytest.raises(C.ArgumentError):
+                getattr(L, name)(wrong, None)
+        assert getattr(L, name)(None, None) == _lib.Q36_EINVAL
+
+
+@pytest.mark.parametrize("name", ["moe", "gdn", "ring", "attn", "oproj", "lmhead", "fp8", "dense8", "addnorm", "decode"])
+def test_packed_arguments_are_the_filled_structure(name):
+    """pack_*(fields in order) gives the structure those fields fill one by one, nested arrays included."""
+    from bundles_amd import _lib
+    pack = getattr(_lib, f"pack_{name}")
+    flat = []
+    st = dict(moe=_lib.MoeArgs, gdn=_lib.GdnArgs, ring=_lib.GdnRingArgs, attn=_lib.AttnArgs,
+              oproj=_lib.OprojArgs, lmhead=_lib.LmheadArgs, fp8=_lib.Fp8LinearArgs, dense8=_lib.Dense8LinearArgs,
+              addnorm=_lib.AddNormArgs, decode=_lib.DecodeArgs)[name]
+    ref = st()
+
+    def fill(obj, fields):
+        for f, t in fields:
+            if hasattr(t, "_length_"):
+                for e in getattr(obj, f):
+                    fill(e, t._type_._fields_)
+                continue
+            v = 0.5 + len(flat) if t is C.c_float else 3 + 7 * len(flat)
+            flat.append(v)
+            setattr(obj, f, v)
+
+    fill(ref, st._fields_)
+    got = pack(*flat)
+    assert type(got) is st and bytes(got) == bytes(ref)
+
+
 def test_invalid_arguments_are_rejected(L):
     from bundles_amd import _lib
     assert L.q36_moe_forward(None, None) == _lib.Q36_EINVAL
