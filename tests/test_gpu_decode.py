@@ -222,13 +222,30 @@ def test_decode_balanced_shares(attn, oracle_mod, dev, NT, seqlens):
     h["pt"] = h["pt"][:, :max(seqlens)].contiguous()     # (the 128-key table: exactly its four steps wide)
     out, _ = _run(attn, h, NT, dev)
     _check(out, _oracle(oracle_mod, h, NT), f"balanced NT={NT} B={len(seqlens)}")
-    # a workspace that holds only the fixed splits' partials is still served
-    ws = attn.DecodeWorkspace(len(seqlens), dev, splits=1)
-    ws.splits = 0
+
+
+@pytest.mark.parametrize("NT,seqlens", [
+    (4, [1700]), (2, [2, 40, 256, 257, 3000]), (4, _ragged(64, 4, 700, [2500, 3000], 1)), (1, _ragged(100, 1, 900, [3000], 5)),
+    (4, _ragged(128, 200, 260, [4000], 2)), (3, _ragged(140, 3, 520, [2100, 900], 3)),
+], ids=["1", "5", "64", "100", "128", "140"])
+def test_decode_workspace_of_the_fixed_splits(attn, dev, NT, seqlens):
+    """A workspace that holds only the equal splits' partials (less than the dealing needs) is still served: by these
+    splits, bit for bit; a smaller one is refused."""
+    from bundles_amd import _lib
+    B = len(seqlens)
+    print(f"attn_decode workspace of the fixed splits NT={NT} B={B}", flush=True)
+    need = _lib.lib().q36_attn_decode_workspace_bytes
+    S = max(1, min(64, torch.cuda.get_device_properties(dev).multi_processor_count // (2 * B)))
+    assert need(B, S) < need(B, 0)
+    h = _make(B, NT, seqlens, seed=3 * NT + B)
     d = {k: h[k].to(dev) for k in ("q", "kc", "vc", "pt", "seqlens")}
-    if ws.buf.numel() >= 66048 * len(seqlens) * max(1, min(64, 128 // len(seqlens))):
-        out2 = attn.attn_decode(d["q"], d["kc"], d["vc"], d["pt"], d["seqlens"], NT, SCALE, ws)
-        assert_bf16_close(bits16(out2).reshape(-1, D), bits16(out).reshape(-1, D), 2e-3, "fixed splits")
+    want, _ = _run(attn, h, NT, dev, splits=S)
+    ws = attn.DecodeWorkspace(B, dev)
+    ws.buf = torch.full((need(B, S),), 0xFF, dtype=torch.uint8, device=dev)
+    assert torch.equal(attn.attn_decode(d["q"], d["kc"], d["vc"], d["pt"], d["seqlens"], NT, SCALE, ws), want)
+    ws.buf = ws.buf[:-1]
+    with pytest.raises(RuntimeError, match="workspace"):
+        attn.attn_decode(d["q"], d["kc"], d["vc"], d["pt"], d["seqlens"], NT, SCALE, ws)
 
 
 @pytest.mark.parametrize("NT,seqlens", [
