@@ -133,9 +133,9 @@ def test_lmhead_fp32_logits_buffer(lmh, dev, R, mode):
 
 @pytest.mark.parametrize("R,two_term,f32", [(1043, False, False), (1024, False, True), (515, True, True), (640, True, False)])
 def test_lmhead_tile_forms_agree(lmh, dev, R, two_term, f32):
-    """A vocabulary long enough for the 256-row tiles (with a tail of one 16-row tile) against its slices,
-    which take the 128-row tiles the oracle cases above run on: the same logits bit for bit, the ids the
-    first largest of them, with the codes in either order."""
+    """Codes in tile order: a vocabulary long enough for the 256-row tiles (with a tail of one 16-row tile) against its
+    slices in the same order, too short for them and so on the 128-row tiles; and the row-major codes' own kernel.
+    The same logits bit for bit, the ids the first largest of them."""
     V = 32784
     print(f"lmhead tile forms R={R} two_term={two_term} f32={f32}", flush=True)
     d, q, s = _setup(lmh, dev, R, V, seed=R)
@@ -147,8 +147,8 @@ def test_lmhead_tile_forms_agree(lmh, dev, R, two_term, f32):
     parts = []
     for v0 in range(0, V, 4096):
         n = min(4096, V - v0)
-        _, lg = lmh.w8a8_lmhead_argmax(d["h"], q[v0:v0 + n].contiguous(), s[v0:v0 + n].contiguous(), ws, want_logits=True,
-                                       two_term=two_term)
+        _, lg = lmh.w8a8_lmhead_argmax(d["h"], None, s[v0:v0 + n].contiguous(), ws, want_logits=True, two_term=two_term,
+                                       q_t=lmh.tile_rows_w16(q[v0:v0 + n].contiguous()))
         parts.append(lg)
     want = torch.cat(parts, dim=1)
     assert torch.equal(logits.to(torch.bfloat16), want) and torch.equal(logits_r, want)
