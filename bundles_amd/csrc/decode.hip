@@ -82,17 +82,31 @@ struct DecodeDev {
   float* oqs;               // [B*NT, 32] group scales
 };
 
+// The gate's 4 values at dims 4c .. 4c + 3 of row (token tok, head); zeros without a gate.  Read through a descriptor, so
+// that no branch holds the load back.
+__device__ __forceinline__ v2i gate_row(const DecodeDev& d, int tok, int head, int c) {
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(d.gate + (size_t)tok * (kQH * kDD)), (short)0, d.oq ? kQH * kDD * 2 : 0, 0x00020000);
+  return __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rs, (head * kDD + 4 * c) * 2, 0, 0));
+}
+// Max over each half of the wave (32 lanes), without LDS.
+__device__ __forceinline__ float half_max(float v) {
+  v = fmaxf(v, __uint_as_float(dpp_u32<0xB1>(__float_as_uint(v))));
+  v = fmaxf(v, __uint_as_float(dpp_u32<0x4E>(__float_as_uint(v))));
+  v = fmaxf(v, __uint_as_float(dpp_u32<0x141>(__float_as_uint(v))));
+  v = fmaxf(v, __uint_as_float(dpp_u32<0x140>(__float_as_uint(v))));
+  const auto p16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(p16[0]), __uint_as_float(p16[1]));
+}
 // The output's 4 values at dims 4c .. 4c + 3 of row (token tok, head) after the bf16 store: the o_proj
 // input bf16(o * sigmoid(gate)) in e4m3 per 128-channel group (32 neighbouring lanes of one wave hold
 // a group), the same arithmetic as the o_proj's own quantization of the bf16 output.
-__device__ __forceinline__ void gated_e4m3(const DecodeDev& d, int tok, int head, int c, uint32_t o01, uint32_t o23) {
+__device__ __forceinline__ void gated_e4m3(const DecodeDev& d, int tok, int head, int c, uint32_t o01, uint32_t o23, v2i gv) {
   const size_t at = (size_t)tok * (kQH * kDD) + head * kDD + 4 * c;
-  const uint2 gv = *reinterpret_cast<const uint2*>(d.gate + at);
-  float f[4] = {rbf_hw(bf_lo(o01) * sigmoid_q(bf_lo(gv.x))), rbf_hw(bf_hi(o01) * sigmoid_q(bf_hi(gv.x))),
-                rbf_hw(bf_lo(o23) * sigmoid_q(bf_lo(gv.y))), rbf_hw(bf_hi(o23) * sigmoid_q(bf_hi(gv.y)))};
-  float m = fmaxf(fmaxf(fabsf(f[0]), fabsf(f[1])), fmaxf(fabsf(f[2]), fabsf(f[3])));
-#pragma unroll
-  for (int o = 16; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+  const uint32_t g01 = (uint32_t)gv.x, g23 = (uint32_t)gv.y;
+  float f[4] = {rbf_hw(bf_lo(o01) * sigmoid_q(bf_lo(g01))), rbf_hw(bf_hi(o01) * sigmoid_q(bf_hi(g01))),
+                rbf_hw(bf_lo(o23) * sigmoid_q(bf_lo(g23))), rbf_hw(bf_hi(o23) * sigmoid_q(bf_hi(g23)))};
+  const float m = half_max(fmaxf(fmaxf(fabsf(f[0]), fabsf(f[1])), fmaxf(fabsf(f[2]), fabsf(f[3]))));
   const float inv = m > 0.f ? 448.f / m : 0.f;
   *reinterpret_cast<uint32_t*>(d.oq + at) = f2e4m3x2_hw(f[0] * inv, f[1] * inv) | (f2e4m3x2_hw(f[2] * inv, f[3] * inv) << 16);
   if ((c & 31) == 0) d.oqs[(size_t)tok * (kQH * kDD / 128) + head * 2 + c / 32] = m / 448.f;
@@ -180,7 +194,7 @@ __device__ __forceinline__ int wave_rows_sum_i(int v) {  // over the wave's four
   const auto p32 = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false);
   return (int)(p32[0] + p32[1]);
 }
-__device__ __forceinline__ int wave_max_i(int v) {
+__device__ __forceinline__ int wave_imax(int v) {
   v = max(v, (int)dpp_u32<0xB1>((uint32_t)v));
   v = max(v, (int)dpp_u32<0x4E>((uint32_t)v));
   v = max(v, (int)dpp_u32<0x141>((uint32_t)v));
@@ -250,7 +264,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
         steps += v, longest = max(longest, v);
       }
     }
-    steps = wave_sum_i(steps), longest = wave_max_i(longest);
+    steps = wave_sum_i(steps), longest = wave_imax(longest);
     if (!few) {
       if (lane == 0) rsum[wv] = steps, rmax[wv] = longest;
       __syncthreads();
@@ -674,7 +688,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
         const uint32_t o01 = pack_bf2_hw(a[0] * il, a[1] * il), o23 = pack_bf2_hw(a[2] * il, a[3] * il);
         *reinterpret_cast<uint2*>(dst) = make_uint2(o01, o23);
         // a wave holds one row (rows * 64 threads, whole waves): its two 128-groups are its lane halves
-        if (d.oq) gated_e4m3(d, b * NT + (row >> 3), h * kGQ + (row & 7), c, o01, o23);
+        if (d.oq) {
+          const int tok = b * NT + (row >> 3), head = h * kGQ + (row & 7);
+          gated_e4m3(d, tok, head, c, o01, o23, gate_row(d, __builtin_amdgcn_readfirstlane(tok), head, c));
+        }
       }
     }
   }
@@ -696,12 +713,12 @@ __device__ __forceinline__ Pieces req_parts(const DecodeDev& d, int b, int h) {
   const int2 w = d.meta[b];
   return Pieces{w.y - w.x + 1, part_slot(w.x, h, 0), part_slot(1, 0, 0), part_slot(0, 0, kFirst)};
 }
-__device__ __forceinline__ void put_row(const DecodeDev& d, int bt, int head, int c, v4f a, float L) {
+__device__ __forceinline__ void put_row(const DecodeDev& d, int bt, int head, int c, v4f a, float L, v2i gate) {
   const float il = L > 0.f ? 1.f / L : 0.f;
   const uint32_t o01 = pack_bf2_hw(a[0] * il, a[1] * il), o23 = pack_bf2_hw(a[2] * il, a[3] * il);
   *reinterpret_cast<uint2*>(d.out + ((size_t)bt * kQH + head) * kDD + 4 * c) = make_uint2(o01, o23);
   // the wave holds the row: lanes 0-31 / 32-63 its two 128-groups
-  if (d.oq) gated_e4m3(d, bt, head, c, o01, o23);
+  if (d.oq) gated_e4m3(d, bt, head, c, o01, o23, gate);
 }
 
 // A workgroup a token, each of its 4 waves 4 query rows, each lane 4 dims of them.  Up to kNF pieces are in flight at
@@ -719,6 +736,9 @@ __global__ __launch_bounds__(256) void decode_combine_few_kernel(DecodeDev d, in
       (void*)(d.ws_o + (size_t)P.g0 * kRows * kDD), (short)0, span * (kDD * 4), 0x00020000);
   const __amdgpu_buffer_rsrc_t mrs = __builtin_amdgcn_make_buffer_rsrc(
       (void*)(d.ws_ml + (size_t)P.g0 * 2 * kRows), (short)0, span * (2 * 4), 0x00020000);
+  v2i gate[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) gate[i] = gate_row(d, bt, head + i, c);
   v4f a[4] = {}, M = {-1e30f, -1e30f, -1e30f, -1e30f}, L = {};  // the pieces' maxima are finite (-1e30: no visible key)
   for (int p0 = 0; p0 < P.n; p0 += kNF) {
     v4f m[kNF], l[kNF], o[kNF][4];
@@ -756,7 +776,7 @@ __global__ __launch_bounds__(256) void decode_combine_few_kernel(DecodeDev d, in
     }
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i) put_row(d, bt, head + i, c, a[i], L[i]);
+  for (int i = 0; i < 4; ++i) put_row(d, bt, head + i, c, a[i], L[i], gate[i]);
 }
 
 // A workgroup a row: wave v adds pieces v, v + WPR, ..., each lane 4 dims, four in flight, and the waves' sums meet in LDS
@@ -778,6 +798,7 @@ __global__ __launch_bounds__(64 * WPR) void decode_combine_kernel(DecodeDev d, i
       o[k] = *reinterpret_cast<const v4f*>(d.ws_o + (slot(p0 + min(q0 + k * WPR, m - 1)) * kRows + gr) * kDD + 4 * c);
   };
   auto ml = [&](int p, int what) { return d.ws_ml[(slot(p) * 2 + what) * kRows + gr]; };
+  const v2i gate = gate_row(d, bt, head, c);
   float mp = ml(min(lane, n - 1), 0), lp = ml(min(lane, n - 1), 1);
   fetch(0, wave, min(64, n));
   float M = mp;
@@ -806,7 +827,7 @@ __global__ __launch_bounds__(64 * WPR) void decode_combine_kernel(DecodeDev d, i
   if (wave != 0) return;
 #pragma unroll
   for (int v = 1; v < WPR; ++v) a += sums[v][lane];
-  put_row(d, bt, head, c, a, L);
+  put_row(d, bt, head, c, a, L, gate);
 }
 
 int decode_cus() {
