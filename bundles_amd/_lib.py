@@ -102,9 +102,8 @@ class DecodeArgs(C.Structure):
 
 
 def _packer(st):
-    """A function of a structure's fields in order (nested arrays flattened) that returns the filled structure.  struct.pack
-    fills it: setting the fields of the ctypes structure one by one took longer than the launch it describes (45 fields:
-    a call 3.4 us against 1.6)."""
+    """struct.pack of a structure's fields in order (nested arrays flattened): the bytes of the filled structure, for packed().
+    Filling the ctypes structure itself took longer than the launch it describes (45 fields: 5 us against 1)."""
     code = {P: "P", I32: "i", SZ: "N", I64: "q", C.c_float: "f"}
     fmt = "@"
     for _, t in st._fields_:
@@ -114,8 +113,7 @@ def _packer(st):
             fmt += "0q" + "".join(code[f] for _, f in t._type_._fields_) * t._length_
     s = struct.Struct(fmt + "0q")
     assert s.size == C.sizeof(st), st
-    pack, filled = s.pack, st.from_buffer_copy
-    return lambda *fields: filled(pack(*fields))
+    return s.pack
 
 
 pack_moe, pack_gdn, pack_ring, pack_attn = map(_packer, (MoeArgs, GdnArgs, GdnRingArgs, AttnArgs))
@@ -123,7 +121,7 @@ pack_oproj, pack_lmhead, pack_fp8, pack_dense8 = map(_packer, (OprojArgs, Lmhead
 pack_addnorm, pack_decode = map(_packer, (AddNormArgs, DecodeArgs))
 
 
-_lib = None
+_lib = _packed = None
 
 # (name, restype, argtypes) of every exported symbol; tests check that each one resolves.
 SYMBOLS = [
@@ -163,21 +161,37 @@ SYMBOLS = [
     ("q36_pack_frag8", I32, [P, C.c_int64, I32, P, P]),
 ]
 OPTIONAL_SYMBOLS: list = []
+ARG_POINTERS = [C.POINTER(s) for s in (MoeArgs, GdnArgs, GdnRingArgs, AttnArgs, OprojArgs, LmheadArgs, Fp8LinearArgs,
+                                       AddNormArgs, Dense8LinearArgs, DecodeArgs)]
+
+
+def _load(arg0):
+    if not os.path.exists(LIB_PATH):
+        raise RuntimeError(f"libq36.so is not built ({LIB_PATH}); run bundles_amd.build.build() first")
+    L = C.CDLL(LIB_PATH)
+    for name, res, args in SYMBOLS:
+        f = getattr(L, name)
+        f.restype = res
+        f.argtypes = [arg0(a) for a in args[:1]] + args[1:]
+    return L
 
 
 def lib():
     """Load libq36.so (built by bundles_amd.build); raise if it is missing."""
     global _lib
     if _lib is None:
-        if not os.path.exists(LIB_PATH):
-            raise RuntimeError(f"libq36.so is not built ({LIB_PATH}); run bundles_amd.build.build() first")
-        L = C.CDLL(LIB_PATH)
-        for name, res, args in SYMBOLS:
-            f = getattr(L, name)
-            f.restype = res
-            f.argtypes = args
-        _lib = L
+        _lib = _load(lambda a: a)
     return _lib
+
+
+def packed():
+    """The same library for this package's own wrappers, which hand an entry the bytes that its structure's pack_* function
+    made: its argument structure goes as a bare pointer.  (lib() refuses anything but the entry's structure; turning the
+    bytes into one costs 0.3 us a call.)"""
+    global _packed
+    if _packed is None:
+        _packed = _load(lambda a: P if a in ARG_POINTERS else a)
+    return _packed
 
 
 def check(rc: int, what: str) -> None:

@@ -123,7 +123,7 @@ def attn_proj(x, w: AttnWeights, q_norm_w, k_norm_w, eps, cos_sin, positions, ws
                  ptr(cos_sin), ptr(positions), ptr(o["q"]), ptr(o["gate"]), ptr(o["k"]), ptr(o["v"]), ptr(o["k8"]),
                  ptr(o["v8"]), ptr(ws.proj), ws.proj.numel(), ptr(None if xq is None else xq.codes),
                  ptr(None if xq is None else xq.scales), ptr(loc), ptr(kc), ptr(vc), slots)
-    check(_lib.lib().q36_attn_proj(a, _lib.stream_handle(stream)), "q36_attn_proj")
+    check(_lib.packed().q36_attn_proj(a, _lib.stream_handle(stream)), "q36_attn_proj")
     return o
 
 
@@ -138,7 +138,7 @@ def attn_oproj(attn, gate, w: AttnWeights, ws: Workspace, out=None, stream=None,
     out = torch.empty((T, HIDDEN), dtype=torch.bfloat16, device=dev) if out is None else out
     a = pack_oproj(T, ptr(attn), ptr(gate), ptr(w.wo_p), ptr(w.so), ptr(out), ptr(ws.oproj), ws.oproj.numel(),
                   ptr(None if aq is None else aq.codes), ptr(None if aq is None else aq.scales))
-    check(_lib.lib().q36_attn_oproj(a, _lib.stream_handle(stream)), "q36_attn_oproj")
+    check(_lib.packed().q36_attn_oproj(a, _lib.stream_handle(stream)), "q36_attn_oproj")
     return out
 
 
@@ -187,5 +187,5 @@ def attn_decode(q, k_cache, v_cache, page_table, seqlens, NT: int, scale: float,
                    k_cache.shape[0], ptr(page_table), page_table.shape[1], ptr(seqlens), ptr(out_loc), ptr(k_new),
                    ptr(v_new), scale, ptr(out), ptr(ws.buf), ws.buf.numel(), ptr(gate),
                    ptr(None if oq is None else oq.codes), ptr(None if oq is None else oq.scales))
-    check(_lib.lib().q36_attn_decode(a, _lib.stream_handle(stream)), "q36_attn_decode")
+    check(_lib.packed().q36_attn_decode(a, _lib.stream_handle(stream)), "q36_attn_decode")
     return out

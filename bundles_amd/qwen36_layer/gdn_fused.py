@@ -50,7 +50,7 @@ def gdn_verify_fused(mixed, z, a, b, conv_state, conv_w, A_log, dt_bias, S0, nor
     conv_state_out = torch.empty_like(conv_state) if conv_state_out is None else conv_state_out
     args = pack_gdn(B, T, ptr(mixed), ptr(z), ptr(a), ptr(b), ptr(conv_state), ptr(conv_state_out), ptr(conv_w),
                    ptr(A_log), ptr(dt_bias), ptr(S0), ptr(norm_w), eps, ptr(out), ptr(snaps))
-    check(_lib.lib().q36_gdn_verify(args, _lib.stream_handle(stream)), "q36_gdn_verify")
+    check(_lib.packed().q36_gdn_verify(args, _lib.stream_handle(stream)), "q36_gdn_verify")
     return out, snaps, conv_state_out
 
 
@@ -140,5 +140,5 @@ def gdn_verify_ring(mixed, z, a, b, conv_state, conv_w, window, A_log, dt_bias, 
         k_ring.stride(0), klo_ring.stride(0), ptr(g_ring), g_ring.stride(0), ptr(qsl), ptr(state_idx),
         ptr(replay_idx), ptr(win_idx), flags, ptr(write_pos), ptr(cache_base), ptr(norm_w), eps, scale, ptr(out),
         ptr(None if oq is None else oq.codes), ptr(None if oq is None else oq.scales))
-    check(_lib.lib().q36_gdn_verify_ring(args, _lib.stream_handle(stream)), "q36_gdn_verify_ring")
+    check(_lib.packed().q36_gdn_verify_ring(args, _lib.stream_handle(stream)), "q36_gdn_verify_ring")
     return out

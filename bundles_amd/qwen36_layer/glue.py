@@ -94,7 +94,7 @@ def fp8_linear(x: torch.Tensor, w: Fp8Weight, ws: LinearWorkspace, segments=None
     a = pack_fp8(T, w.qp.shape[0], K, w.n, ptr(x), ptr(w.qp), ptr(w.s), len(segments), *segs,
                  ptr(ws.buf), ws.buf.numel(), ptr(None if xq is None else xq.codes),
                  ptr(None if xq is None else xq.scales))
-    check(_lib.lib().q36_fp8_linear(a, _lib.stream_handle(stream)), "q36_fp8_linear")
+    check(_lib.packed().q36_fp8_linear(a, _lib.stream_handle(stream)), "q36_fp8_linear")
     return ret
 
 
@@ -134,7 +134,7 @@ def dense8_linear(x: torch.Tensor, q: torch.Tensor, s: torch.Tensor, segments=No
         ret = None
     segs = _segments("dense8_linear", T, N, segments)
     a = pack_dense8(T, N, K, N, ptr(x), ptr(q), ptr(s), s.stride(0), len(segments), *segs, int(bool(tiled)))
-    check(_lib.lib().q36_dense8_linear(a, _lib.stream_handle(stream)), "q36_dense8_linear")
+    check(_lib.packed().q36_dense8_linear(a, _lib.stream_handle(stream)), "q36_dense8_linear")
     return ret
 
 
@@ -149,5 +149,5 @@ def add_rmsnorm(delta, residual: torch.Tensor, norm_w: torch.Tensor, eps: float,
     a = pack_addnorm(T, H, ptr(delta), ptr(residual), ptr(norm_w), eps, ptr(out),
                      ptr(None if q8 is None else q8.codes), ptr(None if q8 is None else q8.scales),
                      int(q8 is not None and q8.frag))
-    check(_lib.lib().q36_add_rmsnorm(a, _lib.stream_handle(stream)), "q36_add_rmsnorm")
+    check(_lib.packed().q36_add_rmsnorm(a, _lib.stream_handle(stream)), "q36_add_rmsnorm")
     return out

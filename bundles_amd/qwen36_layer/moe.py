@@ -179,8 +179,13 @@ class Workspace:
             y=v(L.y, (S + M) * self.H, torch.bfloat16).view(S + M, self.H))
 
 
-def _args(x, positions, router_w, gate_w, ew, topk, ws: Workspace, out, router_bias, debug, norm=None, norm_q8=None,
-          pre_norm=None) -> MoeArgs:
+def _args(*args, **kwargs) -> MoeArgs:
+    return MoeArgs.from_buffer_copy(_packed(*args, **kwargs))
+
+
+def _packed(x, positions, router_w, gate_w, ew, topk, ws: Workspace, out, router_bias, debug, norm=None, norm_q8=None,
+            pre_norm=None) -> bytes:
+    """The checked arguments as the bytes of q36_moe_args."""
     M, H = (x if x is not None else pre_norm[0]).shape
     if M > ws.max_tokens:
         raise ValueError(f"moe_row_batch: {M} rows exceed the workspace's {ws.max_tokens}")
@@ -221,8 +226,8 @@ def _args(x, positions, router_w, gate_w, ew, topk, ws: Workspace, out, router_b
 
 def route(x, positions, router_w, topk: int, ws: Workspace, router_bias=None, stream=None):
     """Routing only (ids, weights, expert lists and quantized x in the workspace); returns ws.views(M)."""
-    a = _args(x, positions, router_w, None, None, topk, ws, None, router_bias, None)
-    check(_lib.lib().q36_moe_route(a, _lib.stream_handle(stream)), "q36_moe_route")
+    a = _packed(x, positions, router_w, None, None, topk, ws, None, router_bias, None)
+    check(_lib.packed().q36_moe_route(a, _lib.stream_handle(stream)), "q36_moe_route")
     return ws.views(x.shape[0])
 
 
@@ -248,8 +253,8 @@ def moe_row_batch(x, positions, router_w, gate_w, ew: ExpertWeights, topk: int, 
         out = torch.empty_like(shape_src)
     if norm_q8 is not None and (norm is None or norm_q8.T != shape_src.shape[0]):
         raise ValueError("moe_row_batch: norm_q8 needs the fused add-norm and one row per token")
-    a = _args(x, positions, router_w, gate_w, ew, topk, ws, out, router_bias, debug, norm, norm_q8, pre_norm)
-    check(_lib.lib().q36_moe_forward(a, _lib.stream_handle(stream)), "q36_moe_forward")
+    a = _packed(x, positions, router_w, gate_w, ew, topk, ws, out, router_bias, debug, norm, norm_q8, pre_norm)
+    check(_lib.packed().q36_moe_forward(a, _lib.stream_handle(stream)), "q36_moe_forward")
     return out
 
 
@@ -257,8 +262,8 @@ def moe_phases(x, positions, router_w, gate_w, ew: ExpertWeights, topk: int, ws:
                stream=None):
     """The same block as moe_row_batch as four separately launched phases (route, up, down, combine);
     returns the list of (name, callable) so a caller can schedule or time each one."""
-    a = _args(x, positions, router_w, gate_w, ew, topk, ws, out, router_bias, None)
-    L = _lib.lib()
+    a = _packed(x, positions, router_w, gate_w, ew, topk, ws, out, router_bias, None)
+    L = _lib.packed()
     # the argument struct holds raw device addresses: the callables keep the tensors they point into
     # alive, so a caller that drops its own references does not leave them pointing at freed memory
     keep = (x, positions, router_w, gate_w, ew, ws, out, router_bias)

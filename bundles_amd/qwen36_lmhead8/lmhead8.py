@@ -75,5 +75,5 @@ def w8a8_lmhead_argmax(h, q, scale, ws: Workspace, norm_w=None, eps: float = 1e-
                     ws.buf.numel(),
                     _lib.Q36_LMH_W8A16 if w8a16 else _lib.Q36_LMH_W8A8X2 if two_term else _lib.Q36_LMH_W8A8,
                     int(logits is not None and logits.dtype == torch.float32), ptr(q_t))
-    check(_lib.lib().q36_lmhead_argmax(a, _lib.stream_handle(stream)), "q36_lmhead_argmax")
+    check(_lib.packed().q36_lmhead_argmax(a, _lib.stream_handle(stream)), "q36_lmhead_argmax")
     return (ids, logits) if (want_logits or logits is not None) else ids

@@ -66,31 +66,28 @@ def test_struct_layouts_match_header(tmp_path):
             assert got[(cname, fname)] == getattr(st, fname).offset, f"{cname}.{fname}"
 
 
-def _entries():
-    """(symbol, its argument structure) of every entry point that takes one."""
-    from bundles_amd import _lib
-    return [(n, a[0]._type_) for n, _, a in _lib.SYMBOLS if a and hasattr(a[0], "_type_") and
-            isinstance(a[0]._type_, type) and issubclass(a[0]._type_, C.Structure)]
-
-
 def test_entry_points_refuse_another_structure(L):
     """Each entry takes its own argument structure; another one, raw bytes or a number never reach the library."""
     from bundles_amd import _lib
-    entries = _entries()
-    assert {n for n, _ in entries} >= {"q36_moe_forward", "q36_gdn_verify", "q36_gdn_verify_ring", "q36_attn_proj",
+    entries = [(n, a[0]._type_) for n, _, a in _lib.SYMBOLS if a and a[0] in _lib.ARG_POINTERS]
+    assert {n for n, _ in entries} == {"q36_moe_route", "q36_moe_up", "q36_moe_down", "q36_moe_combine", "q36_moe_forward",
+                                       "q36_moe_forward_static", "q36_gdn_verify", "q36_gdn_verify_ring", "q36_attn_proj",
                                        "q36_attn_oproj", "q36_fp8_linear", "q36_add_rmsnorm", "q36_dense8_linear",
-                                       "q36_attn_decode", "q36_lmhead_argmax", "q36_moe_route"}
+                                       "q36_attn_decode", "q36_lmhead_argmax"}
     for name, st in entries:
         other = _lib.MoeArgs if st is not _lib.MoeArgs else _lib.GdnArgs
         for wrong in (C.byref(other()), other(), bytes(C.sizeof(st)), 4096):
             with pytest.raises(C.ArgumentError):
                 getattr(L, name)(wrong, None)
         assert getattr(L, name)(None, None) == _lib.Q36_EINVAL
+    # the wrappers' own form: the packed bytes, read as the structure
+    assert _lib.packed().q36_attn_decode(_lib.pack_decode(4, 4, 32, *[0] * 20), None) == _lib.Q36_EINVAL
+    assert b"HQ=32" in L.q36_last_error()
 
 
 @pytest.mark.parametrize("name", ["moe", "gdn", "ring", "attn", "oproj", "lmhead", "fp8", "dense8", "addnorm", "decode"])
 def test_packed_arguments_are_the_filled_structure(name):
-    """pack_*(fields in order) gives the structure those fields fill one by one, nested arrays included."""
+    """pack_*(fields in order) gives the bytes of the structure that those fields fill one by one, nested arrays included."""
     from bundles_amd import _lib
     pack = getattr(_lib, f"pack_{name}")
     flat = []
@@ -110,8 +107,7 @@ def test_packed_arguments_are_the_filled_structure(name):
             setattr(obj, f, v)
 
     fill(ref, st._fields_)
-    got = pack(*flat)
-    assert type(got) is st and bytes(got) == bytes(ref)
+    assert pack(*flat) == bytes(ref)
 
 
 def test_invalid_arguments_are_rejected(L):
