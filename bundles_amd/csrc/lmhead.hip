@@ -191,9 +191,10 @@ __host__ __device__ __forceinline__ int lmh_groups(int nrt) { return nrt >= 8 &&
 //
 // Why this split: with both operands in LDS (8 waves, 128 x 64 a wave) a step's 96 KB of fragment reads and
 // 32 KB of writes took as long as its MFMAs; with the weights in registers a CU reads 64 KB and writes 16.
-// What bounds it now, at 2048 rows: the power the MFMAs draw (a loop of these MFMAs alone with one LDS
-// read per four runs at 3.5 POP/s on random codes and 4.6 on zeros: 367 us for this product), the
-// epilogue (about 30 us) and the weights' latency behind the logits' stores.  Measured, us a call
+// What bounds it now, at 2048 rows: the matrix cores, busy 67 % of the time, at the clock their power leaves (a
+// loop of these MFMAs alone with one LDS read per four runs at 3.6 POP/s on random codes and 4.2 on
+// zeros: 353 us for this product); then the epilogue (about 30 us) and the weights' latency: 1.47 GB are
+// fetched, 2.3 times the two weight reads planned below, and with logits the loads queue behind the stores.  Measured, us a call
 // (before -> now): 2048 rows with bf16 logits 743 -> 585, fp32 800 -> 705, none 548 -> 503; 256 rows two
 // terms 175 -> 153 bf16, 153 -> 139 none; 150 rows two terms fp32 168 -> 133; 64 rows 93 -> 70; 300 rows
 // one term 139 -> 114.  A token's 64 logits of a wave go out as 64-byte runs (16-byte pieces before).
@@ -202,7 +203,7 @@ __host__ __device__ __forceinline__ int lmh_groups(int nrt) { return nrt >= 8 &&
 // row tiles of group x % ngrp and the vocab tiles v = x / ngrp (mod 8 / ngrp).  Its workgroups take
 // tiles j = loc, loc + nloc, ... (loc = blockIdx / 8, nloc = gridDim / 8), tile j being row tile
 // (x % ngrp) * rpg + j % rpg of vocab tile (j / rpg) * (8 / ngrp) + x / ngrp: the row tiles of one
-// vocab tile run side by side on one XCD (its weight tile comes from HBM once per XCD), and an
+// vocab tile run side by side on one XCD (for its weight tile to come from HBM once per XCD), and an
 // XCD's activations (2 MB at 2048 rows) stay resident in its L2 while the weights stream through.
 //
 // STORE: 0 no logits, 1 bf16 logits, 2 fp32 logits (the bf16-rounded values widened); 3 and 4: as 1 and 2
