@@ -240,3 +240,38 @@ def test_oproj_from_decode_codes(attn, dev, B, NT, splits):
     torch.cuda.synchronize()
     _same(o1, o2, "attention out")
     _same(got, ref, "o_proj out")
+
+
+@pytest.mark.parametrize("B,NT,lo,hi", [
+    (20, 4, 500, 2000),    # pieces, four waves a row in the combine
+    (2, 1, 9000, 12000),   # pieces, sixteen
+    (60, 2, 20, 2500),     # line and pieces of a few, in several rounds of one wave
+    (64, 4, 700, 900),     # two pieces each
+    (90, 1, 20, 300),      # whole requests: the split kernel's epilogue alone
+], ids=["20x4", "2x1", "60x2", "64x4", "90x1"])
+def test_oproj_from_dealt_decode_codes(attn, dev, B, NT, lo, hi):
+    """The same over the routes of the default dealing, in a page table much wider than the requests."""
+    print(f"oproj from decode codes, dealt, B={B} NT={NT} {lo}..{hi}", flush=True)
+    T = B * NT
+    g = torch.Generator(device=dev).manual_seed(B * 10 + NT)
+    sl = torch.exp(torch.empty(B, device=dev).uniform_(float(np.log(lo)), float(np.log(hi)), generator=g)).to(torch.int32)
+    slots = 4096
+    q = torch.randn((T, 16, 256), generator=g, device=dev).to(torch.bfloat16)
+    kc = torch.randn((slots, 2, 256), generator=g, device=dev).to(torch.float8_e4m3fn).view(torch.uint8)
+    vc = torch.randn((slots, 2, 256), generator=g, device=dev).to(torch.float8_e4m3fn).view(torch.uint8)
+    pt = torch.randint(0, slots, (B, 32768), generator=g, device=dev, dtype=torch.int32)
+    gate = (torch.randn((T, 4096), generator=g, device=dev) * 2).to(torch.bfloat16)
+    dws = attn.DecodeWorkspace(B, dev)
+    dws.buf.fill_(0xFF)
+    o1 = attn.attn_decode(q, kc, vc, pt, sl, NT, 1.0 / 16, dws)
+    dws.buf.fill_(0xFF)
+    oq = attn.oproj_rows(T, dev)
+    o2 = attn.attn_decode(q, kc, vc, pt, sl, NT, 1.0 / 16, dws, gate=gate, oq=oq)
+    d, w = _setup(attn, dev, T, seed=5)
+    ws = attn.Workspace(T, dev)
+    ref = attn.attn_oproj(o1.view(T, -1), gate, w, ws)
+    got = attn.attn_oproj(None, None, w, ws, aq=oq)
+    torch.cuda.synchronize()
+    assert torch.isfinite(o1.float()).all()
+    _same(o1, o2, "attention out")
+    _same(got, ref, "o_proj out")
